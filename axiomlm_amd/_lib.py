@@ -49,6 +49,7 @@ _SIGNATURES = {
         c_int, [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]
     ),
     "axm_qmm_q4_tile16_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "axm_qmm_q4_tile16_rows_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "axm_qmm_q4_tile16": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p],

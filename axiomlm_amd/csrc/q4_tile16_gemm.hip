@@ -78,27 +78,6 @@ int gemm_splits(int KB, int n_units, int rc, int upw) {
   return splits < 1 ? 1 : splits;
 }
 
-// One output element of the epilogue (identical arithmetic to the GEMV's):
-// v0 the gate / plain accumulator, v1 the up accumulator (SwiGLU).
-template <int EPI>
-__device__ __forceinline__ void t16g_store(const T16Args& a, int tok, int row, float v0, float v1) {
-  if (EPI == Q4_EPI_SWIGLU) {
-    const f16 g = f2h(v0);
-    const f16 u = f2h(v1);
-    const f16 sg = f2h(t16_silu(h2f(g)));
-    a.y[(size_t)tok * a.ldy + row] = f2h(h2f(sg) * h2f(u));
-  } else {
-    f16 h = f2h(v0);
-    if (a.bias != nullptr) h = f2h(h2f(h) + h2f(a.bias[row]));
-    if (EPI == Q4_EPI_STORE) {
-      a.y[(size_t)tok * a.ldy + row] = h;
-    } else {
-      f16* xr = a.resid + (size_t)tok * a.ldr + row;
-      *xr = f2h(h2f(*xr) + h2f(h));
-    }
-  }
-}
-
 // Each wave owns NT weight tiles over the workgroup's K split: a gate/up pair
 // (SwiGLU) or NT adjacent units (store / residual epilogues).  The split's activations of all 16 MB token rows are staged range by
 // range (RC chunks, double-buffered in LDS: range r + 1 is loaded while range r
@@ -297,6 +276,38 @@ __global__ void t16g_reduce_kernel(T16Args a, int n_splits, int up_col, int tok_
   t16g_store<EPI>(a, tok, row, v0, v1);
 }
 
+// The same with a thread per four rows of a token: 16-byte partial loads (N % 4 == 0).  A
+// thread per row read 4 bytes at a time (the 1000 x 12288 x 4096 many-row GEMM from two
+// splits, 128-row tiles: 132 -> 119 us).
+template <int EPI>
+__global__ void __launch_bounds__(256) t16g_reduce4_kernel(T16Args a, int n_splits, int up_col, int tok_stride) {
+  const int nv = a.N / 4;
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  const int tok = (int)(idx / nv), row = 4 * (int)(idx % nv);
+  if (tok >= a.M_tokens) return;
+  f32x4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = v0;
+#pragma unroll 4
+  for (int sp = 0; sp < n_splits; ++sp) {
+    const float* p = a.part_ws + ((size_t)sp * tok_stride + tok) * a.part_cols + row;
+    v0 += *reinterpret_cast<const f32x4*>(p);
+    if (EPI == Q4_EPI_SWIGLU) v1 += *reinterpret_cast<const f32x4*>(p + up_col);
+  }
+  t16g_store4<EPI>(a, tok, row, v0, v1, t16g_vec4<EPI>(a));
+}
+
+template <int EPI>
+void t16g_reduce(const T16Args& a, int M, int splits, int up_col, int ts, hipStream_t s) {
+  if (a.N % 4 == 0) {
+    const long n = (long)M * (a.N / 4);
+    hipLaunchKernelGGL(t16g_reduce4_kernel<EPI>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, splits, up_col,
+                       ts);
+  } else {
+    const long n = (long)M * a.N;
+    hipLaunchKernelGGL(t16g_reduce_kernel<EPI>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, splits, up_col,
+                       ts);
+  }
+}
+
 // Residual epilogue over the split partials of whole token rows, then RMSNorm of
 // each updated row into post_norm_out: one 1024-thread workgroup per token,
 // thread tid owns the 4-row vectors tid + 1024 i (N % 4 == 0, N <= 16384,
@@ -412,6 +423,37 @@ size_t t16_gemm_ws_bytes(int K, int n_units, int NT) {
   return need;
 }
 
+// After a GEMM of `splits` K splits: the epilogue over the summed partials (ts token rows per
+// split), and the RMSNorm of the updated residual rows where it is asked for.
+int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, hipStream_t s) {
+  if (a.split_info != nullptr) {
+    a.split_info[0] = a.split_info[1] = a.split_info[2] = 0;
+    if (splits > 1 && epi == Q4_EPI_STORE && a.post_ln_w == nullptr) {
+      a.split_info[0] = splits;
+      a.split_info[1] = ts;
+      a.split_info[2] = a.part_cols;
+      return 0;
+    }
+  }
+  if (a.post_ln_w != nullptr) {
+    // Residual rows then their RMSNorm: one fused launch over the partials, or
+    // the norm kernel after an unsplit GEMM (and as the general fallback).
+    if (splits > 1 && post_norm_fusable(a)) {
+      hipLaunchKernelGGL(t16g_reduce_resid_norm_kernel, dim3(M), dim3(kRnThreads), 0, s, a, splits, ts);
+      return 0;
+    }
+    if (splits > 1) t16g_reduce<Q4_EPI_RESID>(a, M, splits, 0, ts, s);
+    return launch_rmsnorm(a.resid, a.post_ln_w, a.post_norm_out, M, a.N, a.eps, s);
+  }
+  if (splits > 1) {
+    const int up_col = a.pair_offset * 16;
+    if (epi == Q4_EPI_STORE) t16g_reduce<Q4_EPI_STORE>(a, M, splits, up_col, ts, s);
+    else if (epi == Q4_EPI_RESID) t16g_reduce<Q4_EPI_RESID>(a, M, splits, up_col, ts, s);
+    else t16g_reduce<Q4_EPI_SWIGLU>(a, M, splits, up_col, ts, s);
+  }
+  return 0;
+}
+
 int t16_gemm_launch(T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s) {
   if (M < 1 || M > kTile16GemmMaxTokens || a.ln_w != nullptr || a.argmax_keys != nullptr || a.x_parts != nullptr ||
       (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) || a.K <= 0 || a.K % 64 != 0 ||
@@ -454,42 +496,7 @@ int t16_gemm_launch(T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipSt
       t16g_launch_epi<Q4_EPI_SWIGLU>(a, cfg, grid, s);
       break;
   }
-  const int ts = 16 * cfg.mb;
-  if (a.split_info != nullptr) {
-    a.split_info[0] = a.split_info[1] = a.split_info[2] = 0;
-    if (splits > 1 && epi == Q4_EPI_STORE && a.post_ln_w == nullptr) {
-      a.split_info[0] = splits;
-      a.split_info[1] = ts;
-      a.split_info[2] = a.part_cols;
-      return 0;
-    }
-  }
-  if (a.post_ln_w != nullptr) {
-    // Residual rows then their RMSNorm: one fused launch over the partials, or
-    // the norm kernel after an unsplit GEMM (and as the general fallback).
-    if (splits > 1 && post_norm_fusable(a)) {
-      hipLaunchKernelGGL(t16g_reduce_resid_norm_kernel, dim3(M), dim3(kRnThreads), 0, s, a, splits, ts);
-      return 0;
-    }
-    if (splits > 1) {
-      const long n = (long)M * a.N;
-      hipLaunchKernelGGL(t16g_reduce_kernel<Q4_EPI_RESID>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a,
-                         splits, 0, ts);
-    }
-    return launch_rmsnorm(a.resid, a.post_ln_w, a.post_norm_out, M, a.N, a.eps, s);
-  }
-  if (splits > 1) {
-    const long n = (long)M * a.N;
-    const dim3 rg((unsigned)((n + 255) / 256));
-    const int up_col = a.pair_offset * 16;
-    if (epi == Q4_EPI_STORE)
-      hipLaunchKernelGGL(t16g_reduce_kernel<Q4_EPI_STORE>, rg, dim3(256), 0, s, a, splits, up_col, ts);
-    else if (epi == Q4_EPI_RESID)
-      hipLaunchKernelGGL(t16g_reduce_kernel<Q4_EPI_RESID>, rg, dim3(256), 0, s, a, splits, up_col, ts);
-    else
-      hipLaunchKernelGGL(t16g_reduce_kernel<Q4_EPI_SWIGLU>, rg, dim3(256), 0, s, a, splits, up_col, ts);
-  }
-  return 0;
+  return t16_gemm_finish(a, M, epi, splits, 16 * cfg.mb, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -500,10 +507,20 @@ extern "C" size_t axm_qmm_q4_tile16_workspace_bytes(int K, int N, int swiglu) {
   return t16_gemm_ws_bytes(K, (N + 15) / 16, swiglu ? 2 : 1);
 }
 
+extern "C" size_t axm_qmm_q4_tile16_rows_workspace_bytes(int M, int K, int N, int swiglu) {
+  if (M <= 0 || K <= 0 || N <= 0) return 0;
+  return M <= kTile16GemmMaxTokens ? axm_qmm_q4_tile16_workspace_bytes(K, N, swiglu)
+                                   : t16_rows_gemm_ws_bytes(M, K, (N + 15) / 16, swiglu ? Q4_EPI_SWIGLU : Q4_EPI_STORE);
+}
+
 static int qmm_tile16_rows(const void* x, const void* w16, const void* sb16, const void* bias, void* y, int M, int K,
                            int N, int group_size, int epi, void* ws, size_t ws_bytes, hipStream_t s) {
-  for (int m0 = 0; m0 < M; m0 += kTile16GemmMaxTokens) {
-    const int mc = (M - m0) < kTile16GemmMaxTokens ? (M - m0) : kTile16GemmMaxTokens;
+  // Rows past 64: one launch of the many-row GEMM (rows of x that its 16-byte loads cannot
+  // take go through the 64-row passes).
+  const bool rows = M > kTile16GemmMaxTokens && ((uintptr_t)x & 15) == 0;
+  const int step = rows ? M : kTile16GemmMaxTokens;
+  for (int m0 = 0; m0 < M; m0 += step) {
+    const int mc = (M - m0) < step ? (M - m0) : step;
     T16Args a{};
     a.x = (const f16*)x + (size_t)m0 * K;
     a.ldx = K;
@@ -522,7 +539,8 @@ static int qmm_tile16_rows(const void* x, const void* w16, const void* sb16, con
     a.y = (f16*)y + (size_t)m0 * N;
     a.ldy = N;
     a.bias = (const f16*)bias;
-    const int rc = t16_gemm_launch(a, mc, epi, (float*)ws, ws_bytes, s);
+    const int rc = rows ? t16_rows_gemm_launch(a, mc, epi, (float*)ws, ws_bytes, s)
+                        : t16_gemm_launch(a, mc, epi, (float*)ws, ws_bytes, s);
     if (rc) return rc;
   }
   return 0;

@@ -2,6 +2,7 @@
 // the persistent decode-step kernel).
 #pragma once
 #include "axm_common.h"
+#include "q4_tile16.h"
 
 // Nibble expansion: (w & mask) | magic as one v_and_or_b32.  gfx950 VOP3 takes
 // neither literals nor two scalar operands, so the masks must sit in VGPRs and
@@ -49,3 +50,69 @@ __device__ __forceinline__ f16x8 unpack_word(uint32_t w, const Unpack& u) {
 
 __device__ __forceinline__ float t16_silu(float g) { return g / (1.0f + expf(-g)); }
 
+// One output element of the epilogue (identical arithmetic to the GEMV's):
+// v0 the gate / plain accumulator, v1 the up accumulator (SwiGLU).
+template <int EPI>
+__device__ __forceinline__ void t16g_store(const T16Args& a, int tok, int row, float v0, float v1) {
+  if (EPI == Q4_EPI_SWIGLU) {
+    const f16 g = f2h(v0);
+    const f16 u = f2h(v1);
+    const f16 sg = f2h(t16_silu(h2f(g)));
+    a.y[(size_t)tok * a.ldy + row] = f2h(h2f(sg) * h2f(u));
+  } else {
+    f16 h = f2h(v0);
+    if (a.bias != nullptr) h = f2h(h2f(h) + h2f(a.bias[row]));
+    if (EPI == Q4_EPI_STORE) {
+      a.y[(size_t)tok * a.ldy + row] = h;
+    } else {
+      f16* xr = a.resid + (size_t)tok * a.ldr + row;
+      *xr = f2h(h2f(*xr) + h2f(h));
+    }
+  }
+}
+
+// The same for four consecutive output rows of one token (the accumulators of a lane when
+// the weights are the MFMA's row operand): one 8-byte access each of the residual / output
+// row and the bias where t16g_vec4 allows it, else element by element up to row N.
+template <int EPI>
+__device__ __forceinline__ void t16g_store4(const T16Args& a, int tok, int row, f32x4 v0, f32x4 v1, bool vec) {
+  if (!vec) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (row + e < a.N) t16g_store<EPI>(a, tok, row + e, v0[e], v1[e]);
+    return;
+  }
+  f16x4 h;
+  if (EPI == Q4_EPI_SWIGLU) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f16 g = f2h(v0[e]);
+      const f16 u = f2h(v1[e]);
+      h[e] = f2h(h2f(f2h(t16_silu(h2f(g)))) * h2f(u));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = f2h(v0[e]);
+    if (a.bias != nullptr) {
+      const f16x4 b = *reinterpret_cast<const f16x4*>(a.bias + row);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = f2h(h2f(h[e]) + h2f(b[e]));
+    }
+  }
+  if (EPI == Q4_EPI_RESID) {
+    f16x4* xr = reinterpret_cast<f16x4*>(a.resid + (size_t)tok * a.ldr + row);
+    f16x4 x = *xr;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = f2h(h2f(x[e]) + h2f(h[e]));
+    *xr = x;
+  } else {
+    *reinterpret_cast<f16x4*>(a.y + (size_t)tok * a.ldy + row) = h;
+  }
+}
+// Whether every 4-row access of t16g_store4 is whole and 8-byte aligned.
+template <int EPI>
+__device__ __forceinline__ bool t16g_vec4(const T16Args& a) {
+  const int ld = EPI == Q4_EPI_RESID ? a.ldr : a.ldy;
+  const uintptr_t p = EPI == Q4_EPI_RESID ? (uintptr_t)a.resid : (uintptr_t)a.y;
+  return a.N % 4 == 0 && ld % 4 == 0 && ((p | (uintptr_t)a.bias) & 7) == 0;
+}

@@ -195,8 +195,8 @@ def tile16_group_size(w16, sb16) -> int:
     raise ValueError(f"tile16 copy: {wb} code bytes and {sbb} scale bytes match neither group size")
 
 
-def _qmm_workspace(K: int, N: int, swiglu: bool, device):
-    n = _lib.lib().axm_qmm_q4_tile16_workspace_bytes(K, N, int(swiglu))
+def _qmm_workspace(M: int, K: int, N: int, swiglu: bool, device):
+    n = _lib.lib().axm_qmm_q4_tile16_rows_workspace_bytes(M, K, N, int(swiglu))
     return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
 
 
@@ -223,7 +223,7 @@ def qmv_q4_tile16(x, w16, sb16, out_features: int, bias=None) -> torch.Tensor:
                                                 _lib.ptr(y), M, K, N, gs, _lib.stream_of(x.device)),
                    "qmv_q4_tile16")
         return y
-    ws, n = _qmm_workspace(K, N, False, x.device)
+    ws, n = _qmm_workspace(M, K, N, False, x.device)
     _lib.check(_lib.lib().axm_qmm_q4_tile16(_lib.ptr(xc), _lib.ptr(w16), _lib.ptr(sb16), _lib.ptr(b), _lib.ptr(y),
                                             M, K, N, gs, _lib.ptr(ws), n, _lib.stream_of(x.device)),
                "qmm_q4_tile16")
@@ -271,7 +271,7 @@ def qmv_q4_tile16_swiglu(x, ln_w, eps: float, gu16, gusb16, H: int) -> torch.Ten
         raise RuntimeError("qmv_q4_tile16_swiglu: x must be float16")
     xn = (fused_rmsnorm(x.reshape(M, K), ln_w, eps) if ln_w is not None else x.reshape(M, K)).contiguous()
     y = torch.empty((*x.shape[:-1], int(H)), dtype=torch.float16, device=x.device)
-    ws, n = _qmm_workspace(K, int(H), True, x.device)
+    ws, n = _qmm_workspace(M, K, int(H), True, x.device)
     _lib.check(_lib.lib().axm_qmm_q4_tile16_swiglu(_lib.ptr(xn), _lib.ptr(gu16.contiguous()),
                                                    _lib.ptr(gusb16.contiguous()), _lib.ptr(y), M, K, int(H), gs,
                                                    _lib.ptr(ws), n, _lib.stream_of(x.device)),

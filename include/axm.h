@@ -75,6 +75,9 @@ int axm_qmv_q4_tile16_swiglu(const void* x, const void* ln_w, float eps, const v
  * K is split across workgroups; `workspace` holds the fp32 partial tiles
  * (axm_qmm_q4_tile16_workspace_bytes: enough for any M, 0 when no split is used). */
 size_t axm_qmm_q4_tile16_workspace_bytes(int K, int N, int swiglu);
+/* The workspace that M rows use best: from 65 rows on one launch of the many-row GEMM, which
+ * splits K where M and N leave CUs idle, as far as the workspace given allows. */
+size_t axm_qmm_q4_tile16_rows_workspace_bytes(int M, int K, int N, int swiglu);
 int axm_qmm_q4_tile16(const void* x, const void* w16, const void* sb16, const void* bias, void* y, int M, int K,
                       int N, int group_size, void* workspace, size_t workspace_bytes, void* stream);
 /* silu(g) * u over the tile16 [W_gate; W_up] copy for M tokens whose activations are
