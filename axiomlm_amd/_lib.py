@@ -103,6 +103,12 @@ _SIGNATURES = {
     "axm_runner_create": (c_int, [c_void_p, c_void_p]),
     "axm_runner_destroy": (None, [c_void_p]),
     "axm_runner_step": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_void_p]),
+    "axm_runner_prompt_workspace_bytes": (c_size_t, [c_void_p, c_int]),
+    "axm_runner_prompt_step": (
+        c_int,
+        [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p,
+         ctypes.POINTER(c_void_p)],
+    ),
     "axm_runner_verify_step": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "axm_runner_verify_tree_step": (
         c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, ctypes.POINTER(c_int),

@@ -1250,7 +1250,9 @@ __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows
   }
 }
 
-template <int KVT, int HD>
+// CAUSAL: the T nodes are consecutive tokens at slots prefix + t (no masks, any T); node t
+// sees keys [0, prefix + t], so a row block walks the keys up to its last row's only.
+template <int KVT, int HD, bool CAUSAL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) tree_mfma_kernel(AttnParams p) {
   constexpr int KSTEPS = HD / 32;  // MFMA k-steps over the head dimension
   constexpr int DT = HD / 16;      // 16-wide output dimension tiles
@@ -1266,10 +1268,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   const int l16 = lane & 15, lq = lane >> 4;
   const int kvh = blockIdx.x;
   const int R = p.T * p.n_rep;
-  const int row0 = blockIdx.y * kTreeRows + wave * 16;
+  // The row blocks with the most keys start first.
+  const int rblk = CAUSAL ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y;
+  const int row0 = rblk * kTreeRows + wave * 16;
   const int split = blockIdx.z;
   const int prefix = p.prefix_len;
-  const int n_keys = prefix + p.T;
+  const int n_keys = prefix + (CAUSAL ? min(p.T, (rblk * kTreeRows + kTreeRows - 1) / p.n_rep + 1) : p.T);
   const int per = (n_keys + p.n_splits - 1) / p.n_splits;
   const int k_begin = min(split * per, n_keys);
   const int k_end = min(k_begin + per, n_keys);
@@ -1281,6 +1285,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   // write_pos < S), so one conditional subtraction wraps it.  Selects only: a
   // branch here split the loop body and cost the key buffers their registers.
   auto slot_of = [&](int key) {
+    if (CAUSAL) return key;
     const int w = p.write_pos + (key - prefix);
     const int wrapped = w >= p.kv.S ? w - p.kv.S : w;
     return key < prefix ? key : wrapped;
@@ -1326,6 +1331,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   }
   // D-tile rows of this lane: row0 + 4 lq + v.
   uint64_t mask[4];
+  int key_end[4];  // CAUSAL: keys the row sees
   bool row_ok[4];
   float m[4], l[4];
   f32x4 o[DT];
@@ -1333,7 +1339,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   for (int v = 0; v < 4; ++v) {
     const int r = row0 + 4 * lq + v;
     row_ok[v] = r < R;
-    mask[v] = row_ok[v] ? p.masks[r / p.n_rep] : 0ull;
+    if (CAUSAL) key_end[v] = row_ok[v] ? min(k_end, prefix + r / p.n_rep + 1) : 0;
+    else mask[v] = row_ok[v] ? p.masks[r / p.n_rep] : 0ull;
     m[v] = kNegBig;
     l[v] = 0.f;
   }
@@ -1385,8 +1392,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int key = kb0 + 16 * h + l16;
-        const bool in_tree = ((mask[v] >> ((key - prefix) & 63)) & 1ull) != 0;
-        const bool vis = row_ok[v] && key < k_end && (key < prefix || in_tree);
+        bool vis;
+        if (CAUSAL) {
+          vis = key < key_end[v];
+        } else {
+          const bool in_tree = ((mask[v] >> ((key - prefix) & 63)) & 1ull) != 0;
+          vis = row_ok[v] && key < k_end && (key < prefix || in_tree);
+        }
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
@@ -1435,17 +1447,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   }
 }
 
-template <int HD>
+template <int HD, bool CAUSAL>
 int launch_tree_mfma(const AttnParams& p, dim3 grid, hipStream_t s) {
   switch (p.kv.kv_dtype) {
     case AXM_KV_FP16:
-      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_FP16, HD>), grid, dim3(256), 0, s, p);
+      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_FP16, HD, CAUSAL>), grid, dim3(256), 0, s, p);
       return 0;
     case AXM_KV_FP8:
-      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_FP8, HD>), grid, dim3(256), 0, s, p);
+      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_FP8, HD, CAUSAL>), grid, dim3(256), 0, s, p);
       return 0;
     case AXM_KV_INT4:
-      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_INT4, HD>), grid, dim3(256), 0, s, p);
+      hipLaunchKernelGGL((tree_mfma_kernel<AXM_KV_INT4, HD, CAUSAL>), grid, dim3(256), 0, s, p);
       return 0;
   }
   axm_set_error("tree attention: bad kv dtype %d", p.kv.kv_dtype);
@@ -1697,7 +1709,7 @@ int launch_tree_attention(const f16* q, const KvView& kv, f16* out, int Hq, int 
   int rc;
   if (kv.B == 1 && (kv.hd == 64 || kv.hd == 128) && T <= kv.S) {
     const dim3 grid(kv.Hkv, (rows + kTreeRows - 1) / kTreeRows, n_splits);
-    rc = kv.hd == 128 ? launch_tree_mfma<128>(p, grid, s) : launch_tree_mfma<64>(p, grid, s);
+    rc = kv.hd == 128 ? launch_tree_mfma<128, false>(p, grid, s) : launch_tree_mfma<64, false>(p, grid, s);
   } else {
     const int qr = pick_qr(rows);
     dim3 grid(kv.Hkv * ((rows + qr - 1) / qr), n_splits, 1);
@@ -1706,6 +1718,32 @@ int launch_tree_attention(const f16* q, const KvView& kv, f16* out, int Hq, int 
   if (rc) return rc;
   if (n_splits > 1)
     launch_attn_reduce(ws, out, T * Hq, n_splits, kv.hd, s);
+  return 0;
+}
+
+int launch_prompt_attention(const f16* q, const KvView& kv, f16* out, int Hq, int T, int prefix_len, int n_splits,
+                            float* ws, hipStream_t s) {
+  if (kv.B != 1 || (kv.hd != 64 && kv.hd != 128) || prefix_len + T > kv.S) {
+    axm_set_error("prompt attention: batch %d, head size %d (64 / 128), %d + %d tokens in %d slots", kv.B, kv.hd,
+                  prefix_len, T, kv.S);
+    return -2;
+  }
+  AttnParams p{};
+  p.q = q;
+  p.kv = kv;
+  p.out = out;
+  p.ws = ws;
+  p.Hq = Hq;
+  p.n_rep = Hq / kv.Hkv;
+  p.n_splits = n_splits;
+  p.prefix_len = prefix_len;
+  p.T = T;
+  p.write_pos = prefix_len;
+  p.scale_log2 = kLog2e / sqrtf((float)kv.hd);
+  const dim3 grid(kv.Hkv, (T * p.n_rep + kTreeRows - 1) / kTreeRows, n_splits);
+  const int rc = kv.hd == 128 ? launch_tree_mfma<128, true>(p, grid, s) : launch_tree_mfma<64, true>(p, grid, s);
+  if (rc) return rc;
+  if (n_splits > 1) launch_attn_reduce(ws, out, T * Hq, n_splits, kv.hd, s);
   return 0;
 }
 

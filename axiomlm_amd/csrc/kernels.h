@@ -123,3 +123,7 @@ int launch_tree_attention(const f16* q, const KvView& kv, f16* out, int Hq, int 
 size_t tree_workspace_bytes(int T, int Hq, int hd, int n_splits);
 // Key splits for tree attention (about two 64-row workgroups per CU, >= 64 keys each).
 int tree_choose_splits(int T, int Hq, int Hkv, int n_keys);
+// Causal attention of T consecutive tokens (any T) over slots [0, prefix_len + t]: their keys and
+// values are in the cache at slots prefix_len + t already.  Splits and workspace as the tree's.
+int launch_prompt_attention(const f16* q, const KvView& kv, f16* out, int Hq, int T, int prefix_len, int n_splits,
+                            float* ws, hipStream_t s);

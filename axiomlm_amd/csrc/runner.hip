@@ -142,6 +142,12 @@ __global__ void set_tree_kernel(TreeParams p, int T, int* pos_dev, unsigned long
   }
 }
 
+// RoPE positions of T consecutive tokens.
+__global__ void set_chain_kernel(int* pos_dev, int T, int start_pos, int rope_len) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < T) pos_dev[t] = (int)(((long long)start_pos + t) % rope_len);
+}
+
 // Multi-token RoPE (rope_tree_kv_cache_write_half_kernel, metal_kernels.metal:2862-2918):
 // token t of qkv [T][qkv_dim] (bias already added) is rotated at pos_dev[t]; q rows go to
 // q [T][q_dim], rotated k and raw v rows to kv [T][2 kv_dim] for the cache writer.
@@ -630,11 +636,12 @@ struct axm_runner {
   // Q8_G64 (format 1) or fp16 (format 2) lm_head over T rows into logits: with ln_w the
   // GEMV applies the final RMSNorm itself and writes the normalized rows to xn_out (one
   // launch where a separate norm took two); without, the rows are normalized already.
-  int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s) {
+  int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s, f16* out = nullptr) {
+    if (out == nullptr) out = logits;
     if (d.lm_head_format == 2)
-      return launch_f16_gemv(x, (const f16*)d.lm_head_w, nullptr, logits, T, d.d_model, d.vocab_size, ln_w, d.eps,
+      return launch_f16_gemv(x, (const f16*)d.lm_head_w, nullptr, out, T, d.d_model, d.vocab_size, ln_w, d.eps,
                              s, xn_out);
-    return launch_q8_gemv(x, (const uint8_t*)d.lm_head_w, (const f16*)d.lm_head_sb, nullptr, logits, T, d.d_model,
+    return launch_q8_gemv(x, (const uint8_t*)d.lm_head_w, (const f16*)d.lm_head_sb, nullptr, out, T, d.d_model,
                           d.vocab_size, ln_w, d.eps, s, xn_out);
   }
 
@@ -696,21 +703,32 @@ struct axm_runner {
     return m.fmt != 0 ? run_dense(m, epi, out_rows, c, M, s) : run_gemv(m, epi, out_rows, c, M, s);
   }
 
+  // Buffers of a multi-token step: the runner's own (verify), or a caller's workspace (prompt).
+  struct RowBufs {
+    f16 *x, *norm, *q, *attn_y, *hbuf, *qkvbuf, *kvst;
+    int* pos;
+    float* ws;
+    size_t ws_bytes;
+  };
+  RowBufs own_bufs() const { return {x, norm, q, attn_y, hbuf, qkvbuf, kvst, tree_pos, ws, ws_bytes}; }
+
   // GEMV over T token rows in launches of at most 4 rows, or the multi-token GEMM
   // from kGemmMinTokens rows on.
-  int gemv_rows(const Mat& m, int epi, int out_rows, GemvCall c, int T, hipStream_t s) {
+  int gemv_rows(const RowBufs& b, const Mat& m, int epi, int out_rows, GemvCall c, int T, hipStream_t s) {
     if (m.w16 != nullptr && T >= kGemmMinTokens && c.argmax_keys == nullptr && c.q_dim == 0 &&
         (epi == Q4_EPI_STORE || epi == Q4_EPI_RESID || epi == Q4_EPI_SWIGLU)) {
       // Multi-token GEMM: up to 64 tokens per weight pass, activations normalized first
       // (into x_norm_out when the caller wants them, else into the norm scratch).
       const f16* xall = c.x;
       if (c.ln_w != nullptr) {
-        f16* nrm = c.x_norm_out ? c.x_norm_out : norm;
+        f16* nrm = c.x_norm_out ? c.x_norm_out : b.norm;
         launch_rmsnorm(c.x, c.ln_w, nrm, T, m.K, c.eps, s);
         xall = nrm;
       }
-      for (int t0 = 0; t0 < T; t0 += kTile16GemmMaxTokens) {
-        const int mc = (T - t0) < kTile16GemmMaxTokens ? (T - t0) : kTile16GemmMaxTokens;
+      const bool many = T > kTile16GemmMaxTokens;  // one launch of the many-row GEMM
+      const int step = many ? T : kTile16GemmMaxTokens;
+      for (int t0 = 0; t0 < T; t0 += step) {
+        const int mc = (T - t0) < step ? (T - t0) : step;
         const f16* xin = xall + (size_t)t0 * c.ldx;
         T16Args a{};
         a.x = xin;
@@ -732,8 +750,9 @@ struct axm_runner {
         a.post_ln_w = c.post_ln_w;
         a.post_norm_out = c.post_ln_w ? c.post_norm_out + (size_t)t0 * out_rows : nullptr;
         a.eps = c.eps;
-        a.split_info = T <= kTile16GemmMaxTokens ? c.split_info : nullptr;
-        const int rc = t16_gemm_launch(a, mc, epi, ws, ws_bytes, s);
+        a.split_info = c.split_info;
+        const int rc = many ? t16_rows_gemm_launch(a, mc, epi, b.ws, b.ws_bytes, s)
+                            : t16_gemm_launch(a, mc, epi, b.ws, b.ws_bytes, s);
         if (rc) return rc;
       }
       return 0;
@@ -754,12 +773,20 @@ struct axm_runner {
     return 0;
   }
 
-  // Multi-token step (verify_step / verify_tree_step, mps_kernels.mm:3265-3464).
-  // tree: token t is rotated at start_pos + depth[t], written to slot
+  enum AttnMode { kAttnTree, kAttnAllSlots, kAttnPrompt };
+
+  // The layers of a multi-token step (verify_step / verify_tree_step, mps_kernels.mm:3265-3464).
+  // kAttnTree: token t is rotated at start_pos + depth[t], written to slot
   // (write_pos + t) % S and attends to [0, prefix) plus the tree slots its mask
-  // selects.  !tree (ring wrap-around): all T rows are written, then every token
-  // attends over all S slots, as the reference does in that case.
-  int enqueue_verify(const int64_t* idx_dev, int T, int write_pos, int prefix, bool tree, hipStream_t s) {
+  // selects.  kAttnAllSlots (ring wrap-around): all T rows are written, then every
+  // token attends over all S slots, as the reference does in that case.  kAttnPrompt: T
+  // consecutive tokens at slots prefix + t (prefix == write_pos), each seeing the slots up to
+  // its own.
+  int enqueue_rows(const RowBufs& b, const int64_t* idx_dev, int T, int write_pos, int prefix, AttnMode mode,
+                   hipStream_t s) {
+    f16 *const x = b.x, *const norm = b.norm, *const q = b.q, *const attn_y = b.attn_y, *const hbuf = b.hbuf,
+               *const qkvbuf = b.qkvbuf, *const kvst = b.kvst;
+    float* const ws = b.ws;
     const int D = d.d_model, H = d.hidden_dim;
     // Multi-token GEMMs take normalized activations: there the residual GEMMs
     // (O, down) also write the RMSNorm of the rows they update into `norm` for
@@ -784,22 +811,25 @@ struct axm_runner {
       // cache-write launch, which sums them (no separate split reduce).
       int split_info[3] = {0, 0, 0};
       if (d.head_dim == 128) a.split_info = split_info;
-      int rc = gemv_rows(m_qkv[i], Q4_EPI_STORE, qkv_dim, a, T, s);
+      int rc = gemv_rows(b, m_qkv[i], Q4_EPI_STORE, qkv_dim, a, T, s);
       if (rc) return rc;
       if (d.head_dim == 128) {
         // RoPE and the cache write in one launch.
         if (split_info[0] > 1)
           rc = launch_reduce_rope_kv_write(kv, ws, split_info[0], split_info[1], split_info[2], a.bias, d.n_head, T,
-                                           d.freqs, tree_pos, q, write_pos, s);
+                                           d.freqs, b.pos, q, write_pos, s);
         else
-          rc = launch_rope_kv_write(kv, qkvbuf, d.n_head, T, d.freqs, tree_pos, q, write_pos, s);
+          rc = launch_rope_kv_write(kv, qkvbuf, d.n_head, T, d.freqs, b.pos, q, write_pos, s);
         if (rc) return rc;
       } else {
         hipLaunchKernelGGL(rope_tokens_kernel, dim3((qkv_dim / 8 + 255) / 256, T), dim3(256), 0, s, qkvbuf, q_dim,
-                           kv_dim, d.head_dim, d.freqs, tree_pos, q, kvst);
+                           kv_dim, d.head_dim, d.freqs, b.pos, q, kvst);
         launch_kv_write(kv, kvst, kvst + kv_dim, 2 * kv_dim, T, write_pos, nullptr, s);
       }
-      if (tree) {
+      if (mode == kAttnPrompt) {
+        const int splits = tree_choose_splits(T, d.n_head, d.n_kv_head, prefix + T);
+        rc = launch_prompt_attention(q, kv, attn_y, d.n_head, T, prefix, splits, ws, s);
+      } else if (mode == kAttnTree) {
         const int splits = tree_choose_splits(T, d.n_head, d.n_kv_head, prefix + T);
         rc = launch_tree_attention(q, kv, attn_y, d.n_head, T, prefix, write_pos, (const uint64_t*)tree_mask, splits, ws,
                                    s);
@@ -820,7 +850,7 @@ struct axm_runner {
         o.post_norm_out = norm;
         o.eps = d.eps;
       }
-      rc = gemv_rows(m_o[i], Q4_EPI_RESID, D, o, T, s);
+      rc = gemv_rows(b, m_o[i], Q4_EPI_RESID, D, o, T, s);
       if (rc) return rc;
       GemvCall g{};
       g.x = post ? norm : x;
@@ -830,7 +860,7 @@ struct axm_runner {
       g.ln_w = post ? nullptr : (const f16*)ln2[i];
       g.eps = d.eps;
       g.pair_rows = H;
-      rc = gemv_rows(m_gu[i], Q4_EPI_SWIGLU, H, g, T, s);
+      rc = gemv_rows(b, m_gu[i], Q4_EPI_SWIGLU, H, g, T, s);
       if (rc) return rc;
       GemvCall dn{};
       dn.x = hbuf;
@@ -842,9 +872,19 @@ struct axm_runner {
         dn.post_norm_out = norm;
         dn.eps = d.eps;
       }
-      rc = gemv_rows(m_dn[i], Q4_EPI_RESID, D, dn, T, s);
+      rc = gemv_rows(b, m_dn[i], Q4_EPI_RESID, D, dn, T, s);
       if (rc) return rc;
     }
+    return 0;
+  }
+
+  // verify_step / verify_tree_step: the layers, then the logits of every token.
+  int enqueue_verify(const int64_t* idx_dev, int T, int write_pos, int prefix, bool tree, hipStream_t s) {
+    const RowBufs b = own_bufs();
+    const int D = d.d_model;
+    const bool post = T >= kGemmMinTokens;
+    const int rc = enqueue_rows(b, idx_dev, T, write_pos, prefix, tree ? kAttnTree : kAttnAllSlots, s);
+    if (rc) return rc;
     if (d.lm_head_format == 0) {
       GemvCall l{};
       l.x = post ? norm : x;
@@ -854,10 +894,78 @@ struct axm_runner {
       l.ln_w = post ? nullptr : (const f16*)d.lnf_w;
       l.eps = d.eps;
       l.x_norm_out = post ? nullptr : norm;
-      return gemv_rows(m_lmh, Q4_EPI_STORE, d.vocab_size, l, T, s);
+      return gemv_rows(b, m_lmh, Q4_EPI_STORE, d.vocab_size, l, T, s);
     }
     if (!post) return lm_head_dense(x, T, (const f16*)d.lnf_w, norm, s);
     return lm_head_dense(norm, T, nullptr, nullptr, s);
+  }
+
+  // Workspace of a prompt step of T rows: RowBufs laid out from `base` (null: sizes only).
+  size_t prompt_bufs(int T, unsigned char* base, RowBufs* b) const {
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+      unsigned char* p = base + off;
+      off += (bytes + 255) & ~(size_t)255;
+      return p;
+    };
+    const size_t D = d.d_model, h = sizeof(f16);
+    RowBufs r{};
+    r.x = (f16*)take(T * D * h);
+    r.norm = (f16*)take(T * D * h);
+    r.q = (f16*)take((size_t)T * q_dim * h);
+    r.attn_y = (f16*)take((size_t)T * q_dim * h);
+    r.hbuf = (f16*)take((size_t)T * d.hidden_dim * h);
+    r.qkvbuf = (f16*)take((size_t)T * qkv_dim * h);
+    r.kvst = (f16*)take(d.head_dim == 128 ? 0 : (size_t)T * 2 * kv_dim * h);
+    r.pos = (int*)take((size_t)T * sizeof(int));
+    // Attention partials and GEMM partial tiles share one region.  The split count falls
+    // with the number of keys, so the longest prefix bounds it.
+    size_t w = tree_workspace_bytes(T, d.n_head, d.head_dim,
+                                    tree_choose_splits(T, d.n_head, d.n_kv_head, d.max_seq_len));
+    auto gemm = [&](const Mat& m, int rows, int epi) {
+      if (m.w16 == nullptr) return;
+      const size_t g = T > kTile16GemmMaxTokens ? t16_rows_gemm_ws_bytes(T, m.K, (rows + 15) / 16, epi)
+                                                : t16_gemm_ws_bytes(m.K, (rows + 15) / 16, epi == Q4_EPI_SWIGLU ? 2 : 1);
+      w = g > w ? g : w;
+    };
+    gemm(m_qkv[0], qkv_dim, Q4_EPI_STORE);
+    gemm(m_o[0], d.d_model, Q4_EPI_RESID);
+    gemm(m_gu[0], d.hidden_dim, Q4_EPI_SWIGLU);
+    gemm(m_dn[0], d.d_model, Q4_EPI_RESID);
+    gemm(m_lmh, d.vocab_size, Q4_EPI_STORE);
+    r.ws = (float*)take(w);
+    r.ws_bytes = w;
+    if (b != nullptr) *b = r;
+    return off;
+  }
+
+  // Prompt step: the layers over all T rows, the last norm_rows normalized rows to `norm`
+  // (get_last_norm), and the logits of the last row (n_logits 1, into `logits`), of all rows
+  // (T, into logits_all) or of none (0).  One pass over the weights for all rows (the
+  // many-row GEMM) instead of one per 32: 1000 tokens through four 7B layers and the head
+  // took 32 chunks of ~45 launches, 10.9 ms; in one pass 2.05 ms, of which the GEMMs 1.66
+  // and the causal attention 0.22.
+  int enqueue_prompt(const RowBufs& b, const int64_t* idx_dev, int T, int start_pos, int write_pos, int norm_rows,
+                     int n_logits, f16* logits_all, hipStream_t s) {
+    const int D = d.d_model;
+    hipLaunchKernelGGL(set_chain_kernel, dim3((T + 255) / 256), dim3(256), 0, s, b.pos, T, start_pos, d.rope_len);
+    int rc = enqueue_rows(b, idx_dev, T, write_pos, write_pos, kAttnPrompt, s);
+    if (rc) return rc;
+    if (norm_rows > 0 && hipMemcpyAsync(norm, b.norm + (size_t)(T - norm_rows) * D, (size_t)norm_rows * D * sizeof(f16),
+                                        hipMemcpyDeviceToDevice, s) != hipSuccess) {
+      axm_set_error("runner_prompt_step: norm copy failed");
+      return -5;
+    }
+    if (n_logits == 0) return 0;
+    const f16* rows = n_logits == 1 ? b.norm + (size_t)(T - 1) * D : b.norm;
+    f16* out = n_logits == 1 ? logits : logits_all;
+    if (d.lm_head_format != 0) return lm_head_dense(rows, n_logits, nullptr, nullptr, s, out);
+    GemvCall l{};
+    l.x = rows;
+    l.ldx = D;
+    l.y = out;
+    l.ldy = d.vocab_size;
+    return gemv_rows(b, m_lmh, Q4_EPI_STORE, d.vocab_size, l, n_logits, s);
   }
 
   // Re-tile one matrix for the matrix-core GEMV (runner-owned copy).
@@ -1287,6 +1395,37 @@ extern "C" int axm_runner_verify_tree_step(axm_runner_t r, const void* idx_dev, 
                 prefix_len);
   return verify_common(r, idx_dev, T, start_pos, write_pos, prefix_len, depths_host,
                        (const unsigned long long*)masks_host, true, stream, logits_out);
+}
+
+extern "C" size_t axm_runner_prompt_workspace_bytes(axm_runner_t r, int T) {
+  return r == nullptr || T < kGemmMinTokens ? 0 : r->prompt_bufs(T, nullptr, nullptr);
+}
+
+extern "C" int axm_runner_prompt_step(axm_runner_t r, const void* idx_dev, int T, int start_pos, int write_pos,
+                                      int norm_rows, int n_logits, void* logits_all, void* workspace,
+                                      size_t workspace_bytes, void* stream, void** logits_out) {
+  AXM_CHECK_ARG(r && idx_dev, -1, "runner_prompt_step: null argument");
+  const axm_runner_desc& d = r->d;
+  AXM_CHECK_ARG(T >= kGemmMinTokens, -1, "runner_prompt_step: T=%d below %d", T, kGemmMinTokens);
+  AXM_CHECK_ARG(start_pos >= 0 && write_pos >= 0 && write_pos <= d.max_seq_len - T, -1,
+                "runner_prompt_step: %d rows at slot %d of %d", T, write_pos, d.max_seq_len);
+  AXM_CHECK_ARG(norm_rows >= 0 && norm_rows <= T && norm_rows <= d.max_tokens, -1,
+                "runner_prompt_step: norm_rows %d outside [0, %d]", norm_rows, d.max_tokens);
+  AXM_CHECK_ARG(n_logits == 0 || n_logits == 1 || (n_logits == T && logits_all), -1,
+                "runner_prompt_step: logits of 0, 1 or all %d rows (the last into logits_all)", T);
+  const size_t need = r->prompt_bufs(T, nullptr, nullptr);
+  AXM_CHECK_ARG(workspace && ((uintptr_t)workspace & 255) == 0 && workspace_bytes >= need, -1,
+                "runner_prompt_step: 256-byte aligned workspace of %zu bytes needed, %zu given", need,
+                workspace_bytes);
+  axm_runner::RowBufs b;
+  r->prompt_bufs(T, (unsigned char*)workspace, &b);
+  r->tok_next_valid = false;
+  const int rc = r->enqueue_prompt(b, (const int64_t*)idx_dev, T, start_pos, write_pos, norm_rows, n_logits,
+                                   (f16*)logits_all, (hipStream_t)stream);
+  if (rc) return rc;
+  AXM_LAUNCH_CHECK("runner_prompt_step");
+  if (logits_out) *logits_out = n_logits == T ? logits_all : r->logits;
+  return 0;
 }
 
 // ---------------------------------------------------------------------------

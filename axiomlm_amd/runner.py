@@ -268,6 +268,34 @@ class QuantizedDecodeRunner:
         self._keep_tokens = t
         return _RawBuffer.view(out.value, T * self.vocab_size, self.device).view(1, T, self.vocab_size)
 
+    def prompt_step(self, idx, start_pos: int, write_pos: int, logits: str = "last",
+                    norm_rows: int = 0) -> torch.Tensor | None:
+        """A chain of T >= 4 consecutive tokens (any number, unlike ``verify_step``) in one pass over the
+        weights: written at slots write_pos.. (contiguous), each attending to the slots up to its own.
+        ``logits``: "last" -> (1, 1, V), a view of the runner's buffer; "all" -> (1, T, V), a new
+        tensor; "none" -> None.  The last ``norm_rows`` normalized rows are left for ``get_last_norm``."""
+        if logits not in ("last", "all", "none"):
+            raise ValueError(f"logits must be 'last', 'all' or 'none', got {logits!r}")
+        t = self._tokens(idx)
+        T = int(t.numel())
+        n = _lib.lib().axm_runner_prompt_workspace_bytes(self._h, T)
+        # The pass's activations: torch's allocator hands them out per call, in stream order.
+        ws = torch.empty(n, dtype=torch.uint8, device=self.device)
+        out_all = (torch.empty((1, T, self.vocab_size), dtype=torch.float16, device=self.device)
+                   if logits == "all" else None)
+        out = ctypes.c_void_p()
+        rc = _lib.lib().axm_runner_prompt_step(
+            self._h, _lib.ptr(t), T, int(start_pos), int(write_pos), int(norm_rows),
+            {"last": 1, "all": T, "none": 0}[logits], _lib.ptr(out_all), _lib.ptr(ws), n,
+            _lib.stream_of(self.device), ctypes.byref(out))
+        _lib.check(rc, "QuantizedDecodeRunner.prompt_step")
+        self._keep_tokens = t
+        if logits == "none":
+            return None
+        if out_all is not None:
+            return out_all
+        return _RawBuffer.view(out.value, self.vocab_size, self.device).view(1, 1, self.vocab_size)
+
     def verify_tree_step(self, idx, start_pos: int, write_pos: int, prefix_len: int, depths, masks) -> torch.Tensor:
         """Tree verification -> logits (1, T, V) (mps_kernels.mm:3265-3357).  ``masks[u]`` has bit j set
         when tree node j is visible to node u (Python ints, up to 64 nodes)."""

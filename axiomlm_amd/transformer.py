@@ -16,8 +16,8 @@ optional QKV bias), the reference's
 
 Weights are plain tensors named as in the reference ``state_dict`` (``transformer.wte.weight``,
 ``transformer.h.{i}.attn.c_attn.weight``, ...), so a reference checkpoint's tensors load
-unchanged.  Every kernel runs on the GPU; there is no CPU fallback: sequences longer than
-the runner's multi-token capacity are fed as consecutive ``verify_step`` chunks.
+unchanged.  Every kernel runs on the GPU; there is no CPU fallback: prompts longer than a
+verify chunk are read by the runner's ``prompt_step``, all rows in one pass over the weights.
 """
 
 from __future__ import annotations
@@ -31,6 +31,11 @@ import torch
 from .cache import StaticKVCache
 from .kernels import pack_linear_q4_marlin, pack_linear_q8_g64
 from .runner import DecodeRunner, QuantizedDecodeRunner
+
+VERIFY_CHUNK = 32  # tokens of a verify chunk: the shortest prompts, and those over the end of a ring cache
+# Most tokens of one prompt step: bounds its activations (160 MB at the 7B shape) while every pass over the
+# weights still serves many rows.
+PROMPT_ROWS = 2048
 
 
 @dataclass
@@ -250,6 +255,15 @@ class Transformer:
                        for b in bias],
             k_scales=cache0.k_scales, v_scales=cache0.v_scales, kv_dtype=cache0.cache_dtype, max_tokens=64)
 
+    @staticmethod
+    def _prompt_rows(cache0: StaticKVCache, n: int) -> int:
+        """Tokens of the n left that the next pass takes as one prompt step, or 0: a verify chunk takes the
+        rest, a whole number of chunks goes before what does not fit the cache's tail (where the ring wraps)."""
+        rows = min(n, PROMPT_ROWS, cache0.max_seq_len - cache0.total_seen_tokens[0])
+        if rows < n:
+            rows -= rows % VERIFY_CHUNK
+        return rows if rows > VERIFY_CHUNK else 0
+
     def _positions(self, cache0: StaticKVCache, T: int):
         seen = cache0.total_seen_tokens[0]
         S = cache0.max_seq_len
@@ -272,19 +286,30 @@ class Transformer:
             raise RuntimeError("forward expects idx of shape (1, T)")
         runner = self.get_decode_runner(cache0)
         T = idx.shape[1]
-        chunk = 32
         outs = []
-        for t0 in range(0, T, chunk):
-            part = idx[:, t0:t0 + chunk]
-            Tc = part.shape[1]
+        t0 = 0
+        while t0 < T:
+            rows = self._prompt_rows(cache0, T - t0)
+            Tc = rows or min(T - t0, VERIFY_CHUNK)
+            part = idx[:, t0:t0 + Tc]
             seen, write_pos, active, rope_pos = self._positions(cache0, Tc)
-            if Tc == 1:
+            if rows:
+                last = t0 + Tc == T
+                logits = runner.prompt_step(part, rope_pos, write_pos,
+                                            "all" if return_all_logits else ("last" if last else "none"),
+                                            (Tc - 1) % VERIFY_CHUNK + 1)
+            elif Tc == 1:
                 logits = runner.step(part.to(self.device), rope_pos, write_pos, active)
             else:
                 logits = runner.verify_step(part, rope_pos, write_pos, active)
-            outs.append(logits.clone() if (return_all_logits and T > chunk) else logits)
+            if logits is not None:
+                # verify_step's logits are a view that the next chunk overwrites
+                outs.append(logits.clone() if (return_all_logits and T > Tc and not rows) else logits)
+            t0 += Tc
             cache0.total_seen_tokens[:] = [seen + Tc] * cache0.n_layer
             cache0.layer_seq_lens[:] = [active] * cache0.n_layer
+        if not return_all_logits:
+            outs = outs[-1:]
         logits = torch.cat(outs, dim=1) if len(outs) > 1 else outs[0]
         return (logits if return_all_logits else logits[:, -1:, :]), None, kv_caches
 

@@ -316,6 +316,18 @@ int axm_runner_verify_step(axm_runner_t r, const void* idx_dev, int T, int start
 int axm_runner_verify_tree_step(axm_runner_t r, const void* idx_dev, int T, int start_pos, int write_pos,
                                 int prefix_len, const int* depths_host, const uint64_t* masks_host, void* stream,
                                 void** logits_out);
+/* T consecutive tokens (idx_dev: device int64 [T], any T >= 4) in one pass: rotated at
+ * start_pos + t, written to slot write_pos + t (write_pos + T <= max_seq_len) and attending
+ * causally to slots [0, write_pos + t], as verify_step's contiguous chain does.  The caller
+ * gives the activations' workspace (axm_runner_prompt_workspace_bytes, 256-byte aligned, used
+ * until the work on `stream` is done).  The last norm_rows (<= max_tokens) normalized rows are
+ * left for axm_runner_last_norm.  n_logits 1: the last token's logits into the runner's buffer;
+ * T: every token's into logits_all (fp16 [T][V]); 0: none.  Prompts of the reference's
+ * quantized forward (transformer.py:1036-1200). */
+size_t axm_runner_prompt_workspace_bytes(axm_runner_t r, int T);
+int axm_runner_prompt_step(axm_runner_t r, const void* idx_dev, int T, int start_pos, int write_pos, int norm_rows,
+                           int n_logits, void* logits_all, void* workspace, size_t workspace_bytes, void* stream,
+                           void** logits_out);
 /* Native prompt-lookup speculative decoding with greedy acceptance: n-gram
  * candidates from the token history are verified in one multi-token pass, the
  * matching prefix plus one corrected / bonus token is kept.  Host arrays;

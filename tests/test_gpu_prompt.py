@@ -1,0 +1,115 @@
+"""Prompts read in one pass (prompt_step) against the oracle's multi-token forward, and Transformer.forward's choice
+between prompt steps and verify chunks."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import model as om
+from test_gpu_runner import (TOL, _check_codes, _check_logits, _code_diffs, _gqa128_model, _prefill,
+                             _sync_frozen, build_runner, c1_model, run_steps)
+
+pytestmark = pytest.mark.gpu
+
+
+def _models(name):
+    return c1_model() if name == "c1" else _gqa128_model()
+
+
+# 4: the smallest; 33, 64: the 64-row GEMM; 65, 150: the many-row GEMM with a ragged last row tile and, with heads of
+# 128, its K splits summed by the RoPE launch; attention row blocks of 64 that end inside a token's heads (GQA 4).
+@pytest.mark.parametrize("name", ["c1", "gqa128"])
+@pytest.mark.parametrize("kv", ["fp16", "fp8", "int4"])
+@pytest.mark.parametrize("T,past", [(4, 0), (33, 7), (64, 0), (65, 40), (150, 0)])
+def test_prompt_step_matches_oracle(dev, name, kv, T, past):
+    print(f"[prompt_step] {name} kv={kv} T={T} past={past}", flush=True)
+    cfg, ow, cos, sin = _models(name)
+    model = om.OracleModel(cfg, ow, cos, sin)
+    S = 192
+    runner, cache = build_runner(cfg, ow, cos, sin, dev, S, kv)
+    ocache = om.OracleKVCache(S, cfg.n_layer, cfg.n_kv_head, cfg.head_dim, kv)
+    frozen = kv != "fp16"  # the oracle attends over the GPU's codes, as in the verify tests
+    ocache.frozen = frozen
+    rng = np.random.default_rng(T + past)
+    prefix = rng.integers(0, cfg.vocab, past).tolist()
+    if frozen:
+        run_steps(runner, cache, prefix, dev)
+    else:
+        _prefill(runner, cache, ocache, model, prefix, dev)
+    toks = rng.integers(0, cfg.vocab, T).tolist()
+    idx = torch.tensor([toks], device=dev)
+    got = runner.prompt_step(idx, past, past, "all", min(T, 32))[0].float().cpu().numpy()
+    if frozen:
+        _sync_frozen(ocache, cache, past, S)
+    ref = model.forward(toks, ocache, return_all_logits=True)
+    for t in range(T):
+        _check_logits(got[t], ref[t], f"prompt token {t} of {T}")
+    if frozen:
+        _check_codes(kv, _code_diffs(kv, ocache), f"prompt {name} T={T}")
+    norm = runner.get_last_norm(min(T, 32))
+    last = runner.prompt_step(idx, past, past, "last", 1)[0, 0].float().cpu().numpy()
+    _check_logits(last, ref[-1], "last token's logits alone")
+    assert np.abs(norm[0, -1].float().cpu().numpy() - runner.get_last_norm(1)[0, 0].float().cpu().numpy()).max() == 0
+    cache.total_seen_tokens[:] = [past + T] * cfg.n_layer
+    tok = int(rng.integers(0, cfg.vocab))
+    got = run_steps(runner, cache, [tok], dev)[0]
+    if frozen:
+        _sync_frozen(ocache, cache, past + T, S)
+    _check_logits(got, model.forward([tok], ocache)[-1], "step after the prompt")
+
+
+def test_prompt_step_rejects_rows_past_the_cache(dev):
+    cfg, ow, cos, sin = c1_model()
+    runner, _ = build_runner(cfg, ow, cos, sin, dev, 64)
+    idx = torch.zeros((1, 40), dtype=torch.int64, device=dev)
+    with pytest.raises(RuntimeError, match="rows at slot"):
+        runner.prompt_step(idx, 25, 25)
+    with pytest.raises(RuntimeError, match="below"):
+        runner.prompt_step(idx[:, :3], 0, 0)
+    with pytest.raises(RuntimeError, match="norm_rows"):
+        runner.prompt_step(idx, 0, 0, "last", 41)
+
+
+@pytest.mark.parametrize("ring,S,T", [(False, 128, 100), (True, 64, 150), (True, 128, 150), (False, 96, 70)])
+@pytest.mark.parametrize("every", [False, True])
+def test_forward_prompt_equals_verify_chunks(dev, ring, S, T, every):
+    """Transformer.forward against the same tokens as 32-token verify chunks: contiguous prompts, and ring caches
+    whose end falls inside the prompt (the chunks after it attend over all slots, as verify_step's do)."""
+    from axiomlm_amd.cache import StaticKVCache
+    from axiomlm_amd.transformer import ModelConfig, Transformer
+
+    cfg = ModelConfig(block_size=256, vocab_size=1024, n_layer=2, n_head=4, n_embd=256, rms_norm_eps=1e-5,
+                      tie_word_embeddings=False)
+    g = torch.Generator(device=dev)
+    g.manual_seed(2)
+    r = lambda *s: (torch.randn(*s, generator=g, device=dev) * 0.02).half()  # noqa: E731
+    sd = {"transformer.wte.weight": r(1024, 256), "lm_head.weight": r(1024, 256),
+          "transformer.ln_f.weight": 1 + r(256)}
+    for i in range(2):
+        pre = f"transformer.h.{i}."
+        sd.update({pre + "ln_1.weight": 1 + r(256), pre + "ln_2.weight": 1 + r(256), pre + "attn.c_attn.weight": r(768, 256),
+                   pre + "attn.c_proj.weight": r(256, 256), pre + "mlp.w_gate.weight": r(cfg.hidden, 256),
+                   pre + "mlp.w_up.weight": r(cfg.hidden, 256), pre + "mlp.w_down.weight": r(256, cfg.hidden)})
+    idx = torch.randint(0, 1024, (1, T), generator=g, device=dev)
+
+    def run(chunks):
+        model = Transformer(cfg, sd, device=dev).quantize("q4_rtn")
+        cache = StaticKVCache(1, S, 2, 4, 64, device=dev, ring_buffer=ring)
+        if not chunks:
+            out = model.forward(idx, kv_caches=cache, return_all_logits=every)[0].clone()
+        else:
+            out = torch.cat([model.forward(idx[:, t:t + 32], kv_caches=cache, return_all_logits=True)[0].clone()
+                             for t in range(0, T, 32)], dim=1)
+            out = out if every else out[:, -1:]
+        n = (T - 1) % 32 + 1
+        return out, cache, model.get_decode_runner(cache).get_last_norm(n)
+
+    a, ca, na = run(False)
+    b, cb, nb = run(True)
+    assert a.shape == b.shape == (1, T if every else 1, 1024)
+    assert ca.total_seen_tokens == cb.total_seen_tokens and ca.layer_seq_lens == cb.layer_seq_lens
+    # both within the oracle bar of the same values
+    assert (a.float() - b.float()).abs().max().item() <= 2 * TOL
+    assert (na.float() - nb.float()).abs().max().item() <= 2e-2
+    used = min(T, S)
+    assert (ca.cache[..., :used, :].float() - cb.cache[..., :used, :].float()).abs().max().item() <= 2e-2
