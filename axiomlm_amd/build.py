@@ -52,6 +52,7 @@ FILE_FLAGS = {
                       # The GEMV's leading scalar arguments land in SGPRs before the wave
                       # starts: its first requests do not wait for an argument load.
                       "-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "codes_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "rows_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "lowbit_gemv.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "q2k_gguf.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],

@@ -1,0 +1,16 @@
+// Several-row GEMM over row-major code matrices with 64-column groups (codes_gemm.hip).
+#pragma once
+#include "q4_tile16.h"
+
+enum { kCodesQ8 = 0, kCodesQ2 = 1, kCodesTernary = 2 };
+
+// a.w16 / a.sb16: the codes (uint8 [rows][K], or 2-bit [rows][K / 4]) and scales (fp16 (scale,
+// bias) [rows][K / 64][2], ternary [rows][K / 64]); a.x 16-byte aligned with ldx % 8 == 0; K % 64
+// == 0; a.N output rows (SwiGLU: gate rows [0, N), up rows [N, 2 N)).  Epilogues, residual norm
+// and split_info as t16_gemm_launch.  K is split as far as ws_bytes allows.
+bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int rows, int fmt);
+size_t codes_gemm_ws_bytes(int M, int K, int N, int epi);
+int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s);
+// Rows from which Q8 uses it: its GEMV takes four rows a launch (12288 x 4096: four rows 16.6 us
+// against 24; five 29.8 against 24.5, sixteen 67 against 25, 64 rows 244 against 40).
+constexpr int kCodesQ8MinRows = 5;

@@ -1,0 +1,474 @@
+// Several-row GEMM over row-major code matrices with a scale (and bias) per 64 columns --
+// Q8_G64, ternary and affine 2-bit -- on v_mfma_f32_16x16x32_f16, with exact code products:
+//
+//   y[m][n] = sum_g s_ng (sum_k q_nk x_mk) + b_ng (sum_k x_mk)       (g: 64 columns)
+//
+// The codes enter the MFMA as the integers themselves (fp16 holds them exactly), a group's two
+// MFMAs start from zero and its fp32 sum is scaled into the accumulator, so nothing is rounded
+// before fp32 (rounding each weight to fp16 first would add as much error as the fp16 result
+// has).  The bias term is one bf16 MFMA per four groups on the activations' group sums: a sum
+// is three bf16 parts (24 bits, cut exactly), a bias two (11 bits), and the six products fill
+// one lane's eight k slots; two multiply-adds per group and element on the vector units would
+// take as long as the code products.
+//
+// Workgroup: four waves, 16 MB rows of x, NT weight tiles of 16 rows per wave.  Lane (row r of a
+// tile, quarter q) holds columns 16 q .. + 15 of a group, so its codes of a group are 16 (Q8) or
+// 4 contiguous bytes; the MFMA's k order is that order of columns, also for the x fragments.
+// Activations go to LDS and weights to registers one 128-column stage ahead as in the
+// many-row tile16 GEMM (rows_gemm.hip).
+//
+// Measured (us, graph of back-to-back calls, against the GEMVs of up to 4 / 16 rows a launch):
+// Q8 12288 x 4096, 16 rows 67 -> 25, 64 rows 244 -> 40, 1000 rows -> 227 (443 TFLOP/s); ternary 64
+// rows 91 -> 35, 1000 rows 202 (498).  Large launches are bound by the vector units: per group
+// and 16 x 16 tile four multiply-adds (16 cycles) and a share of the code expansion stand beside
+// 32 MFMA cycles.
+#include <type_traits>
+
+#include "axm.h"
+#include "codes_gemm.h"
+#include "kernels.h"
+#include "t16_device.h"
+
+namespace {
+
+constexpr int kCThreads = 256;
+constexpr int kCWaves = kCThreads / 64;
+constexpr int kCStage = 128;
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// One lane's codes of one group (16 columns) and their two MFMA operands (8 columns each).
+template <int F>
+struct Codes;
+template <>
+struct Codes<kCodesQ8> {
+  static constexpr int kRowBytes64 = 64;  // code bytes of a row per group
+  u32x4 w;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+  }
+  // Bytes to halves 1024 + q by one permute per pair with the exponent byte 0x64, then the
+  // exact difference.
+  __device__ __forceinline__ f16x8 operand(int c) const {
+    const f16x2 off = {(f16)1024.f, (f16)1024.f};
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t d = w[2 * c + i];
+      o[2 * i] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, d, 0x04010400u)) - off);
+      o[2 * i + 1] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, d, 0x04030402u)) - off);
+    }
+    return __builtin_bit_cast(f16x8, o);
+  }
+};
+// Sixteen 2-bit fields, element i at bits 2 i.
+struct Codes2 {
+  static constexpr int kRowBytes64 = 16;
+  uint32_t w;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    w = __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
+  }
+  // Fields 8 c .. 8 c + 7 minus sub: the fields in the low half and, one field on, in the high
+  // half, so that a mask yields neighbours as a pair (1024 + q or 64 + q, as unpack_word).
+  __device__ __forceinline__ static f16x8 fields(uint32_t w, int c, float sub) {
+    const uint32_t h = c == 0 ? w : w >> 16;
+    const uint32_t v = (h & 0xFFFFu) | ((c == 0 ? w << 14 : w >> 2) & 0xFFFF0000u);
+    const uint32_t v8 = v >> 8;
+    const u32x4 u = {(v & 0x00030003u) | 0x64006400u, (v & 0x00300030u) | 0x54005400u,
+                     (v8 & 0x00030003u) | 0x64006400u, (v8 & 0x00300030u) | 0x54005400u};
+    const f16 lo = (f16)(1024.f + sub), hi = (f16)(64.f + sub);
+    const f16x8 m = {lo, lo, hi, hi, lo, lo, hi, hi};
+    return __builtin_bit_cast(f16x8, u) - m;
+  }
+};
+template <>
+struct Codes<kCodesQ2> : Codes2 {
+  __device__ __forceinline__ f16x8 operand(int c) const { return fields(w, c, 0.f); }
+};
+template <>
+struct Codes<kCodesTernary> : Codes2 {
+  // Codes 0, 1, 2, 3 stand for 0, 1, -1, 0: the fields become value + 1.
+  __device__ __forceinline__ f16x8 operand(int c) const {
+    const uint32_t lo = w & 0x55555555u, hi = (w >> 1) & 0x55555555u;
+    return fields(((lo & ~hi) << 1) | (~(lo ^ hi) & 0x55555555u), c, 1.f);
+  }
+};
+
+template <int F, int EPI, int MB, int NT>
+__global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
+  constexpr bool kPair = EPI == Q4_EPI_SWIGLU;
+  constexpr bool kBias = F != kCodesTernary;
+  constexpr int TOK = 16 * MB;
+  constexpr int UPW = kPair ? NT / 2 : NT;  // units per wave
+  __shared__ __align__(16) f16 xs[2][TOK * kCStage];
+  // Group sums of four groups (a pair of stages) as bf16 parts (s0, s1, s2, s0, s1, s2, 0, 0).
+  __shared__ __align__(16) u32x4 sx[kBias ? 2 : 1][kBias ? TOK * 4 : 1];
+
+  const int per = gridDim.x / 8;  // XCD-contiguous tiles, rows fastest (rows_gemm.hip)
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= n_tile) return;
+  const int m0 = (tile % n_mblk) * TOK;
+  const int sp = (tile / n_mblk) % n_split;
+  const int nblk = tile / (n_mblk * n_split);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int unit = (nblk * kCWaves + wave) * UPW;
+  const int kbA = sp * a.kb_per_split;
+  const int n_st = min(a.KB, kbA + a.kb_per_split) - kbA;  // stages of this split (>= 1)
+  const int KG = a.K / 64;
+  constexpr int RB = Codes<F>::kRowBytes64;
+  constexpr int SB = kBias ? 4 : 2;  // scale bytes of a row per group
+  const __amdgpu_buffer_rsrc_t rw =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.w16, (short)0, (int)a.w16_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.sb16, (short)0, (int)a.sb16_bytes, 0x00020000);
+
+  // This lane's codes and scales of tile 0, and the (wave-uniform) distance of tile t from it:
+  // an up tile starts a.N rows after its gate tile.  Rows past the matrix read zeros and are
+  // never stored.
+  const int wlane = l16 * KG * RB + kq * (RB / 4), slane = l16 * KG * SB;
+  int row0[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) row0[t] = (unit + t % UPW) * 16 + (kPair && t >= UPW ? a.N : 0);
+  // Codes and scales of one group per buffer: the next group's are requested before a group
+  // is consumed.  (A whole stage ahead took 64 more registers with Q8; eight waves of a CU with
+  // 4 KB each in flight already cover the memory's latency.)
+  Codes<F> wr[2][NT];
+  uint32_t sr[2][NT];
+  // The row's last stage has one group only if K % 128 == 64: its second one reads that group
+  // again, and zeros of x.
+  const int s_tail = a.K % kCStage != 0 && kbA + n_st == a.KB ? n_st - 1 : -1;
+  const int n_grp = 2 * n_st - (s_tail >= 0 ? 1 : 0);
+  auto load_w = [&](int gi, auto bc) {
+    constexpr int b = decltype(bc)::value;
+    const int g = 2 * kbA + min(gi, n_grp - 1);  // past the split: its last group again (never used)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int ch = row0[t] * KG + g;  // of the tile's first row
+      wr[b][t].load(rw, wlane, ch * RB);
+      if (kBias) sr[b][t] = __builtin_amdgcn_raw_buffer_load_b32(rs, slane, ch * SB, 0);
+      else sr[b][t] = __builtin_amdgcn_raw_buffer_load_b16(rs, slane, ch * SB, 0);
+    }
+  };
+
+  // Activations to LDS as in rows_gemm.hip: row r's 16-byte piece p at position p ^ (r % 16).
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
+  const int xrow = 4 * wave + kq;
+  const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  auto load_x = [&](int s, auto bc) {
+    constexpr int b = decltype(bc)::value;
+    const int so = (kbA + min(s, n_st - 1)) * (kCStage * 2);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
+                                               so + i * 32 * a.ldx, 0, 0);
+  };
+
+  f32x4 acc[NT][MB];
+  uint32_t bb[NT];  // fp16 bias of group slot kq of the pair of stages
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    bb[t] = 0;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  auto stage = [&](int s, auto bc, auto bn) {
+    constexpr int b = decltype(bc)::value;
+    if (s == s_tail) {
+      for (int i = tid; i < TOK * 8; i += kCThreads) {
+        const int r = i >> 3, c = 8 + (i & 7);
+        *reinterpret_cast<u32x4*>(&xs[b][r * kCStage + ((c ^ (r & 15)) * 8)]) = u32x4{0, 0, 0, 0};
+      }
+      __syncthreads();
+    }
+    load_x(s + 1, bn);
+    if (kBias) {
+      // Sums of the stage's two groups per row, TPP threads each.
+      constexpr int TPP = MB == 1 ? 8 : (MB == 2 ? 4 : 2);
+      const f16x2 one = {(f16)1.f, (f16)1.f};
+      // An opaque copy of the thread index: the addresses below are then formed here, in a few
+      // operations, and not kept in registers across the loop (25 of them spilled with Q8's
+      // 64-row tiles).
+      int tq = tid;
+      asm volatile("" : "+v"(tq));
+      for (int p = tq / TPP; p < 2 * TOK; p += kCThreads / TPP) {
+        const int r = p >> 1, g = p & 1;
+        float v = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8 / TPP; ++i) {
+          const int c = 8 * g + (tq % TPP) * (8 / TPP) + i;
+          const u32x4 x = *reinterpret_cast<const u32x4*>(&xs[b][r * kCStage + ((c ^ (r & 15)) * 8)]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_fdot2(as_h2(x[e]), one, v, false);
+        }
+        v += dpp_move<0xB1>(v);                    // lane ^ 1
+        if (TPP >= 4) v += dpp_move<0x4E>(v);      // lane ^ 2
+        if (TPP >= 8) v += dpp_move<0x141>(v);     // the other quad of eight
+        if (tq % TPP == 0) {
+          const uint32_t s0 = __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u;
+          const float r1 = v - __builtin_bit_cast(float, s0);
+          const uint32_t s1 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+          const uint32_t s2 = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, s1));
+          sx[(s >> 1) & 1][r * 4 + 2 * b + g] =
+              u32x4{(s0 >> 16) | s1, (s2 >> 16) | s0, (s1 >> 16) | (s2 & 0xFFFF0000u), 0u};
+        }
+      }
+    }
+    const f16* xa = &xs[b][l16 * kCStage];
+    auto group = [&](auto gc, auto gn) {
+      constexpr int g = decltype(gc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(2 * s + g + 1, gn);
+      if (kBias) {
+        // Slot 2 b + g of the pair of stages belongs to the lanes of quarter kq == 2 b + g; a pair's
+        // first group clears the others.
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const uint32_t bv = g == 1 && s == s_tail ? 0u : sr[g][t] >> 16;
+          bb[t] = kq == 2 * b + g ? bv : (b + g == 0 ? 0u : bb[t]);
+        }
+      }
+      f16x8 A[2][MB];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          A[c][mb] = *reinterpret_cast<const f16x8*>(xa + mb * 16 * kCStage + (((8 * g + 2 * kq + c) ^ l16) * 8));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        __builtin_amdgcn_sched_barrier(0);
+        const f16x8 q0 = wr[g][t].operand(0), q1 = wr[g][t].operand(1);
+        const float sc = h2f(u16_as_h((uint16_t)sr[g][t]));
+        f32x4 d[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[0][mb], q0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) d[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[1][mb], q1, d[mb], 0, 0, 0);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[t][mb][v] = __builtin_fmaf(sc, d[mb][v], acc[t][mb][v]);
+      }
+    };
+    group(B0{}, B1{});
+    group(B1{}, B0{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
+  // The bias term of the pair of stages that holds stage s (after its barrier).
+  auto flush = [&](int s) {
+    if constexpr (kBias) {
+      const u32x4* sp4 = sx[(s >> 1) & 1];
+      bf16x8 S[MB];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) S[mb] = __builtin_bit_cast(bf16x8, sp4[(16 * mb + l16) * 4 + kq]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const float bf = h2f(u16_as_h((uint16_t)bb[t]));
+        const uint32_t b0 = __builtin_bit_cast(uint32_t, bf) & 0xFFFF0000u;
+        const uint32_t b1 = __builtin_bit_cast(uint32_t, bf - __builtin_bit_cast(float, b0));
+        const u32x4 bw = {(b0 >> 16) | b0, (b0 >> 16) | (b1 & 0xFFFF0000u), (b1 >> 16) | (b1 & 0xFFFF0000u), 0u};
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[t][mb] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(S[mb], __builtin_bit_cast(bf16x8, bw), acc[t][mb], 0, 0, 0);
+      }
+    }
+  };
+
+  if (kBias)
+    for (int i = tid; i < TOK * 4; i += kCThreads) sx[0][i] = sx[kBias ? 1 : 0][i] = u32x4{0, 0, 0, 0};
+  load_x(0, B0{});
+  load_w(0, B0{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int s = 0;;) {
+    stage(s, B0{}, B1{});
+    if (++s >= n_st) break;
+    stage(s, B1{}, B0{});
+    flush(s);
+    if (++s >= n_st) break;
+  }
+  if (n_st & 1) flush(n_st - 1);
+
+  // Lane: weight row l16 of each tile, tokens 4 kq .. + 3 of each 16.
+#pragma unroll
+  for (int t = 0; t < (n_split == 1 ? UPW : NT); ++t) {
+    const int u = unit + t % UPW, row = u * 16 + l16;
+    if (u >= a.n_units || (n_split == 1 && row >= a.N)) continue;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int tok = m0 + 16 * mb + 4 * kq + v;
+        if (tok >= a.M_tokens) continue;
+        if (n_split == 1)
+          t16g_store<EPI>(a, tok, row, acc[t][mb][v], acc[kPair ? t + UPW : t][mb][v]);
+        else
+          a.part_ws[((size_t)sp * a.M_tokens + tok) * a.part_cols + row + (kPair && t >= UPW ? a.n_units * 16 : 0)] =
+              acc[t][mb][v];
+      }
+  }
+}
+
+struct CodesPlan {
+  int mb, nt, splits;
+};
+// Row tile: the fewest row blocks of up to 64 rows, evenly filled.  Up to 32 rows the launch is
+// bound by the weights' stream: two tiles per wave, K split until three workgroups per CU are in
+// flight (12288 x 4096 Q8, 16 rows: one split 51 us, four 26, eight 24); more rows take four
+// tiles per wave (each x fragment read from LDS feeds four) and two workgroups per CU (64 rows: one split
+// 94 us, four 38).  Each split keeps two stages.
+CodesPlan codes_plan(int M, int KB, int n_units, int epi) {
+  CodesPlan p;
+  const int nb = axm_ceil_div(M, 64);
+  p.mb = axm_ceil_div(M, 16 * nb);
+  p.nt = p.mb <= 2 ? 2 : 4;
+  const int upw = epi == Q4_EPI_SWIGLU ? p.nt / 2 : p.nt;
+  const int tiles = axm_ceil_div(n_units, kCWaves * upw) * axm_ceil_div(M, 16 * p.mb);
+  int s = (p.mb <= 2 ? 3 : 2) * axm_num_cus() / tiles;
+  s = s > KB / 2 ? KB / 2 : s;
+  p.splits = s < 1 ? 1 : (s > 16 ? 16 : s);
+  return p;
+}
+
+template <int F, int EPI, int MB, int NT>
+void codes_launch(const T16Args& a, int M, int splits, hipStream_t s) {
+  constexpr int kUnits = kCWaves * (EPI == Q4_EPI_SWIGLU ? NT / 2 : NT);
+  const int n_mblk = axm_ceil_div(M, 16 * MB);
+  const int n_tile = n_mblk * splits * axm_ceil_div(a.n_units, kUnits);
+  hipLaunchKernelGGL((codes_gemm_kernel<F, EPI, MB, NT>), dim3(8 * axm_ceil_div(n_tile, 8)), dim3(kCThreads), 0, s, a,
+                     n_mblk, splits, n_tile);
+}
+template <int F, int EPI>
+void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t s) {
+  switch (p.mb) {
+    case 1: return codes_launch<F, EPI, 1, 2>(a, M, p.splits, s);
+    case 2: return codes_launch<F, EPI, 2, 2>(a, M, p.splits, s);
+    case 3: return codes_launch<F, EPI, 3, 4>(a, M, p.splits, s);
+    default: return codes_launch<F, EPI, 4, 4>(a, M, p.splits, s);
+  }
+}
+
+}  // namespace
+
+bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int rows, int fmt) {
+  const size_t code_bytes = (size_t)rows * K / (fmt == kCodesQ8 ? 1 : 4);
+  const uintptr_t wa = fmt == kCodesQ8 ? 15 : 3, sa = fmt == kCodesTernary ? 1 : 3;
+  return K > 0 && K % 64 == 0 && K <= 32768 && code_bytes < (size_t)0x7FFFFFF0 && ((uintptr_t)x & 15) == 0 &&
+         ((uintptr_t)w & wa) == 0 && ((uintptr_t)sb & sa) == 0;
+}
+
+size_t codes_gemm_ws_bytes(int M, int K, int N, int epi) {
+  const int n_units = (N + 15) / 16;
+  const int splits = codes_plan(M, (K + 127) / 128, n_units, epi).splits;
+  return splits <= 1 ? 0 : (size_t)splits * M * n_units * (epi == Q4_EPI_SWIGLU ? 32 : 16) * sizeof(float);
+}
+
+int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s) {
+  const int rows = epi == Q4_EPI_SWIGLU ? 2 * a.N : a.N;
+  if (M < 1 || !codes_gemm_takes(a.x, a.w16, a.sb16, a.K, rows, fmt) || a.ldx % 8 != 0 || a.ln_w != nullptr ||
+      (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) || (fmt != kCodesQ8 && epi != Q4_EPI_STORE) ||
+      (a.post_ln_w != nullptr && (epi != Q4_EPI_RESID || a.post_norm_out == nullptr || a.ldr != a.N))) {
+    axm_set_error("codes gemm: format %d, M=%d, epi=%d, K=%d unsupported", fmt, M, epi, a.K);
+    return -2;
+  }
+  a.KB = (a.K + 127) / 128;
+  a.n_units = (a.N + 15) / 16;
+  a.M_tokens = M;
+  a.part_ws = ws;
+  a.part_cols = a.n_units * (epi == Q4_EPI_SWIGLU ? 32 : 16);
+  a.pair_offset = a.n_units;  // of the partial tiles' columns
+  CodesPlan p = codes_plan(M, a.KB, a.n_units, epi);
+  const size_t one = (size_t)M * a.part_cols * sizeof(float);
+  if (ws == nullptr || ws_bytes < 2 * one) p.splits = 1;
+  else if (ws_bytes < p.splits * one) p.splits = (int)(ws_bytes / one);
+  a.kb_per_split = axm_ceil_div(a.KB, p.splits);
+  p.splits = axm_ceil_div(a.KB, a.kb_per_split);
+  a.w16_bytes = (size_t)rows * a.K / (fmt == kCodesQ8 ? 1 : 4);
+  a.sb16_bytes = (size_t)rows * (a.K / 64) * (fmt == kCodesTernary ? 2 : 4);
+  if (fmt == kCodesQ2) codes_launch_shape<kCodesQ2, Q4_EPI_STORE>(a, M, p, s);
+  else if (fmt == kCodesTernary) codes_launch_shape<kCodesTernary, Q4_EPI_STORE>(a, M, p, s);
+  else if (epi == Q4_EPI_STORE) codes_launch_shape<kCodesQ8, Q4_EPI_STORE>(a, M, p, s);
+  else if (epi == Q4_EPI_RESID) codes_launch_shape<kCodesQ8, Q4_EPI_RESID>(a, M, p, s);
+  else codes_launch_shape<kCodesQ8, Q4_EPI_SWIGLU>(a, M, p, s);
+  return t16_gemm_finish(a, M, epi, p.splits, M, s);
+}
+
+// ---------------------------------------------------------------------------
+// C ABI: products of several rows with a workspace for split K.
+// ---------------------------------------------------------------------------
+// The 2-bit GEMVs' own matrix-core launches take up to 16 rows each (fewer at large K, whose rows
+// fill LDS); this kernel takes over where they need four, or two of a large matrix (ternary,
+// 12288 x 4096: 16 rows in one launch 23.3 us against 22.3 here, 17 in two 28.7 / 23.2, 64 in four
+// 90.7 / 35.4; 4096 x 4096: 32 in two 13.6 / 16.4, 48 in three 20.2 / 20.9, 64 in four 26.4 / 24.1;
+// 4096 x 11008: six in one 11.5 / 17.4, eight in two 20.2 / 17.4).
+static bool lowbit_rows_use_codes(int M, int K, int N) {
+  const int per = lowbit_mfma_rows(N, K);
+  const int launches = per > 0 ? axm_ceil_div(M, per) : M;
+  return launches >= 4 || (launches >= 2 && (size_t)N * K >= (size_t)32 << 20);
+}
+
+// Whether M rows of a format go through this kernel (shapes and alignment apart).
+static bool rows_use_codes(int fmt, int M, int K, int N) {
+  return fmt == kCodesQ8 ? M >= kCodesQ8MinRows : M > 4 && lowbit_rows_use_codes(M, K, N);
+}
+
+extern "C" size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N) {
+  if (format < kCodesQ8 || format > kCodesTernary || M <= 0 || K <= 0 || N <= 0) return 0;
+  return rows_use_codes(format, M, K, N) ? codes_gemm_ws_bytes(M, K, N, Q4_EPI_STORE) : 0;
+}
+
+static int qmm_codes(int fmt, const char* who, const void* x, const void* w, const void* sb, const void* bias, void* y,
+                     int M, int K, int N, void* ws, size_t ws_bytes, hipStream_t s) {
+  T16Args a{};
+  a.x = (const f16*)x;
+  a.ldx = K;
+  a.w16 = (const u32x4*)w;
+  a.sb16 = (const u32x2*)sb;
+  a.K = K;
+  a.N = N;
+  a.y = (f16*)y;
+  a.ldy = N;
+  a.bias = (const f16*)bias;
+  const int rc = codes_gemm_launch(fmt, a, M, Q4_EPI_STORE, (float*)ws, ws_bytes, s);
+  if (rc) return rc;
+  AXM_LAUNCH_CHECK(who);
+  return 0;
+}
+
+extern "C" int axm_qmm_q8_g64(const void* x, const void* w_packed, const void* sb, const void* bias, void* y, int M,
+                              int K, int N, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!rows_use_codes(kCodesQ8, M, K, N) || !codes_gemm_takes(x, w_packed, sb, K, N, kCodesQ8))
+    return axm_qmv_q8_g64(x, w_packed, sb, bias, y, M, K, N, stream);
+  AXM_CHECK_ARG(w_packed && sb && x && y && N > 0, -1, "qmm_q8_g64: bad arguments");
+  return qmm_codes(kCodesQ8, "qmm_q8_g64", x, w_packed, sb, bias, y, M, K, N, workspace, workspace_bytes,
+                   (hipStream_t)stream);
+}
+
+extern "C" int axm_qmm_ternary(const void* x, const void* w_packed, const void* scales, const void* bias, void* y,
+                               int M, int K, int N, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!rows_use_codes(kCodesTernary, M, K, N) || !codes_gemm_takes(x, w_packed, scales, K, N, kCodesTernary))
+    return axm_qmv_ternary(x, w_packed, scales, bias, y, M, K, N, stream);
+  AXM_CHECK_ARG(x && w_packed && scales && y && N > 0, -1, "qmm_ternary: bad arguments");
+  return qmm_codes(kCodesTernary, "qmm_ternary", x, w_packed, scales, bias, y, M, K, N, workspace, workspace_bytes,
+                   (hipStream_t)stream);
+}
+
+extern "C" int axm_qmm_q2_k(const void* x, const void* w_packed, const void* scales_biases, const void* bias, void* y,
+                            int M, int K, int N, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!rows_use_codes(kCodesQ2, M, K, N) || !codes_gemm_takes(x, w_packed, scales_biases, K, N, kCodesQ2))
+    return axm_qmv_q2_k(x, w_packed, scales_biases, bias, y, M, K, N, stream);
+  AXM_CHECK_ARG(x && w_packed && scales_biases && y && N > 0, -1, "qmm_q2_k: bad arguments");
+  return qmm_codes(kCodesQ2, "qmm_q2_k", x, w_packed, scales_biases, bias, y, M, K, N, workspace, workspace_bytes,
+                   (hipStream_t)stream);
+}

@@ -127,3 +127,6 @@ int tree_choose_splits(int T, int Hq, int Hkv, int n_keys);
 // values are in the cache at slots prefix_len + t already.  Splits and workspace as the tree's.
 int launch_prompt_attention(const f16* q, const KvView& kv, f16* out, int Hq, int T, int prefix_len, int n_splits,
                             float* ws, hipStream_t s);
+// Rows of one matrix-core launch of the 2-bit GEMVs at this K (lowbit_gemv.hip), 0 where they
+// have none.
+int lowbit_mfma_rows(int N, int K);

@@ -483,7 +483,7 @@ int lowbit_gemv(const void* x, const void* w, const void* s, const void* bias, v
   // 9.4 us, three 10.0 / 9.5, four 11.2 / 9.6; at 11008 -> 4096 four tokens 17.5 /
   // 10.3 us).
   constexpr int kMinTokens = 3;
-  const int mt = (size_t)N * K / 4 < (size_t)kLbOOB && K <= kLbMfmaMaxK ? lb_mfma_max_tokens(K) : 0;
+  const int mt = lowbit_mfma_rows(N, K);
   int m0 = 0;
   while (mt >= kMinTokens && M - m0 >= kMinTokens) {
     const int mc = (M - m0) < mt ? (M - m0) : mt;
@@ -509,6 +509,10 @@ int lowbit_gemv(const void* x, const void* w, const void* s, const void* bias, v
 }
 
 }  // namespace
+
+int lowbit_mfma_rows(int N, int K) {
+  return (size_t)N * K / 4 < (size_t)kLbOOB && K <= kLbMfmaMaxK ? lb_mfma_max_tokens(K) : 0;
+}
 
 extern "C" int axm_qmv_ternary(const void* x, const void* w_packed, const void* scales, const void* bias, void* y,
                                int M, int K, int N, void* stream) {

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "axm.h"
+#include "codes_gemm.h"
 #include "kernels.h"
 #include "step_kernel.h"
 #include "q4_tile16.h"
@@ -633,11 +634,35 @@ struct axm_runner {
     return lm_head_dense(x, 1, (const f16*)d.lnf_w, norm, s);
   }
 
+  // Buffers of a multi-token step: the runner's own (verify), or a caller's workspace (prompt).
+  struct RowBufs {
+    f16 *x, *norm, *q, *attn_y, *hbuf, *qkvbuf, *kvst;
+    int* pos;
+    float* ws;
+    size_t ws_bytes;
+  };
+  RowBufs own_bufs() const { return {x, norm, q, attn_y, hbuf, qkvbuf, kvst, tree_pos, ws, ws_bytes}; }
+
   // Q8_G64 (format 1) or fp16 (format 2) lm_head over T rows into logits: with ln_w the
   // GEMV applies the final RMSNorm itself and writes the normalized rows to xn_out (one
   // launch where a separate norm took two); without, the rows are normalized already.
-  int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s, f16* out = nullptr) {
+  int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s, f16* out = nullptr,
+                    const RowBufs* b = nullptr) {
     if (out == nullptr) out = logits;
+    if (b != nullptr && ln_w == nullptr && d.lm_head_format == 1 && T >= kCodesQ8MinRows) {
+      Mat m;
+      m.w = d.lm_head_w;
+      m.sb = d.lm_head_sb;
+      m.N = d.vocab_size;
+      m.K = d.d_model;
+      m.fmt = 1;
+      GemvCall c{};
+      c.x = x;
+      c.ldx = d.d_model;
+      c.y = out;
+      c.ldy = d.vocab_size;
+      return gemv_rows(*b, m, Q4_EPI_STORE, d.vocab_size, c, T, s);
+    }
     if (d.lm_head_format == 2)
       return launch_f16_gemv(x, (const f16*)d.lm_head_w, nullptr, out, T, d.d_model, d.vocab_size, ln_w, d.eps,
                              s, xn_out);
@@ -703,15 +728,6 @@ struct axm_runner {
     return m.fmt != 0 ? run_dense(m, epi, out_rows, c, M, s) : run_gemv(m, epi, out_rows, c, M, s);
   }
 
-  // Buffers of a multi-token step: the runner's own (verify), or a caller's workspace (prompt).
-  struct RowBufs {
-    f16 *x, *norm, *q, *attn_y, *hbuf, *qkvbuf, *kvst;
-    int* pos;
-    float* ws;
-    size_t ws_bytes;
-  };
-  RowBufs own_bufs() const { return {x, norm, q, attn_y, hbuf, qkvbuf, kvst, tree_pos, ws, ws_bytes}; }
-
   // GEMV over T token rows in launches of at most 4 rows, or the multi-token GEMM
   // from kGemmMinTokens rows on.
   int gemv_rows(const RowBufs& b, const Mat& m, int epi, int out_rows, GemvCall c, int T, hipStream_t s) {
@@ -756,6 +772,33 @@ struct axm_runner {
         if (rc) return rc;
       }
       return 0;
+    }
+    if (m.fmt == 1 && T >= kCodesQ8MinRows && c.argmax_keys == nullptr && c.q_dim == 0 &&
+        (epi == Q4_EPI_STORE || epi == Q4_EPI_RESID || epi == Q4_EPI_SWIGLU) &&
+        codes_gemm_takes(c.x, m.w, m.sb, m.K, m.N, kCodesQ8)) {
+      // Q8_G64: all rows in one launch over the codes as stored.
+      T16Args a{};
+      a.x = c.x;
+      if (c.ln_w != nullptr) {
+        f16* nrm = c.x_norm_out ? c.x_norm_out : b.norm;
+        launch_rmsnorm(c.x, c.ln_w, nrm, T, m.K, c.eps, s);
+        a.x = nrm;
+      }
+      a.ldx = c.ldx;
+      a.w16 = (const u32x4*)m.w;
+      a.sb16 = (const u32x2*)m.sb;
+      a.K = m.K;
+      a.N = out_rows;
+      a.y = c.y;
+      a.ldy = c.ldy;
+      a.bias = c.bias;
+      a.resid = c.resid;
+      a.ldr = c.ldr;
+      a.post_ln_w = c.post_ln_w;
+      a.post_norm_out = c.post_norm_out;
+      a.eps = c.eps;
+      a.split_info = c.split_info;
+      return codes_gemm_launch(kCodesQ8, a, T, epi, b.ws, b.ws_bytes, s);
     }
     for (int t0 = 0; t0 < T; t0 += 4) {
       const int mc = (T - t0) < 4 ? (T - t0) : 4;
@@ -897,7 +940,7 @@ struct axm_runner {
       return gemv_rows(b, m_lmh, Q4_EPI_STORE, d.vocab_size, l, T, s);
     }
     if (!post) return lm_head_dense(x, T, (const f16*)d.lnf_w, norm, s);
-    return lm_head_dense(norm, T, nullptr, nullptr, s);
+    return lm_head_dense(norm, T, nullptr, nullptr, s, nullptr, &b);
   }
 
   // Workspace of a prompt step of T rows: RowBufs laid out from `base` (null: sizes only).
@@ -923,8 +966,9 @@ struct axm_runner {
     size_t w = tree_workspace_bytes(T, d.n_head, d.head_dim,
                                     tree_choose_splits(T, d.n_head, d.n_kv_head, d.max_seq_len));
     auto gemm = [&](const Mat& m, int rows, int epi) {
-      if (m.w16 == nullptr) return;
-      const size_t g = T > kTile16GemmMaxTokens ? t16_rows_gemm_ws_bytes(T, m.K, (rows + 15) / 16, epi)
+      if (m.w16 == nullptr && m.fmt != 1) return;
+      const size_t g = m.fmt == 1 ? codes_gemm_ws_bytes(T, m.K, rows, epi)
+                       : T > kTile16GemmMaxTokens ? t16_rows_gemm_ws_bytes(T, m.K, (rows + 15) / 16, epi)
                                                 : t16_gemm_ws_bytes(m.K, (rows + 15) / 16, epi == Q4_EPI_SWIGLU ? 2 : 1);
       w = g > w ? g : w;
     };
@@ -932,7 +976,14 @@ struct axm_runner {
     gemm(m_o[0], d.d_model, Q4_EPI_RESID);
     gemm(m_gu[0], d.hidden_dim, Q4_EPI_SWIGLU);
     gemm(m_dn[0], d.d_model, Q4_EPI_RESID);
-    gemm(m_lmh, d.vocab_size, Q4_EPI_STORE);
+    if (d.lm_head_format == 1) {
+      Mat head;
+      head.K = d.d_model;
+      head.fmt = 1;
+      gemm(head, d.vocab_size, Q4_EPI_STORE);
+    } else {
+      gemm(m_lmh, d.vocab_size, Q4_EPI_STORE);
+    }
     r.ws = (float*)take(w);
     r.ws_bytes = w;
     if (b != nullptr) *b = r;
@@ -959,7 +1010,7 @@ struct axm_runner {
     if (n_logits == 0) return 0;
     const f16* rows = n_logits == 1 ? b.norm + (size_t)(T - 1) * D : b.norm;
     f16* out = n_logits == 1 ? logits : logits_all;
-    if (d.lm_head_format != 0) return lm_head_dense(rows, n_logits, nullptr, nullptr, s, out);
+    if (d.lm_head_format != 0) return lm_head_dense(rows, n_logits, nullptr, nullptr, s, out, &b);
     GemvCall l{};
     l.x = rows;
     l.ldx = D;
@@ -1089,6 +1140,15 @@ extern "C" int axm_runner_create(const axm_runner_desc* desc, axm_runner_t* out)
                         t16_gemm_ws_bytes(d.d_model, d.hidden_dim / 16, 2),
                         t16_gemm_ws_bytes(d.hidden_dim, (d.d_model + 15) / 16, 1),
                         t16_gemm_ws_bytes(d.d_model, (d.vocab_size + 15) / 16, 1)};
+    for (size_t b : g) r->ws_bytes = b > r->ws_bytes ? b : r->ws_bytes;
+  }
+  for (int t = kCodesQ8MinRows; t <= T; ++t) {
+    // Partial tiles of the Q8_G64 several-row GEMM.
+    const size_t g[] = {d.qkv_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, r->qkv_dim, Q4_EPI_STORE) : 0,
+                        d.o_format == 1 ? codes_gemm_ws_bytes(t, r->q_dim, d.d_model, Q4_EPI_RESID) : 0,
+                        d.gu_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, d.hidden_dim, Q4_EPI_SWIGLU) : 0,
+                        d.down_format == 1 ? codes_gemm_ws_bytes(t, d.hidden_dim, d.d_model, Q4_EPI_RESID) : 0,
+                        d.lm_head_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, d.vocab_size, Q4_EPI_STORE) : 0};
     for (size_t b : g) r->ws_bytes = b > r->ws_bytes ? b : r->ws_bytes;
   }
   struct {

@@ -316,6 +316,12 @@ def dequant_q8_rows(indices, w_packed, scales_biases) -> torch.Tensor:
     return out.view(*indices.shape, K)
 
 
+def _codes_workspace(fmt: int, M: int, K: int, N: int, device):
+    """Workspace of the several-row products (0 Q8_G64, 1 affine 2-bit, 2 ternary)."""
+    n = _lib.lib().axm_qmm_codes_workspace_bytes(fmt, M, K, N)
+    return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
+
+
 def qmv_q8_g64(x, w_packed, scales_biases, bias=None) -> torch.Tensor:
     """y = x @ W^T (+ bias, this build's addition) with Q8_G64 weights (quant.py:201-218)."""
     _lib.require_gpu(x, "qmv_q8_g64")
@@ -324,9 +330,16 @@ def qmv_q8_g64(x, w_packed, scales_biases, bias=None) -> torch.Tensor:
     N = w_packed.shape[0]
     y = torch.empty((*x.shape[:-1], N), dtype=torch.float16, device=x.device)
     b = None if bias is None else bias.to(device=x.device, dtype=torch.float16).contiguous()
-    _lib.check(_lib.lib().axm_qmv_q8_g64(_lib.ptr(x.contiguous()), _lib.ptr(w_packed.contiguous()),
+    if M <= 4:  # the GEMV
+        _lib.check(_lib.lib().axm_qmv_q8_g64(_lib.ptr(x.contiguous()), _lib.ptr(w_packed.contiguous()),
+                                             _lib.ptr(scales_biases.contiguous()), _lib.ptr(b), _lib.ptr(y), M, K, N,
+                                             _lib.stream_of(x.device)),
+                   "qmv_q8_g64")
+        return y
+    ws, n = _codes_workspace(0, M, K, N, x.device)
+    _lib.check(_lib.lib().axm_qmm_q8_g64(_lib.ptr(x.contiguous()), _lib.ptr(w_packed.contiguous()),
                                          _lib.ptr(scales_biases.contiguous()), _lib.ptr(b), _lib.ptr(y), M, K, N,
-                                         _lib.stream_of(x.device)),
+                                         _lib.ptr(ws), n, _lib.stream_of(x.device)),
                "qmv_q8_g64")
     return y
 
@@ -383,7 +396,7 @@ def dequantize_q2_k(w_packed, scales_biases, K: int | None = None) -> torch.Tens
     return (q * scales_biases[..., 0:1] + scales_biases[..., 1:2]).view(N, K).to(torch.float16)
 
 
-def _lowbit_qmv(fn, name, x, w_packed, s, bias):
+def _lowbit_qmv(fmt, gemv, fn, name, x, w_packed, s, bias):
     _lib.require_gpu(x, name)
     if x.dtype != torch.float16:
         raise RuntimeError(f"{name}: x must be float16")
@@ -394,14 +407,20 @@ def _lowbit_qmv(fn, name, x, w_packed, s, bias):
         raise RuntimeError(f"{name}: K={K} does not match packed K={int(w_packed.shape[1]) * 4}")
     y = torch.empty((*x.shape[:-1], N), dtype=torch.float16, device=x.device)
     b = None if bias is None else bias.to(device=x.device, dtype=torch.float16).contiguous()
+    if M <= 4:  # the GEMVs
+        _lib.check(gemv(_lib.ptr(x.contiguous()), _lib.ptr(w_packed.contiguous()), _lib.ptr(s.contiguous()), _lib.ptr(b),
+                        _lib.ptr(y), M, K, N, _lib.stream_of(x.device)), name)
+        return y
+    ws, n = _codes_workspace(fmt, M, K, N, x.device)
     _lib.check(fn(_lib.ptr(x.contiguous()), _lib.ptr(w_packed.contiguous()), _lib.ptr(s.contiguous()), _lib.ptr(b),
-                  _lib.ptr(y), M, K, N, _lib.stream_of(x.device)), name)
+                  _lib.ptr(y), M, K, N, _lib.ptr(ws), n, _lib.stream_of(x.device)), name)
     return y
 
 
 def qmv_ternary(x, w_packed, scales, bias=None) -> torch.Tensor:
     """y = x @ W^T (+ bias) on BitNet 1.58 ternary rows (quant.py:298-318); M > 1 rows batched."""
-    return _lowbit_qmv(_lib.lib().axm_qmv_ternary, "qmv_ternary", x, w_packed, scales, bias)
+    L = _lib.lib()
+    return _lowbit_qmv(2, L.axm_qmv_ternary, L.axm_qmm_ternary, "qmv_ternary", x, w_packed, scales, bias)
 
 
 def qmm_ternary(x, w_packed, scales, bias=None) -> torch.Tensor:
@@ -411,7 +430,8 @@ def qmm_ternary(x, w_packed, scales, bias=None) -> torch.Tensor:
 
 def qmv_q2_k(x, w_packed, scales_biases, bias=None) -> torch.Tensor:
     """y = x @ W^T (+ bias) on reference affine 2-bit rows (quant.py:406-426)."""
-    return _lowbit_qmv(_lib.lib().axm_qmv_q2_k, "qmv_q2_k", x, w_packed, scales_biases, bias)
+    L = _lib.lib()
+    return _lowbit_qmv(1, L.axm_qmv_q2_k, L.axm_qmm_q2_k, "qmv_q2_k", x, w_packed, scales_biases, bias)
 
 
 def qmm_q2_k(x, w_packed, scales_biases, bias=None) -> torch.Tensor:

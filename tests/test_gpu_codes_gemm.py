@@ -1,0 +1,119 @@
+"""Several-row GEMM over Q8_G64, ternary and affine 2-bit codes against the float64 product of the decoded codes.
+
+Code products are exact and sums fp32, so the result is the float64 one to the fp16 rounding of the output: 2^-11 of
+each value at most, plus fp32 sums whose error (2^-24 of the sum of magnitudes per add) matters only where a row's
+terms cancel; 1.05 x 2^-11 in the 2-norm covers both."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import formats as fm
+
+pytestmark = pytest.mark.gpu
+REL = 1.05 * 2.0 ** -11
+
+
+def _packed(fmt, rng, N, K):
+    """(device arrays, float64 weights)"""
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float16)
+    if fmt == "q8":
+        p, s = fm.pack_linear_q8_g64(w)
+        q = p.reshape(N, K // 64, 64).astype(np.float64)
+        return (p.view(np.int32).reshape(N, K // 4), s), (q * s[..., 0:1] + s[..., 1:2].astype(np.float64)).reshape(N, K)
+    if fmt == "ternary":
+        p, s = fm.pack_linear_ternary(w)
+        q = fm.ternary_decode_bytes(p).reshape(N, K // 64, 64).astype(np.float64)
+        return (p, s), (q * s[..., None]).reshape(N, K)
+    p, s = fm.pack_linear_q2_k(w)
+    q = ((p[..., None] >> (2 * np.arange(4))) & 3).reshape(N, K // 64, 64).astype(np.float64)
+    return (p, s), (q * s[..., 0:1] + s[..., 1:2].astype(np.float64)).reshape(N, K)
+
+
+def _run(fmt, x, packs, N, bias=None, ws=True):
+    """The several-row entry itself (the Python wrappers choose by size)."""
+    from axiomlm_amd import _lib
+
+    L = _lib.lib()
+    M, K = x.shape
+    fn = {"q8": L.axm_qmm_q8_g64, "ternary": L.axm_qmm_ternary, "q2": L.axm_qmm_q2_k}[fmt]
+    y = torch.empty((M, N), dtype=torch.float16, device=x.device)
+    n = L.axm_qmm_codes_workspace_bytes({"q8": 0, "q2": 1, "ternary": 2}[fmt], M, K, N) if ws else 0
+    buf = torch.empty(max(n, 1), dtype=torch.uint8, device=x.device)
+    _lib.check(fn(_lib.ptr(x), _lib.ptr(packs[0]), _lib.ptr(packs[1]), _lib.ptr(bias), _lib.ptr(y), M, K, N,
+                  _lib.ptr(buf) if n else None, n, _lib.stream_of(x.device)), fmt)
+    return y
+
+
+# Row tiles of 16 - 64 with remainders, several row blocks, weight tiles past N, one and two stages, odd and even
+# counts, half a stage, split and unsplit K; 2-bit sizes beyond what their GEMV launches take.
+SHAPES = [(5, 16, 64), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96, 8192), (70, 130, 320),
+          (129, 2056, 1024), (17, 40, 192)]
+
+
+@pytest.mark.parametrize("fmt", ["q8", "ternary", "q2"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("ws", [True, False])
+def test_codes_gemm_matches_float64(dev, fmt, M, N, K, ws):
+    if fmt != "q8":
+        M += 64  # four launches of 16 rows and more
+    rng = np.random.default_rng(M + N + K)
+    packs, w = _packed(fmt, rng, N, K)
+    packs = [torch.from_numpy(a).to(dev) for a in packs]
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    x[:, : K // 2] += 1  # group sums far from zero: the bias term counts
+    bad = M // 3
+    x[bad, :64] = np.inf  # this row only: row bad - 1's last half stage is followed by it in memory
+    buf = torch.full((M * K + 256,), float("inf"), dtype=torch.float16, device=dev)
+    buf[: M * K] = torch.from_numpy(x.reshape(-1)).to(dev)
+    bias = rng.standard_normal(N).astype(np.float16)
+    keep = np.arange(M) != bad
+    ref = x[keep].astype(np.float64) @ w.T
+    got = _run(fmt, buf[: M * K].view(M, K), packs, N, None, ws).cpu().numpy()[keep].astype(np.float64)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got - ref) <= REL * np.linalg.norm(ref)
+    got = _run(fmt, buf[: M * K].view(M, K), packs, N, torch.from_numpy(bias).to(dev), ws).cpu().numpy()[keep]
+    # a second fp16 rounding
+    assert np.linalg.norm(got.astype(np.float64) - (ref + bias)) <= 2 * REL * np.linalg.norm(ref + bias)
+
+
+@pytest.mark.parametrize("fmt", ["q8", "q2"])
+def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
+    """Group sums beyond the fp16 range and activations near its bottom keep 24 bits in the bias term."""
+    rng = np.random.default_rng(1)
+    N, K, M = 32, 512, 80
+    packs, w = _packed(fmt, rng, N, K)
+    packs = [torch.from_numpy(a).to(dev) for a in packs]
+    for scale in (3000.0, 2.0 ** -18):
+        x = (np.abs(rng.standard_normal((M, K))) * scale).astype(np.float16)
+        wn = w
+        if scale > 1:  # keep the results in range: smaller scales and biases, same codes
+            packs[1] = (packs[1].double() * 2.0 ** -6).half()
+            s = packs[1].cpu().numpy().astype(np.float64)
+            p = packs[0].cpu().numpy()
+            codes = (p.view(np.uint8).reshape(N, K // 64, 64) if fmt == "q8" else
+                     ((p[..., None] >> (2 * np.arange(4))) & 3).reshape(N, K // 64, 64)).astype(np.float64)
+            wn = (codes * s[..., 0:1] + s[..., 1:2]).reshape(N, K)
+        ref = x.astype(np.float64) @ wn.T
+        got = _run(fmt, torch.from_numpy(x).to(dev), packs, N).cpu().numpy().astype(np.float64)
+        # fp16 results: half a unit of the last place, which near the bottom of the range is 2^-25
+        tol = np.maximum(np.abs(ref) * 2.0 ** -11, 2.0 ** -25) * 1.05 + 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(wn).T)
+        assert np.isfinite(got).all() and (np.abs(got - ref) <= tol).all()
+        packs, w = _packed(fmt, np.random.default_rng(1), N, K)
+        packs = [torch.from_numpy(a).to(dev) for a in packs]
+
+
+def test_wrappers_choose_the_same_result_on_both_sides(dev):
+    """The Python products just below and above the rows at which the launch changes."""
+    from axiomlm_amd.kernels import qmv_q2_k, qmv_q8_g64, qmv_ternary
+
+    rng = np.random.default_rng(5)
+    for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("ternary", qmv_ternary, (48, 49), 96, 320),
+                                ("q2", qmv_q2_k, (48, 49), 96, 320), ("ternary", qmv_ternary, (16, 17), 8192, 4096)):
+        packs, w = _packed(fmt, rng, N, K)
+        packs = [torch.from_numpy(a).to(dev) for a in packs]
+        x = rng.standard_normal((rows[1], K)).astype(np.float16)
+        ref = x.astype(np.float64) @ w.T
+        for M in rows:
+            got = fn(torch.from_numpy(x[:M]).to(dev), *packs).cpu().numpy().astype(np.float64)
+            assert np.linalg.norm(got - ref[:M]) <= REL * np.linalg.norm(ref[:M])
