@@ -1071,6 +1071,26 @@ int attn_flash_splits(int B, int Hq, int Hkv, int hd, int kv_dtype, int active_l
   return splits;
 }
 
+// A decode step of one sequence.  Grouped-query heads take the matrix-core kernel at every
+// length, with splits of about 128 keys up to one workgroup per CU: the vector kernel with eight
+// splits per head set fills 64 CUs at 8 KV heads and multiplies every key once per query head (us per
+// layer of a 7B-shape step with 32 / 8 heads and an FP8 cache, vector kernel / four / eight / 32
+// splits here: 100 keys 46.1 / 43.5 / 43.6 / 44.6, 1000 keys 48.9 / 44.9 / 44.1 / 44.8, 4000 keys
+// 61.0 / 50.5 / 47.0 / 45.6, 16000 keys 113 / 73 / 59 / 51).  One query head per KV head: splits
+// merged by a reduce launch only where eight leave over half of the CUs idle for long (4 heads
+// of 64, FP8: 4000 keys eight merged by the O projection 31.9, 32 splits 33.0; 8000 keys 36.4 / 34.1;
+// 16000 keys 43.1 / 35.7; 32 heads: never faster).
+int attn_step_splits(int Hq, int Hkv, int active_len) {
+  const int n_rep = Hq / Hkv;
+  const int fill = axm_ceil_div(axm_num_cus(), Hkv);  // one workgroup per CU
+  if (n_rep >= 2 && n_rep <= 16) {
+    int splits = 4;
+    while (splits < fill && splits < 64 && 128 * splits < active_len) splits <<= 1;
+    return splits;
+  }
+  return kAttnMaxParts * Hkv <= axm_num_cus() / 2 && active_len >= 1000 * kAttnMaxParts ? (fill < 32 ? fill : 32) : 0;
+}
+
 int attn_parts_splits(int B, int Hkv, int active_len) {
   // Split partials merged by the consumer cost no reduce launch, so the split
   // count aims at one workgroup per CU (measured on 32 heads x 128: eight
@@ -1110,10 +1130,10 @@ int launch_flash_decode_parts(const f16* q, const KvView& kv, int Hq, int active
   return launch_attn_dispatch<false>(p, qr, grid, s);
 }
 
-int launch_decode_mfma(const AttnParams& p, dim3 grid, hipStream_t s);
+int launch_decode_mfma(const AttnParams& p, dim3 grid, bool p32, hipStream_t s);
 
 int launch_flash_decode(const f16* q, const KvView& kv, f16* out, int Hq, int active_len, const int* active_len_dev,
-                        int n_splits, float* ws, hipStream_t s) {
+                        int n_splits, float* ws, hipStream_t s, bool p32) {
   AttnParams p{};
   p.q = q;
   p.kv = kv;
@@ -1128,7 +1148,7 @@ int launch_flash_decode(const f16* q, const KvView& kv, f16* out, int Hq, int ac
   p.scale_log2 = kLog2e / sqrtf((float)kv.hd);
   int rc;
   if (p.n_rep >= 2 && p.n_rep <= 16 && (kv.hd == 64 || kv.hd == 128)) {
-    rc = launch_decode_mfma(p, dim3(kv.B * kv.Hkv, n_splits), s);
+    rc = launch_decode_mfma(p, dim3(kv.B * kv.Hkv, n_splits), p32, s);
   } else {
     const int qr = pick_qr(p.n_rep);
     dim3 grid(kv.B * kv.Hkv, n_splits, (p.n_rep + qr - 1) / qr);
@@ -1224,10 +1244,11 @@ constexpr int kTreeRows = 64;    // query rows per workgroup (four waves of 16)
 // rescaling path takes the row maxima.  The caller sums l over each row's 16
 // lanes once after the last block.  The quotient o / l does not depend on m; the
 // fp16 weights P keep their relative precision up to 2^kMaxSlack.
+// With pt_lo the rest of each weight (what its fp16 rounding left out) goes to a second tile.
 constexpr float kMaxSlack = 8.f;
 template <int DT>
 __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows, float (&m)[4], float (&l)[4],
-                                              f32x4 (&o)[DT], f16* pt, int lq, int l16) {
+                                              f32x4 (&o)[DT], f16* pt, int lq, int l16, f16* pt_lo = nullptr) {
   if (__builtin_amdgcn_ballot_w64(grows)) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1246,7 +1267,11 @@ __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows
     for (int h = 0; h < 2; ++h) pr[h] = s[v][h] == kNegBig ? 0.f : fast_exp2(s[v][h] - m[v]);
     l[v] += pr[0] + pr[1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) pt[pt_index(4 * lq + v, 16 * h + l16)] = f2h(pr[h]);
+    for (int h = 0; h < 2; ++h) {
+      const f16 hi = f2h(pr[h]);
+      pt[pt_index(4 * lq + v, 16 * h + l16)] = hi;
+      if (pt_lo != nullptr) pt_lo[pt_index(4 * lq + v, 16 * h + l16)] = f2h(pr[h] - h2f(hi));
+    }
   }
 }
 
@@ -1473,7 +1498,9 @@ int launch_tree_mfma(const AttnParams& p, dim3 grid, hipStream_t s) {
 // (wave-private transposed V and P tiles, no barrier in the loop) and merge
 // their (m, l, o) through LDS at the end.
 // ---------------------------------------------------------------------------
-template <int KVT, int HD>
+// P32: the weights enter P V as two fp16 parts (22 bits, as the vector kernel's fp32 weights),
+// one more MFMA per tile.
+template <int KVT, int HD, bool P32>
 __global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
   constexpr int KSTEPS = HD / 32;
   constexpr int DT = HD / 16;
@@ -1482,6 +1509,7 @@ __global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
   constexpr int VROW = HD + 16;
   __shared__ __align__(16) f16 vr[4][kTreeKeys * VROW];
   __shared__ __align__(16) f16 pt[4][16 * kTreeKeys];
+  __shared__ __align__(16) f16 pt_lo[P32 ? 4 : 1][P32 ? 16 * kTreeKeys : 8];
   __shared__ float mrg[4][16][2 + HD];
   auto pt_at = pt_index;
   const int lane = threadIdx.x & 63;
@@ -1592,14 +1620,17 @@ __global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16);
+    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16, P32 ? pt_lo[wave] : nullptr);
     // The wave reads back its own LDS writes: DS operations of one wave complete
     // in order, and the reads below wait for them.
     const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
+    f16x8 pb;
+    if constexpr (P32) pb = *reinterpret_cast<const f16x8*>(&pt_lo[wave][pt_at(l16, 8 * lq)]);
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
       const f16x8 vb = v_operand(&vr[wave][16 * d], VROW, l16, lq);
       o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[d], 0, 0, 0);
+      if constexpr (P32) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pb, vb, o[d], 0, 0, 0);
     }
   };
   // With two buffers both blocks of an iteration run unconditionally and an odd
@@ -1658,20 +1689,26 @@ __global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
   }
 }
 
-int launch_decode_mfma(const AttnParams& p, dim3 grid, hipStream_t s) {
+template <int KVT, int HD>
+void launch_decode_mfma_p(const AttnParams& p, dim3 grid, bool p32, hipStream_t s) {
+  if (p32) hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, true>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, false>), grid, dim3(256), 0, s, p);
+}
+
+int launch_decode_mfma(const AttnParams& p, dim3 grid, bool p32, hipStream_t s) {
   const int hd = p.kv.hd;
   switch (p.kv.kv_dtype) {
     case AXM_KV_FP16:
-      if (hd == 128) hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_FP16, 128>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_FP16, 64>), grid, dim3(256), 0, s, p);
+      if (hd == 128) launch_decode_mfma_p<AXM_KV_FP16, 128>(p, grid, p32, s);
+      else launch_decode_mfma_p<AXM_KV_FP16, 64>(p, grid, p32, s);
       return 0;
     case AXM_KV_FP8:
-      if (hd == 128) hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_FP8, 128>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_FP8, 64>), grid, dim3(256), 0, s, p);
+      if (hd == 128) launch_decode_mfma_p<AXM_KV_FP8, 128>(p, grid, p32, s);
+      else launch_decode_mfma_p<AXM_KV_FP8, 64>(p, grid, p32, s);
       return 0;
     case AXM_KV_INT4:
-      if (hd == 128) hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_INT4, 128>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((decode_mfma_kernel<AXM_KV_INT4, 64>), grid, dim3(256), 0, s, p);
+      if (hd == 128) launch_decode_mfma_p<AXM_KV_INT4, 128>(p, grid, p32, s);
+      else launch_decode_mfma_p<AXM_KV_INT4, 64>(p, grid, p32, s);
       return 0;
   }
   axm_set_error("decode attention: bad kv dtype %d", p.kv.kv_dtype);

@@ -470,17 +470,40 @@ struct axm_runner {
     return v;
   }
 
+  // How a one-token step over active_len keys runs its attention: key splits (bucketed, so
+  // that one graph covers a range of lengths), splits of at most 64 keys on a smaller launch
+  // shape, and whether the split partials stay for the O projection to merge while staging its
+  // activations (parts) or a reduce launch merges them.
+  struct StepAttn {
+    int splits;
+    bool short_splits, parts;
+    int key() const { return 4 * splits + (parts ? 2 : 0) + (short_splits ? 1 : 0); }
+  };
+  StepAttn step_attn(int active_len) const {
+    int want = attn_step_splits(d.n_head, d.n_kv_head, active_len);
+    bool parts = false;
+    if (want == 0) {
+      want = parts_ok ? attn_parts_splits(1, d.n_kv_head, active_len)
+                      : attn_choose_splits(1, d.n_kv_head, active_len);
+      parts = parts_ok && want > 1;
+    }
+    int bucket = 1;
+    while (bucket < want) bucket <<= 1;
+    if (bucket > max_splits) bucket = max_splits;
+    return {bucket, active_len <= 64 * bucket, parts};
+  }
+
   // Enqueue the whole single-token step on stream s (no host synchronization).
   // The decode step after set_params_kernel, which has written the token's
   // embedding row into x.  Each launch group of a layer is its own member
   // (axm_runner_time_kernels times them one at a time).
-  int enqueue_step(int n_splits, bool short_splits, hipStream_t s) {
+  int enqueue_step(const StepAttn& at, hipStream_t s) {
     for (int i = 0; i < d.n_layer; ++i) {
       int rc = enqueue_qkv(i, s);
       if (rc) return rc;
-      rc = enqueue_attention(i, n_splits, short_splits, s);
+      rc = enqueue_attention(i, at, s);
       if (rc) return rc;
-      rc = enqueue_o(i, n_splits, s);
+      rc = enqueue_o(i, at, s);
       if (rc) return rc;
       rc = enqueue_gate_up(i, s);
       if (rc) return rc;
@@ -489,23 +512,6 @@ struct axm_runner {
     }
     return enqueue_lm_head(s);
   }
-
-  // The attention split count of a one-token step over active_len keys, bucketed
-  // so that one graph covers a range of lengths; splits of at most 64 keys use a
-  // smaller attention launch shape (the graph key carries both).
-  void split_shape(int active_len, int* bucket_out, bool* short_out) const {
-    const int splits = parts_ok ? attn_parts_splits(1, d.n_kv_head, active_len)
-                                : attn_choose_splits(1, d.n_kv_head, active_len);
-    int bucket = 1;
-    while (bucket < splits) bucket <<= 1;
-    if (bucket > max_splits) bucket = max_splits;
-    *bucket_out = bucket;
-    *short_out = active_len <= 64 * bucket;
-  }
-
-  // With parts_ok and more than one split, the attention leaves its split
-  // partials for the O projection to merge while staging its activations.
-  bool merge_in_o(int n_splits) const { return parts_ok && n_splits > 1; }
 
   // 1. QKV with RMSNorm prologue and RoPE / KV-write epilogue.
   int enqueue_qkv(int i, hipStream_t s) {
@@ -569,25 +575,25 @@ struct axm_runner {
   }
 
   // 2. attention over slots [0, active_len).
-  int enqueue_attention(int i, int n_splits, bool short_splits, hipStream_t s) {
+  int enqueue_attention(int i, const StepAttn& at, hipStream_t s) {
     KvView kv = kv_view(i);
-    if (merge_in_o(n_splits))
-      return launch_flash_decode_parts(q, kv, d.n_head, 0, params + P_ACTIVE, n_splits, parts_o, parts_ml,
-                                       short_splits, s);
-    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, n_splits, ws, s);
+    if (at.parts)
+      return launch_flash_decode_parts(q, kv, d.n_head, 0, params + P_ACTIVE, at.splits, parts_o, parts_ml,
+                                       at.short_splits, s);
+    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, at.splits, ws, s, true);
   }
 
   // 3. O projection, residual add into x.
-  int enqueue_o(int i, int n_splits, hipStream_t s) {
+  int enqueue_o(int i, const StepAttn& at, hipStream_t s) {
     GemvCall o{};
     o.x = attn_y;
     o.ldx = q_dim;
     o.resid = x;
     o.ldr = d.d_model;
-    if (merge_in_o(n_splits)) {
+    if (at.parts) {
       o.x_parts = parts_o;
       o.x_ml = parts_ml;
-      o.n_parts = n_splits;
+      o.n_parts = at.splits;
       o.parts_hd = d.head_dim;
     }
     return gemv(m_o[i], Q4_EPI_RESID, d.d_model, o, 1, s);
@@ -1258,12 +1264,10 @@ extern "C" int axm_runner_step(axm_runner_t r, const void* idx_dev, int64_t tok_
   const EmbedArgs emb{d.wte, (const f16*)d.wte_sb, d.wte_format, d.d_model, d.vocab_size, r->x};
   hipLaunchKernelGGL(set_params_kernel, dim3(1), dim3(256), 0, s, r->params, (const int64_t*)idx_dev, tok_host,
                      rope_pos, write_pos, active_len, r->argmax_keys, (d.vocab_size + 7) / 8, emb);
-  int bucket = 1;
-  bool short_splits = false;
-  r->split_shape(active_len, &bucket, &short_splits);
-  const int key = 2 * bucket + (short_splits ? 1 : 0);
+  const axm_runner::StepAttn at = r->step_attn(active_len);
+  const int key = at.key();
   if (r->mode == AXM_RUNNER_MODE_EAGER) {
-    int rc = r->enqueue_step(bucket, short_splits, s);
+    int rc = r->enqueue_step(at, s);
     if (rc) return rc;
   } else {
     auto it = r->graphs.find(key);
@@ -1273,7 +1277,7 @@ extern "C" int axm_runner_step(axm_runner_t r, const void* idx_dev, int64_t tok_
         axm_set_error("runner_step: stream capture failed to start");
         return -5;
       }
-      int rc = r->enqueue_step(bucket, short_splits, r->cap_stream);
+      int rc = r->enqueue_step(at, r->cap_stream);
       hipError_t e = hipStreamEndCapture(r->cap_stream, &g);
       if (rc) {
         if (g) (void)hipGraphDestroy(g);
@@ -1315,9 +1319,7 @@ extern "C" int axm_runner_time_kernels(axm_runner_t r, int position, int active_
   const EmbedArgs emb{d.wte, (const f16*)d.wte_sb, d.wte_format, d.d_model, d.vocab_size, r->x};
   hipLaunchKernelGGL(set_params_kernel, dim3(1), dim3(256), 0, s, r->params, (const int64_t*)nullptr, (int64_t)0,
                      position % d.rope_len, position, active_len, r->argmax_keys, (d.vocab_size + 7) / 8, emb);
-  int bucket = 1;
-  bool short_splits = false;
-  r->split_shape(active_len, &bucket, &short_splits);
+  const axm_runner::StepAttn at = r->step_attn(active_len);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
     if (e0) (void)hipEventDestroy(e0);
@@ -1330,8 +1332,8 @@ extern "C" int axm_runner_time_kernels(axm_runner_t r, int position, int active_
       const int i = j % d.n_layer;
       switch (k) {
         case 0: return r->enqueue_qkv(i, cs);
-        case 1: return r->enqueue_attention(i, bucket, short_splits, cs);
-        case 2: return r->enqueue_o(i, bucket, cs);
+        case 1: return r->enqueue_attention(i, at, cs);
+        case 2: return r->enqueue_o(i, at, cs);
         case 3: return r->enqueue_gate_up(i, cs);
         case 4: return r->enqueue_down(i, cs);
         default: return r->enqueue_lm_head(cs);
