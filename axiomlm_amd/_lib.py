@@ -67,6 +67,9 @@ _SIGNATURES = {
     "axm_pack_ternary": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "axm_qmv_q8_g64": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "axm_qmm_codes_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "axm_qmm_q2_k_gguf": (
+        c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]
+    ),
     "axm_qmm_q8_g64": (
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]
     ),

@@ -2,7 +2,7 @@
 #pragma once
 #include "q4_tile16.h"
 
-enum { kCodesQ8 = 0, kCodesQ2 = 1, kCodesTernary = 2 };
+enum { kCodesQ8 = 0, kCodesQ2 = 1, kCodesTernary = 2, kCodesQ2kGguf = 3 };  // the last: axm_qmm_q2_k_gguf only
 
 // a.w16 / a.sb16: the codes (uint8 [rows][K], or 2-bit [rows][K / 4]) and scales (fp16 (scale,
 // bias) [rows][K / 64][2], ternary [rows][K / 64]); a.x 16-byte aligned with ldx % 8 == 0; K % 64

@@ -320,6 +320,193 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   }
 }
 
+// The same over GGUF Q2_K blocks (84 bytes per 256 columns: 16 x (scale | min << 4), 64 bytes of
+// codes, d, dmin): y = sum_blocks d (sum_k sc q x) - dmin sum_s m_s (sum_k x), s: 16 columns.  A
+// stage is half a block, 32 code bytes per row of which lane quarter kq holds 8 kq .. + 7: column
+// 32 j + 8 kq + i of the half sits at bits 2 j of byte 8 kq + i, so k-step j of the MFMA takes the
+// columns in order.  sc q (at most 45) comes from a four-entry byte table of multiples of sc by one byte
+// permute and enters the MFMA as an exact half; the min term is one bf16 MFMA per half block
+// whose A holds the sixteen-column sums in three parts and whose B the integers m.
+template <int MB, int NT>
+__global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
+  constexpr int TOK = 16 * MB;
+  constexpr int kBlock = 84;
+  __shared__ __align__(16) f16 xs[2][TOK * kCStage];
+  __shared__ __align__(16) u32x2 sx[2][TOK * 8];  // bf16 parts (s0, s1, s2, 0) of each sub-block's sum
+
+  const int per = gridDim.x / 8;
+  const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (tile >= n_tile) return;
+  const int m0 = (tile % n_mblk) * TOK;
+  const int sp = (tile / n_mblk) % n_split;
+  const int nblk = tile / (n_mblk * n_split);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int unit = (nblk * kCWaves + wave) * NT;
+  const int kbA = sp * a.kb_per_split;
+  const int n_st = min(a.KB, kbA + a.kb_per_split) - kbA;  // half blocks of this split (>= 1)
+  const int NB = a.K / 256;
+  const __amdgpu_buffer_rsrc_t rw =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.w16, (short)0, (int)a.w16_bytes, 0x00020000);
+  const int wlane = l16 * NB * kBlock;
+
+  u32x2 cw[2][NT], sw[2][NT];
+  uint32_t dw[2][NT];
+  auto load_w = [&](int s, auto bc) {
+    constexpr int b = decltype(bc)::value;
+    const int hb = kbA + min(s, n_st - 1);  // past the split: its last half block again (never used)
+    const int h = hb & 1;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int base = ((unit + t) * 16 * NB + (hb >> 1)) * kBlock;  // wave-uniform; rows past N read zeros
+      cw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane + 8 * kq, base + 16 + 32 * h, 0));
+      sw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane, base + 8 * h, 0));
+      dw[b][t] = __builtin_amdgcn_raw_buffer_load_b32(rw, wlane, base + 80, 0);
+    }
+  };
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
+  const int xrow = 4 * wave + kq;
+  const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  auto load_x = [&](int s, auto bc) {
+    constexpr int b = decltype(bc)::value;
+    const int so = (kbA + min(s, n_st - 1)) * (kCStage * 2);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
+                                               so + i * 32 * a.ldx, 0, 0);
+  };
+
+  f32x4 acc[NT][MB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  auto stage = [&](int s, auto bc, auto bn) {
+    constexpr int b = decltype(bc)::value;
+    load_x(s + 1, bn);
+    load_w(s + 1, bn);
+    {
+      const f16x2 one = {(f16)1.f, (f16)1.f};
+      int tq = tid;
+      asm volatile("" : "+v"(tq));  // addresses formed here (see codes_gemm_kernel)
+      for (int p = tq; p < 8 * TOK; p += kCThreads) {
+        const int r = p >> 3, g = p & 7;
+        float v = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const u32x4 x = *reinterpret_cast<const u32x4*>(&xs[b][r * kCStage + (((2 * g + i) ^ (r & 15)) * 8)]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_fdot2(as_h2(x[e]), one, v, false);
+        }
+        const uint32_t s0 = __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u;
+        const float r1 = v - __builtin_bit_cast(float, s0);
+        const uint32_t s1 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+        const uint32_t s2 = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, s1));
+        sx[b][p] = u32x2{(s0 >> 16) | s1, s2 >> 16};
+      }
+    }
+    const f16* xa = &xs[b][l16 * kCStage];
+    // Two passes of NT / 2 tiles bound the sums in flight.
+    constexpr int NH = NT / 2;
+#pragma unroll
+    for (int th = 0; th < 2; ++th) {
+      f32x4 d[NH][MB];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
+        f16x8 A[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          A[mb] = *reinterpret_cast<const f16x8*>(xa + mb * 16 * kCStage + (((4 * j + kq) ^ l16) * 8));
+#pragma unroll
+        for (int u = 0; u < NH; ++u) {
+          const int t = th * NH + u;
+          const uint32_t sc = (sw[b][t][j >> 1] >> (16 * (j & 1) + 8 * (kq >> 1))) & 15u;
+          const uint32_t lut = sc * 0x03020100u;  // bytes 0, sc, 2 sc, 3 sc
+          const f16x2 off = {(f16)1024.f, (f16)1024.f};
+          u32x4 o;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const uint32_t v = __builtin_amdgcn_perm(0u, lut, (cw[b][t][i] >> (2 * j)) & 0x03030303u);
+            o[2 * i] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)) - off);
+            o[2 * i + 1] = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)) - off);
+          }
+          const f16x8 q = __builtin_bit_cast(f16x8, o);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            d[u][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mb], q, j == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[u][mb], 0,
+                                                              0, 0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NH; ++u) {
+        const float dd = h2f(u16_as_h((uint16_t)dw[b][th * NH + u]));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            acc[th * NH + u][mb][v] = __builtin_fmaf(dd, d[u][mb][v], acc[th * NH + u][mb][v]);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    // The half block's min term: its sums are all written now; scales stay in buffer b.
+    bf16x8 S[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+      S[mb] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&sx[b][(16 * mb + l16) * 8 + 2 * kq]));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      // Sub-blocks 2 kq and 2 kq + 1 of the half: their bytes, mins in the high nibbles.
+      const uint32_t by = (kq & 2 ? sw[b][t].y : sw[b][t].x) >> (16 * (kq & 1));
+      const uint32_t ma = __builtin_bit_cast(uint32_t, (float)((by >> 4) & 15u)) & 0xFFFF0000u;
+      const uint32_t mc = __builtin_bit_cast(uint32_t, (float)((by >> 12) & 15u)) & 0xFFFF0000u;
+      const u32x4 bw = {(ma >> 16) | ma, ma >> 16, (mc >> 16) | mc, mc >> 16};
+      const float dm = -h2f(u16_as_h((uint16_t)(dw[b][t] >> 16)));
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const f32x4 e = __builtin_amdgcn_mfma_f32_16x16x32_bf16(S[mb], __builtin_bit_cast(bf16x8, bw),
+                                                                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[t][mb][v] = __builtin_fmaf(dm, e[v], acc[t][mb][v]);
+      }
+    }
+  };
+
+  load_x(0, B0{});
+  load_w(0, B0{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int s = 0;;) {
+    stage(s, B0{}, B1{});
+    if (++s >= n_st) break;
+    stage(s, B1{}, B0{});
+    if (++s >= n_st) break;
+  }
+
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int row = (unit + t) * 16 + l16;
+    if (unit + t >= a.n_units || (n_split == 1 && row >= a.N)) continue;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int tok = m0 + 16 * mb + 4 * kq + v;
+        if (tok >= a.M_tokens) continue;
+        if (n_split == 1) t16g_store<Q4_EPI_STORE>(a, tok, row, acc[t][mb][v], 0.f);
+        else a.part_ws[((size_t)sp * a.M_tokens + tok) * a.part_cols + row] = acc[t][mb][v];
+      }
+  }
+}
+
 struct CodesPlan {
   int mb, nt, splits;
 };
@@ -349,6 +536,22 @@ void codes_launch(const T16Args& a, int M, int splits, hipStream_t s) {
   hipLaunchKernelGGL((codes_gemm_kernel<F, EPI, MB, NT>), dim3(8 * axm_ceil_div(n_tile, 8)), dim3(kCThreads), 0, s, a,
                      n_mblk, splits, n_tile);
 }
+template <int MB, int NT>
+void q2k_launch(const T16Args& a, int M, int splits, hipStream_t s) {
+  const int n_mblk = axm_ceil_div(M, 16 * MB);
+  const int n_tile = n_mblk * splits * axm_ceil_div(a.n_units, kCWaves * NT);
+  hipLaunchKernelGGL((q2k_gemm_kernel<MB, NT>), dim3(8 * axm_ceil_div(n_tile, 8)), dim3(kCThreads), 0, s, a, n_mblk,
+                     splits, n_tile);
+}
+void q2k_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t s) {
+  switch (p.mb) {
+    case 1: return q2k_launch<1, 2>(a, M, p.splits, s);
+    case 2: return q2k_launch<2, 2>(a, M, p.splits, s);
+    case 3: return q2k_launch<3, 4>(a, M, p.splits, s);
+    default: return q2k_launch<4, 4>(a, M, p.splits, s);
+  }
+}
+
 template <int F, int EPI>
 void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t s) {
   switch (p.mb) {
@@ -362,6 +565,9 @@ void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t
 }  // namespace
 
 bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int rows, int fmt) {
+  if (fmt == kCodesQ2kGguf)
+    return K > 0 && K % 256 == 0 && K <= 16384 && (size_t)rows * (K / 256) * 84 < (size_t)0x7FFFFFF0 &&
+           ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 3) == 0;
   const size_t code_bytes = (size_t)rows * K / (fmt == kCodesQ8 ? 1 : 4);
   const uintptr_t wa = fmt == kCodesQ8 ? 15 : 3, sa = fmt == kCodesTernary ? 1 : 3;
   return K > 0 && K % 64 == 0 && K <= 32768 && code_bytes < (size_t)0x7FFFFFF0 && ((uintptr_t)x & 15) == 0 &&
@@ -394,9 +600,11 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
   else if (ws_bytes < p.splits * one) p.splits = (int)(ws_bytes / one);
   a.kb_per_split = axm_ceil_div(a.KB, p.splits);
   p.splits = axm_ceil_div(a.KB, a.kb_per_split);
-  a.w16_bytes = (size_t)rows * a.K / (fmt == kCodesQ8 ? 1 : 4);
+  a.w16_bytes = fmt == kCodesQ2kGguf ? (size_t)rows * (a.K / 256) * 84
+                                    : (size_t)rows * a.K / (fmt == kCodesQ8 ? 1 : 4);
   a.sb16_bytes = (size_t)rows * (a.K / 64) * (fmt == kCodesTernary ? 2 : 4);
-  if (fmt == kCodesQ2) codes_launch_shape<kCodesQ2, Q4_EPI_STORE>(a, M, p, s);
+  if (fmt == kCodesQ2kGguf) q2k_launch_shape(a, M, p, s);
+  else if (fmt == kCodesQ2) codes_launch_shape<kCodesQ2, Q4_EPI_STORE>(a, M, p, s);
   else if (fmt == kCodesTernary) codes_launch_shape<kCodesTernary, Q4_EPI_STORE>(a, M, p, s);
   else if (epi == Q4_EPI_STORE) codes_launch_shape<kCodesQ8, Q4_EPI_STORE>(a, M, p, s);
   else if (epi == Q4_EPI_RESID) codes_launch_shape<kCodesQ8, Q4_EPI_RESID>(a, M, p, s);
@@ -411,20 +619,21 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
 // fill LDS); this kernel takes over where they need four, or two of a large matrix (ternary,
 // 12288 x 4096: 16 rows in one launch 23.3 us against 22.3 here, 17 in two 28.7 / 23.2, 64 in four
 // 90.7 / 35.4; 4096 x 4096: 32 in two 13.6 / 16.4, 48 in three 20.2 / 20.9, 64 in four 26.4 / 24.1;
-// 4096 x 11008: six in one 11.5 / 17.4, eight in two 20.2 / 17.4).
-static bool lowbit_rows_use_codes(int M, int K, int N) {
-  const int per = lowbit_mfma_rows(N, K);
+// 4096 x 11008: six in one 11.5 / 17.4, eight in two 20.2 / 17.4; GGUF 4096 x 11008: eight in two
+// 16.2 / 16.8, twelve 17.8 / 17.2, sixteen in three 25.5 / 17.7, 64 in ten 87.5 / 31.9).
+static bool lowbit_rows_use_codes(int fmt, int M, int K, int N) {
+  const int per = fmt == kCodesQ2kGguf ? q2k_gguf_mfma_rows(K) : lowbit_mfma_rows(N, K);
   const int launches = per > 0 ? axm_ceil_div(M, per) : M;
-  return launches >= 4 || (launches >= 2 && (size_t)N * K >= (size_t)32 << 20);
+  return launches >= 4 || (launches >= 2 && M >= (fmt == kCodesQ2kGguf ? 12 : 5) && (size_t)N * K >= (size_t)32 << 20);
 }
 
 // Whether M rows of a format go through this kernel (shapes and alignment apart).
 static bool rows_use_codes(int fmt, int M, int K, int N) {
-  return fmt == kCodesQ8 ? M >= kCodesQ8MinRows : M > 4 && lowbit_rows_use_codes(M, K, N);
+  return fmt == kCodesQ8 ? M >= kCodesQ8MinRows : M > 4 && lowbit_rows_use_codes(fmt, M, K, N);
 }
 
 extern "C" size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N) {
-  if (format < kCodesQ8 || format > kCodesTernary || M <= 0 || K <= 0 || N <= 0) return 0;
+  if (format < kCodesQ8 || format > kCodesQ2kGguf || M <= 0 || K <= 0 || N <= 0) return 0;
   return rows_use_codes(format, M, K, N) ? codes_gemm_ws_bytes(M, K, N, Q4_EPI_STORE) : 0;
 }
 
@@ -470,5 +679,14 @@ extern "C" int axm_qmm_q2_k(const void* x, const void* w_packed, const void* sca
     return axm_qmv_q2_k(x, w_packed, scales_biases, bias, y, M, K, N, stream);
   AXM_CHECK_ARG(x && w_packed && scales_biases && y && N > 0, -1, "qmm_q2_k: bad arguments");
   return qmm_codes(kCodesQ2, "qmm_q2_k", x, w_packed, scales_biases, bias, y, M, K, N, workspace, workspace_bytes,
+                   (hipStream_t)stream);
+}
+
+extern "C" int axm_qmm_q2_k_gguf(const void* x, const void* blocks, const void* bias, void* y, int M, int K, int N,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
+  if (K <= 0 || !rows_use_codes(kCodesQ2kGguf, M, K, N) || !codes_gemm_takes(x, blocks, nullptr, K, N, kCodesQ2kGguf))
+    return axm_qmv_q2_k_gguf(x, blocks, bias, y, M, K, N, stream);
+  AXM_CHECK_ARG(x && blocks && y && N > 0, -1, "qmm_q2_k_gguf: bad arguments");
+  return qmm_codes(kCodesQ2kGguf, "qmm_q2_k_gguf", x, blocks, nullptr, bias, y, M, K, N, workspace, workspace_bytes,
                    (hipStream_t)stream);
 }

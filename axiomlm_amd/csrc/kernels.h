@@ -134,3 +134,4 @@ int launch_prompt_attention(const f16* q, const KvView& kv, f16* out, int Hq, in
 // Rows of one matrix-core launch of the 2-bit GEMVs at this K (lowbit_gemv.hip), 0 where they
 // have none.
 int lowbit_mfma_rows(int N, int K);
+int q2k_gguf_mfma_rows(int K);  // the same of the GGUF Q2_K GEMV (q2k_gguf.hip)

@@ -502,6 +502,8 @@ extern "C" int axm_dequantize_q2_k_gguf(const void* blocks, int N, int K, void* 
   return 0;
 }
 
+int q2k_gguf_mfma_rows(int K) { return q2k_mfma_max_tokens(K); }
+
 extern "C" int axm_qmv_q2_k_gguf(const void* x, const void* blocks, const void* bias, void* y, int M, int K, int N,
                                  void* stream) {
   AXM_CHECK_ARG(x && blocks && y, -1, "qmv_q2_k_gguf: null pointer");

@@ -317,7 +317,7 @@ def dequant_q8_rows(indices, w_packed, scales_biases) -> torch.Tensor:
 
 
 def _codes_workspace(fmt: int, M: int, K: int, N: int, device):
-    """Workspace of the several-row products (0 Q8_G64, 1 affine 2-bit, 2 ternary)."""
+    """Workspace of the several-row products (0 Q8_G64, 1 affine 2-bit, 2 ternary, 3 GGUF Q2_K)."""
     n = _lib.lib().axm_qmm_codes_workspace_bytes(fmt, M, K, N)
     return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
 
@@ -485,8 +485,14 @@ def qmv_q2_k_gguf(x, blocks, bias=None) -> torch.Tensor:
     M = x.numel() // K
     y = torch.empty((*x.shape[:-1], N), dtype=torch.float16, device=x.device)
     b = None if bias is None else bias.to(device=x.device, dtype=torch.float16).contiguous()
-    _lib.check(_lib.lib().axm_qmv_q2_k_gguf(_lib.ptr(x.contiguous()), _lib.ptr(blocks.contiguous()), _lib.ptr(b),
-                                            _lib.ptr(y), M, K, N, _lib.stream_of(x.device)),
+    if M <= 4:  # the GEMV
+        _lib.check(_lib.lib().axm_qmv_q2_k_gguf(_lib.ptr(x.contiguous()), _lib.ptr(blocks.contiguous()), _lib.ptr(b),
+                                                _lib.ptr(y), M, K, N, _lib.stream_of(x.device)),
+                   "qmv_q2_k_gguf")
+        return y
+    ws, n = _codes_workspace(3, M, K, N, x.device)
+    _lib.check(_lib.lib().axm_qmm_q2_k_gguf(_lib.ptr(x.contiguous()), _lib.ptr(blocks.contiguous()), _lib.ptr(b),
+                                            _lib.ptr(y), M, K, N, _lib.ptr(ws), n, _lib.stream_of(x.device)),
                "qmv_q2_k_gguf")
     return y
 

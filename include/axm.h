@@ -128,7 +128,7 @@ int axm_qmv_q2_k(const void* x, const void* w_packed, const void* scales_biases,
  * (exact code products, fp32 sums), with K split across workgroups as far as the workspace
  * (axm_qmm_codes_workspace_bytes for the preferred split; NULL / 0 is allowed) lets it; fewer
  * rows as the qmv entries.  Replaces qmm_q8_g64_mps, qmm_ternary_mps, qmm_q2_k_mps. */
-size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N); /* 0: Q8_G64, 1: affine 2-bit, 2: ternary */
+size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N); /* 0: Q8_G64, 1: affine 2-bit, 2: ternary, 3: GGUF */
 int axm_qmm_q8_g64(const void* x, const void* w_packed, const void* sb, const void* bias, void* y, int M, int K, int N,
                    void* workspace, size_t workspace_bytes, void* stream);
 int axm_qmm_ternary(const void* x, const void* w_packed, const void* scales, const void* bias, void* y, int M, int K,
@@ -151,6 +151,9 @@ int axm_dequantize_q2_k_gguf(const void* blocks, int N, int K, void* out, void* 
  * products: one token on v_dot2_f32_f16, two to sixteen per launch on MFMA. */
 int axm_qmv_q2_k_gguf(const void* x, const void* blocks, const void* bias, void* y, int M, int K, int N,
                       void* stream);
+
+int axm_qmm_q2_k_gguf(const void* x, const void* blocks, const void* bias, void* y, int M, int K, int N,
+                      void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- norms / activations / argmax ---------------------------------------- */
 /* rmsnorm_infer_mps (mps_kernels.mm:247-266; math of axiomlm/models/modules.py:41-43). */

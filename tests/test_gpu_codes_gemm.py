@@ -25,6 +25,13 @@ def _packed(fmt, rng, N, K):
         p, s = fm.pack_linear_ternary(w)
         q = fm.ternary_decode_bytes(p).reshape(N, K // 64, 64).astype(np.float64)
         return (p, s), (q * s[..., None]).reshape(N, K)
+    if fmt == "gguf":
+        b = fm.pack_q2_k_gguf(w)
+        at, shift, sub = fm.q2k_element_maps()
+        q = ((b[:, :, 16:80][:, :, at] >> shift) & 3).astype(np.float64)
+        sc = b[:, :, :16][:, :, sub]
+        d, dmin = (b[:, :, o:o + 2].copy().view(np.float16).astype(np.float64) for o in (80, 82))
+        return (b, b), (d * (sc & 15) * q - dmin * (sc >> 4)).reshape(N, K)
     p, s = fm.pack_linear_q2_k(w)
     q = ((p[..., None] >> (2 * np.arange(4))) & 3).reshape(N, K // 64, 64).astype(np.float64)
     return (p, s), (q * s[..., 0:1] + s[..., 1:2].astype(np.float64)).reshape(N, K)
@@ -36,11 +43,12 @@ def _run(fmt, x, packs, N, bias=None, ws=True):
 
     L = _lib.lib()
     M, K = x.shape
-    fn = {"q8": L.axm_qmm_q8_g64, "ternary": L.axm_qmm_ternary, "q2": L.axm_qmm_q2_k}[fmt]
+    fn = {"q8": L.axm_qmm_q8_g64, "ternary": L.axm_qmm_ternary, "q2": L.axm_qmm_q2_k, "gguf": L.axm_qmm_q2_k_gguf}[fmt]
+    weights = [_lib.ptr(p) for p in (packs[:1] if fmt == "gguf" else packs)]
     y = torch.empty((M, N), dtype=torch.float16, device=x.device)
-    n = L.axm_qmm_codes_workspace_bytes({"q8": 0, "q2": 1, "ternary": 2}[fmt], M, K, N) if ws else 0
+    n = L.axm_qmm_codes_workspace_bytes({"q8": 0, "q2": 1, "ternary": 2, "gguf": 3}[fmt], M, K, N) if ws else 0
     buf = torch.empty(max(n, 1), dtype=torch.uint8, device=x.device)
-    _lib.check(fn(_lib.ptr(x), _lib.ptr(packs[0]), _lib.ptr(packs[1]), _lib.ptr(bias), _lib.ptr(y), M, K, N,
+    _lib.check(fn(_lib.ptr(x), *weights, _lib.ptr(bias), _lib.ptr(y), M, K, N,
                   _lib.ptr(buf) if n else None, n, _lib.stream_of(x.device)), fmt)
     return y
 
@@ -51,12 +59,14 @@ SHAPES = [(5, 16, 64), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96,
           (129, 2056, 1024), (17, 40, 192)]
 
 
-@pytest.mark.parametrize("fmt", ["q8", "ternary", "q2"])
+@pytest.mark.parametrize("fmt", ["q8", "ternary", "q2", "gguf"])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("ws", [True, False])
 def test_codes_gemm_matches_float64(dev, fmt, M, N, K, ws):
     if fmt != "q8":
         M += 64  # four launches of 16 rows and more
+    if fmt == "gguf":
+        K = (K + 255) // 256 * 256
     rng = np.random.default_rng(M + N + K)
     packs, w = _packed(fmt, rng, N, K)
     packs = [torch.from_numpy(a).to(dev) for a in packs]
@@ -77,7 +87,7 @@ def test_codes_gemm_matches_float64(dev, fmt, M, N, K, ws):
     assert np.linalg.norm(got.astype(np.float64) - (ref + bias)) <= 2 * REL * np.linalg.norm(ref + bias)
 
 
-@pytest.mark.parametrize("fmt", ["q8", "q2"])
+@pytest.mark.parametrize("fmt", ["q8", "q2", "gguf"])
 def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
     """Group sums beyond the fp16 range and activations near its bottom keep 24 bits in the bias term."""
     rng = np.random.default_rng(1)
@@ -87,7 +97,16 @@ def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
     for scale in (3000.0, 2.0 ** -18):
         x = (np.abs(rng.standard_normal((M, K))) * scale).astype(np.float16)
         wn = w
-        if scale > 1:  # keep the results in range: smaller scales and biases, same codes
+        if scale > 1 and fmt == "gguf":  # smaller d and dmin
+            b = packs[0].cpu().numpy()
+            d = (b[:, :, 80:84].copy().view(np.float16).astype(np.float32) * 2.0 ** -6).astype(np.float16)
+            b[:, :, 80:84] = d.view(np.uint8)
+            packs = [torch.from_numpy(b).to(dev)] * 2
+            at, shift, sub = fm.q2k_element_maps()
+            sc = b[:, :, :16][:, :, sub]
+            d = d.astype(np.float64)
+            wn = (d[:, :, :1] * (sc & 15) * ((b[:, :, 16:80][:, :, at] >> shift) & 3) - d[:, :, 1:] * (sc >> 4)).reshape(N, K)
+        elif scale > 1:  # keep the results in range: smaller scales and biases, same codes
             packs[1] = (packs[1].double() * 2.0 ** -6).half()
             s = packs[1].cpu().numpy().astype(np.float64)
             p = packs[0].cpu().numpy()
