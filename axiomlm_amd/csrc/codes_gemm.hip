@@ -649,6 +649,7 @@ static int qmm_codes(int fmt, const char* who, const void* x, const void* w, con
   a.y = (f16*)y;
   a.ldy = N;
   a.bias = (const f16*)bias;
+  a.bias_f32 = fmt != kCodesQ8;  // as the formats' GEMVs
   const int rc = codes_gemm_launch(fmt, a, M, Q4_EPI_STORE, (float*)ws, ws_bytes, s);
   if (rc) return rc;
   AXM_LAUNCH_CHECK(who);

@@ -16,6 +16,7 @@ struct T16Args {
   f16* y;
   int ldy;
   const f16* bias;
+  int bias_f32;        // several-row GEMMs: the bias joins the fp32 sum (one rounding), not the fp16 result
   const f16* ln_w;     // optional fused RMSNorm (torch-CPU fp16 semantics)
   float eps;
   f16* x_norm_out;     // optional export of the normalized activations [M][K]

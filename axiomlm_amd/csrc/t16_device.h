@@ -60,8 +60,9 @@ __device__ __forceinline__ void t16g_store(const T16Args& a, int tok, int row, f
     const f16 sg = f2h(t16_silu(h2f(g)));
     a.y[(size_t)tok * a.ldy + row] = f2h(h2f(sg) * h2f(u));
   } else {
+    if (a.bias_f32 && a.bias != nullptr) v0 += h2f(a.bias[row]);
     f16 h = f2h(v0);
-    if (a.bias != nullptr) h = f2h(h2f(h) + h2f(a.bias[row]));
+    if (!a.bias_f32 && a.bias != nullptr) h = f2h(h2f(h) + h2f(a.bias[row]));
     if (EPI == Q4_EPI_STORE) {
       a.y[(size_t)tok * a.ldy + row] = h;
     } else {
@@ -91,12 +92,13 @@ __device__ __forceinline__ void t16g_store4(const T16Args& a, int tok, int row, 
       h[e] = f2h(h2f(f2h(t16_silu(h2f(g)))) * h2f(u));
     }
   } else {
+    f16x4 b = {};
+    if (a.bias != nullptr) b = *reinterpret_cast<const f16x4*>(a.bias + row);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) h[e] = f2h(v0[e]);
-    if (a.bias != nullptr) {
-      const f16x4 b = *reinterpret_cast<const f16x4*>(a.bias + row);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) h[e] = f2h(h2f(h[e]) + h2f(b[e]));
+    for (int e = 0; e < 4; ++e) {
+      if (a.bias_f32) v0[e] += h2f(b[e]);
+      h[e] = f2h(v0[e]);
+      if (!a.bias_f32 && a.bias != nullptr) h[e] = f2h(h2f(h[e]) + h2f(b[e]));
     }
   }
   if (EPI == Q4_EPI_RESID) {

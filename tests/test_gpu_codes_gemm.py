@@ -87,6 +87,29 @@ def test_codes_gemm_matches_float64(dev, fmt, M, N, K, ws):
     assert np.linalg.norm(got.astype(np.float64) - (ref + bias)) <= 2 * REL * np.linalg.norm(ref + bias)
 
 
+@pytest.mark.parametrize("fmt", ["ternary", "q2", "gguf"])
+@pytest.mark.parametrize("N", [64, 70])
+@pytest.mark.parametrize("ws", [True, False])
+def test_codes_gemm_bias_joins_the_fp32_sum(dev, fmt, N, ws):
+    """A bias that cancels the fp16 product leaves what that rounding would have dropped: the 2-bit formats round
+    once, after the bias.  Rounding before it would leave about 2^-13 of the product (its own rounding, rms); the
+    bound is the final rounding and the fp32 sums: K / 32 matrix-core adds and eight more, rounding at random, each
+    2^-24 of at most the sum of magnitudes, a weight's code and bias parts taken as three times the weight."""
+    M, K = 80, 512
+    rng = np.random.default_rng(N)
+    packs, w = _packed(fmt, rng, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    ref = x.astype(np.float64) @ w.T
+    bias = -ref[7].astype(np.float16)
+    got = _run(fmt, torch.from_numpy(x).to(dev), [torch.from_numpy(a).to(dev) for a in packs], N,
+               torch.from_numpy(bias).to(dev), ws).cpu().numpy()[7].astype(np.float64)
+    want = ref[7] + bias
+    sums = 3 * np.abs(x[7].astype(np.float64)) @ np.abs(w).T
+    bound = 2.0 ** -11 * np.linalg.norm(want) + np.sqrt(K / 32 + 8) * 2.0 ** -24 * np.linalg.norm(sums)
+    assert bound < 2.0 ** -14 * np.linalg.norm(ref[7])  # below what the extra rounding would leave
+    assert np.linalg.norm(got - want) <= bound
+
+
 @pytest.mark.parametrize("fmt", ["q8", "q2", "gguf"])
 def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
     """Group sums beyond the fp16 range and activations near its bottom keep 24 bits in the bias term."""
