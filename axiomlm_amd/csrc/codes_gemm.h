@@ -12,5 +12,6 @@ bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int r
 size_t codes_gemm_ws_bytes(int M, int K, int N, int epi);
 int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s);
 // Rows from which Q8 uses it: its GEMV takes four rows a launch (12288 x 4096: four rows 16.6 us
-// against 24; five 29.8 against 24.5, sixteen 67 against 25, 64 rows 244 against 40).
+// against 20; five 29.8 against 20, sixteen 67 against 21, 64 rows 244 against 33.5; 4096 x 4096: five
+// 14.5 against 11.9).
 constexpr int kCodesQ8MinRows = 5;

@@ -14,12 +14,14 @@
 // Workgroup: four waves, 16 MB rows of x, NT weight tiles of 16 rows per wave.  Lane (row r of a
 // tile, quarter q) holds columns 16 q .. + 15 of a group, so its codes of a group are 16 (Q8) or
 // 4 contiguous bytes; the MFMA's k order is that order of columns, also for the x fragments.
-// Activations go to LDS and weights to registers one 128-column stage ahead as in the
-// many-row tile16 GEMM (rows_gemm.hip).
+// Activations go to LDS one 128-column stage ahead as in the many-row tile16 GEMM
+// (rows_gemm.hip), Q8 codes to registers a stage ahead (64-row tiles: a group), scales and 2-bit
+// codes two stages at a time (load_pair).
 //
 // Measured (us, graph of back-to-back calls, against the GEMVs of up to 4 / 16 rows a launch):
-// Q8 12288 x 4096, 16 rows 67 -> 25, 64 rows 244 -> 40, 1000 rows -> 227 (443 TFLOP/s); ternary 64
-// rows 91 -> 35, 1000 rows 202 (498).  Large launches are bound by the vector units: per group
+// Q8 12288 x 4096, 16 rows 67 -> 21, 64 rows 244 -> 33.5, 1000 rows -> 177 (569 TFLOP/s); ternary 64
+// rows 91 -> 31, 1000 rows 150 (671).  (Scales and codes loaded group by group: 25, 40, 227; 35,
+// 202.)  Large launches are bound by the vector units: per group
 // and 16 x 16 tile four multiply-adds (16 cycles) and a share of the code expansion stand beside
 // 32 MFMA cycles.
 #include <type_traits>
@@ -37,6 +39,25 @@ constexpr int kCStage = 128;
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Lane row i (lanes 16 i .. + 15) of v, in every lane row: i = 0, 1 in the first result pair
+// (v_permlane32_swap of two copies gives rows 0 1 0 1 and 2 3 2 3, v_permlane16_swap of two
+// copies of those one row each).
+template <int HALF>
+__device__ __forceinline__ u32x2 lane_rows(uint32_t v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  const uint32_t h = HALF == 0 ? p[0] : p[1];
+  const auto q = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+  return u32x2{q[0], q[1]};
+}
+// 4 x 4 transpose of words between a lane's four registers and the four lane rows.
+__device__ __forceinline__ u32x4 lane_transpose(u32x4 w) {
+  const auto a = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return u32x4{c[0], c[1], d[0], d[1]};
+}
 
 // One lane's codes of one group (16 columns) and their two MFMA operands (8 columns each).
 template <int F>
@@ -66,9 +87,6 @@ struct Codes<kCodesQ8> {
 struct Codes2 {
   static constexpr int kRowBytes64 = 16;
   uint32_t w;
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    w = __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-  }
   // Fields 8 c .. 8 c + 7 minus sub: the fields in the low half and, one field on, in the high
   // half, so that a mask yields neighbours as a pair (1024 + q or 64 + q, as unpack_word).
   __device__ __forceinline__ static f16x8 fields(uint32_t w, int c, float sub) {
@@ -95,12 +113,20 @@ struct Codes<kCodesTernary> : Codes2 {
   }
 };
 
+// Waits until all but the wave's last N loads are done.  (Loads complete in issue order.)
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 template <int F, int EPI, int MB, int NT>
 __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
   constexpr bool kPair = EPI == Q4_EPI_SWIGLU;
   constexpr bool kBias = F != kCodesTernary;
   constexpr int TOK = 16 * MB;
   constexpr int UPW = kPair ? NT / 2 : NT;  // units per wave
+  constexpr bool kQ8 = F == kCodesQ8;
+  constexpr int RING = MB > 3 ? 2 : 4;
   __shared__ __align__(16) f16 xs[2][TOK * kCStage];
   // Group sums of four groups (a pair of stages) as bf16 parts (s0, s1, s2, s0, s1, s2, 0, 0).
   __shared__ __align__(16) u32x4 sx[kBias ? 2 : 1][kBias ? TOK * 4 : 1];
@@ -127,31 +153,43 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc((void*)a.sb16, (short)0, (int)a.sb16_bytes, 0x00020000);
 
-  // This lane's codes and scales of tile 0, and the (wave-uniform) distance of tile t from it:
-  // an up tile starts a.N rows after its gate tile.  Rows past the matrix read zeros and are
-  // never stored.
-  const int wlane = l16 * KG * RB + kq * (RB / 4), slane = l16 * KG * SB;
+  // This lane's codes of tile 0, and the (wave-uniform) first row of tile t: an up tile starts
+  // a.N rows after its gate tile.  Tiles past the matrix read the last one, the last one's rows
+  // past it zeros; neither is stored.
+  const int wlane = l16 * KG * RB + kq * (RB / 4);
   int row0[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) row0[t] = (unit + t % UPW) * 16 + (kPair && t >= UPW ? a.N : 0);
-  // Codes and scales of one group per buffer: the next group's are requested before a group
-  // is consumed.  (A whole stage ahead took 64 more registers with Q8; eight waves of a CU with
-  // 4 KB each in flight already cover the memory's latency.)
-  Codes<F> wr[2][NT];
-  uint32_t sr[2][NT];
+  for (int t = 0; t < NT; ++t) row0[t] = min(unit + t % UPW, a.n_units - 1) * 16 + (kPair && t >= UPW ? a.N : 0);
   // The row's last stage has one group only if K % 128 == 64: its second one reads that group
   // again, and zeros of x.
   const int s_tail = a.K % kCStage != 0 && kbA + n_st == a.KB ? n_st - 1 : -1;
   const int n_grp = 2 * n_st - (s_tail >= 0 ? 1 : 0);
-  auto load_w = [&](int gi, auto bc) {
-    constexpr int b = decltype(bc)::value;
-    const int g = 2 * kbA + min(gi, n_grp - 1);  // past the split: its last group again (never used)
+
+  // Scales (and biases), and 2-bit codes, are requested for two stages at a time, lane quarter kq
+  // taking group kq of the four: 16 (64) contiguous bytes per row and request.  Group by group each
+  // request touched 16 cache lines for 4 bytes each, and those requests, not bytes or latency,
+  // bound the launch (Q8, 22016 x 4096, 75 rows: 87 us, 59 with constant scales).
+  uint32_t sv[NT], sn[NT];
+  u32x4 cv[kQ8 ? 1 : NT], cn[kQ8 ? 1 : NT];
+  auto load_pair = [&](int p) {
+    const int g = min(4 * p + kq, n_grp - 1);  // past the split: its last group again
+    const int so = (l16 * KG + g) * SB, wo = (l16 * KG + g) * RB;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int ch = row0[t] * KG + g;  // of the tile's first row
-      wr[b][t].load(rw, wlane, ch * RB);
-      if (kBias) sr[b][t] = __builtin_amdgcn_raw_buffer_load_b32(rs, slane, ch * SB, 0);
-      else sr[b][t] = __builtin_amdgcn_raw_buffer_load_b16(rs, slane, ch * SB, 0);
+      const int ch = row0[t] * KG + 2 * kbA;
+      if (kBias) sn[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, so, ch * SB, 0);
+      else sn[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, so, ch * SB, 0);
+      if constexpr (!kQ8) cn[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, ch * RB, 0));
+    }
+  };
+  // Q8 codes of RING groups: a stage ahead, or (64-row tiles, for their registers) a group ahead.
+  Codes<F> wr[kQ8 ? RING : 1][kQ8 ? NT : 1];
+  auto load_w = [&](int gi, auto bc) {
+    if constexpr (kQ8) {
+      constexpr int b = decltype(bc)::value;
+      const int g = 2 * kbA + min(gi, n_grp - 1);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wr[b][t].load(rw, wlane, (row0[t] * KG + g) * RB);
     }
   };
 
@@ -170,7 +208,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   };
 
   f32x4 acc[NT][MB];
-  uint32_t bb[NT];  // fp16 bias of group slot kq of the pair of stages
+  uint32_t bb[NT];  // fp16 bias of group kq of the pair of stages
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     bb[t] = 0;
@@ -190,6 +228,23 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       __syncthreads();
     }
     load_x(s + 1, bn);
+    if constexpr (kQ8 && RING == 4) {
+      load_w(2 * s + 2, std::integral_constant<int, 2 - 2 * b>{});
+      load_w(2 * s + 3, std::integral_constant<int, 3 - 2 * b>{});
+    }
+    if constexpr (b == 0) {
+      // A pair of stages begins: its scales and codes are there, the next pair's are requested.
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        sv[t] = sn[t];
+        if constexpr (!kQ8) cv[t] = lane_transpose(cn[t]);
+        if (kBias) bb[t] = 2 * s + kq < n_grp ? sv[t] >> 16 : 0u;
+      }
+      load_pair((s >> 1) + 1);
+    }
+    u32x2 sc2[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) sc2[t] = lane_rows<b>(sv[t]);
     if (kBias) {
       // Sums of the stage's two groups per row, TPP threads each.
       constexpr int TPP = MB == 1 ? 8 : (MB == 2 ? 4 : 2);
@@ -223,19 +278,11 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       }
     }
     const f16* xa = &xs[b][l16 * kCStage];
-    auto group = [&](auto gc, auto gn) {
+    auto group = [&](auto gc) {
       constexpr int g = decltype(gc)::value;
       __builtin_amdgcn_sched_barrier(0);
-      load_w(2 * s + g + 1, gn);
-      if (kBias) {
-        // Slot 2 b + g of the pair of stages belongs to the lanes of quarter kq == 2 b + g; a pair's
-        // first group clears the others.
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const uint32_t bv = g == 1 && s == s_tail ? 0u : sr[g][t] >> 16;
-          bb[t] = kq == 2 * b + g ? bv : (b + g == 0 ? 0u : bb[t]);
-        }
-      }
+      constexpr int w = kQ8 ? (2 * b + g) % RING : 0;  // a pair starts at an even stage
+      if constexpr (kQ8 && RING == 2) load_w(2 * s + g + 1, std::integral_constant<int, 1 - g>{});
       f16x8 A[2][MB];
 #pragma unroll
       for (int c = 0; c < 2; ++c)
@@ -245,8 +292,11 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         __builtin_amdgcn_sched_barrier(0);
-        const f16x8 q0 = wr[g][t].operand(0), q1 = wr[g][t].operand(1);
-        const float sc = h2f(u16_as_h((uint16_t)sr[g][t]));
+        Codes<F> q;
+        if constexpr (kQ8) q = wr[w][t];
+        else q.w = cv[t][2 * b + g];
+        const f16x8 q0 = q.operand(0), q1 = q.operand(1);
+        const float sc = h2f(u16_as_h((uint16_t)sc2[t][g]));
         f32x4 d[MB];
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -259,9 +309,11 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
           for (int v = 0; v < 4; ++v) acc[t][mb][v] = __builtin_fmaf(sc, d[mb][v], acc[t][mb][v]);
       }
     };
-    group(B0{}, B1{});
-    group(B1{}, B0{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    group(B0{});
+    group(B1{});
+    // The next stage's x (requested first in this one) is in LDS; of the loads after it some may
+    // still be under way.
+    wait_loads<kQ8 || b == 0 ? NT : 0>();
     __syncthreads();
   };
   // The bias term of the pair of stages that holds stage s (after its barrier).
@@ -288,8 +340,10 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   if (kBias)
     for (int i = tid; i < TOK * 4; i += kCThreads) sx[0][i] = sx[kBias ? 1 : 0][i] = u32x4{0, 0, 0, 0};
   load_x(0, B0{});
+  load_pair(0);
   load_w(0, B0{});
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (RING == 4) load_w(1, B1{});
+  wait_loads<0>();
   __syncthreads();
   for (int s = 0;;) {
     stage(s, B0{}, B1{});
@@ -361,7 +415,8 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
     const int h = hb & 1;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int base = ((unit + t) * 16 * NB + (hb >> 1)) * kBlock;  // wave-uniform; rows past N read zeros
+      // Wave-uniform; tiles past the matrix read the last one, the last one's rows past it zeros.
+      const int base = (min(unit + t, a.n_units - 1) * 16 * NB + (hb >> 1)) * kBlock;
       cw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane + 8 * kq, base + 16 + 32 * h, 0));
       sw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane, base + 8 * h, 0));
       dw[b][t] = __builtin_amdgcn_raw_buffer_load_b32(rw, wlane, base + 80, 0);
@@ -512,7 +567,7 @@ struct CodesPlan {
 };
 // Row tile: the fewest row blocks of up to 64 rows, evenly filled.  Up to 32 rows the launch is
 // bound by the weights' stream: two tiles per wave, K split until three workgroups per CU are in
-// flight (12288 x 4096 Q8, 16 rows: one split 51 us, four 26, eight 24); more rows take four
+// flight (12288 x 4096 Q8, 16 rows: one split 51 us, four 26, eight 24, before the paired loads); more rows take four
 // tiles per wave (each x fragment read from LDS feeds four) and two workgroups per CU (64 rows: one split
 // 94 us, four 38).  Each split keeps two stages.
 CodesPlan codes_plan(int M, int KB, int n_units, int epi) {
@@ -616,15 +671,20 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
 // C ABI: products of several rows with a workspace for split K.
 // ---------------------------------------------------------------------------
 // The 2-bit GEMVs' own matrix-core launches take up to 16 rows each (fewer at large K, whose rows
-// fill LDS); this kernel takes over where they need four, or two of a large matrix (ternary,
-// 12288 x 4096: 16 rows in one launch 23.3 us against 22.3 here, 17 in two 28.7 / 23.2, 64 in four
-// 90.7 / 35.4; 4096 x 4096: 32 in two 13.6 / 16.4, 48 in three 20.2 / 20.9, 64 in four 26.4 / 24.1;
-// 4096 x 11008: six in one 11.5 / 17.4, eight in two 20.2 / 17.4; GGUF 4096 x 11008: eight in two
+// fill LDS); this kernel takes over where they need four, and for a large matrix (32 Mi weights)
+// where they need two, or one of ternary or affine codes with more than eight rows and a K that
+// splits well (us, ternary, 12288 x 4096: eight rows in one launch 13.3, ten 20.6 against 15.8 here,
+// sixteen 23.2 / 16.8, 17 in two 28.7 / 17.7, 64 in four 90.7 / 30.6; 32000 x 2048 affine: ten 17.8 / 18.7;
+// 4096 x 4096: 32 in two 13.6 / 15.2, 48 in three 20.2 / 18.9, 64 in four 26.4 / 22.5;
+// 4096 x 11008: six in one 11.5 / 14.6, eight in two 20.2 / 14.8; GGUF 4096 x 11008: eight in two
 // 16.2 / 16.8, twelve 17.8 / 17.2, sixteen in three 25.5 / 17.7, 64 in ten 87.5 / 31.9).
 static bool lowbit_rows_use_codes(int fmt, int M, int K, int N) {
-  const int per = fmt == kCodesQ2kGguf ? q2k_gguf_mfma_rows(K) : lowbit_mfma_rows(N, K);
+  const bool gguf = fmt == kCodesQ2kGguf;
+  const int per = gguf ? q2k_gguf_mfma_rows(K) : lowbit_mfma_rows(N, K);
   const int launches = per > 0 ? axm_ceil_div(M, per) : M;
-  return launches >= 4 || (launches >= 2 && M >= (fmt == kCodesQ2kGguf ? 12 : 5) && (size_t)N * K >= (size_t)32 << 20);
+  if (launches >= 4) return true;
+  if ((size_t)N * K < (size_t)32 << 20) return false;
+  return gguf ? launches >= 2 && M >= 12 : launches >= 2 || (M > 8 && K >= 4096);
 }
 
 // Whether M rows of a format go through this kernel (shapes and alignment apart).

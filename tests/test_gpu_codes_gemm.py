@@ -159,3 +159,18 @@ def test_wrappers_choose_the_same_result_on_both_sides(dev):
         for M in rows:
             got = fn(torch.from_numpy(x[:M]).to(dev), *packs).cpu().numpy().astype(np.float64)
             assert np.linalg.norm(got - ref[:M]) <= REL * np.linalg.norm(ref[:M])
+
+
+@pytest.mark.parametrize("fmt", ["ternary", "q2", "gguf"])
+def test_codes_gemm_few_rows_of_a_large_matrix(dev, fmt):
+    """2-bit row tiles of 16 and 32, taken where one GEMV launch no longer pays; N ends inside a tile."""
+    N, K = 8200, 4096
+    rng = np.random.default_rng(3)
+    packs, w = _packed(fmt, rng, N, K)
+    packs = [torch.from_numpy(a).to(dev) for a in packs]
+    x = rng.standard_normal((40, K)).astype(np.float16)
+    ref = x.astype(np.float32) @ w.astype(np.float32).T
+    for M in (9, 16, 17, 31, 40):
+        for ws in (True, False):
+            got = _run(fmt, torch.from_numpy(x[:M]).to(dev), packs, N, None, ws).cpu().numpy()
+            assert np.linalg.norm(got.astype(np.float32) - ref[:M]) <= REL * np.linalg.norm(ref[:M]), (M, ws)
