@@ -1,5 +1,5 @@
-// Several-row GEMM over row-major code matrices with a scale (and bias) per 64 columns --
-// Q8_G64, ternary and affine 2-bit -- on v_mfma_f32_16x16x32_f16, with exact code products:
+// Several-row GEMM over code matrices with a scale (and bias) per 64 columns -- row-major Q8_G64,
+// ternary and affine 2-bit, and the MARLIN Q4 tiles -- on v_mfma_f32_16x16x32_f16, with exact code products:
 //
 //   y[m][n] = sum_g s_ng (sum_k q_nk x_mk) + b_ng (sum_k x_mk)       (g: 64 columns)
 //
@@ -20,7 +20,8 @@
 //
 // Measured (us, graph of back-to-back calls, against the GEMVs of up to 4 / 16 rows a launch):
 // Q8 12288 x 4096, 16 rows 67 -> 21, 64 rows 244 -> 33.5, 1000 rows -> 177 (569 TFLOP/s); ternary 64
-// rows 91 -> 31, 1000 rows 150 (671).  (Scales and codes loaded group by group: 25, 40, 227; 35,
+// rows 91 -> 31, 1000 rows 150 (671); MARLIN, whose GEMV takes 4, 16 rows 98 -> 15.5, 64 rows 373 -> 30.5,
+// 1000 rows 5703 -> 186 (541).  (Scales and codes loaded group by group: 25, 40, 227; 35,
 // 202.)  Large launches are bound by the vector units: per group
 // and 16 x 16 tile four multiply-adds (16 cycles) and a share of the code expansion stand beside
 // 32 MFMA cycles.
@@ -83,6 +84,33 @@ struct Codes<kCodesQ8> {
     return __builtin_bit_cast(f16x8, o);
   }
 };
+// MARLIN tiles (q4_marlin.hip): a word of a row pair holds four columns 8 apart of both rows.
+// The pair's lanes load two of its four words of quarter kq each and swap halves (own_rows), which
+// leaves a lane word j with columns 32 j + 8 s + 2 kq (low half, nibble s) and + 1 (high half) of its row:
+// operand j is those eight in pairs, and x is staged in that order.
+template <>
+struct Codes<kCodesMarlin> {
+  static constexpr int kRowBytes64 = 32;
+  u32x2 w;
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    w = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+  }
+  __device__ __forceinline__ void own_rows(uint32_t sel) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[j], 0xB1, 0xF, 0xF, true);  // lane ^ 1
+      w[j] = __builtin_amdgcn_perm(other, w[j], sel);
+    }
+  }
+  __device__ __forceinline__ f16x8 operand(int c) const {
+    const uint32_t v = w[c], v8 = v >> 8;
+    const u32x4 u = {(v & 0x000F000Fu) | 0x64006400u, (v & 0x00F000F0u) | 0x54005400u,
+                     (v8 & 0x000F000Fu) | 0x64006400u, (v8 & 0x00F000F0u) | 0x54005400u};
+    const f16 lo = (f16)1024.f, hi = (f16)64.f;
+    const f16x8 m = {lo, lo, hi, hi, lo, lo, hi, hi};
+    return __builtin_bit_cast(f16x8, u) - m;
+  }
+};
 // Sixteen 2-bit fields, element i at bits 2 i.
 struct Codes2 {
   static constexpr int kRowBytes64 = 16;
@@ -125,8 +153,9 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   constexpr bool kBias = F != kCodesTernary;
   constexpr int TOK = 16 * MB;
   constexpr int UPW = kPair ? NT / 2 : NT;  // units per wave
-  constexpr bool kQ8 = F == kCodesQ8;
-  constexpr int RING = MB > 3 ? 2 : 4;
+  constexpr bool kMarlin = F == kCodesMarlin;
+  constexpr bool kRing = F == kCodesQ8 || kMarlin;  // codes requested by the group
+  constexpr int RING = F == kCodesQ8 && MB > 3 ? 2 : 4;
   __shared__ __align__(16) f16 xs[2][TOK * kCStage];
   // Group sums of four groups (a pair of stages) as bf16 parts (s0, s1, s2, s0, s1, s2, 0, 0).
   __shared__ __align__(16) u32x4 sx[kBias ? 2 : 1][kBias ? TOK * 4 : 1];
@@ -156,7 +185,13 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   // This lane's codes of tile 0, and the (wave-uniform) first row of tile t: an up tile starts
   // a.N rows after its gate tile.  Tiles past the matrix read the last one, the last one's rows
   // past it zeros; neither is stored.
-  const int wlane = l16 * KG * RB + kq * (RB / 4);
+  // (MARLIN: 256 code and 32 scale bytes per eight rows and group.)
+  const int tile8 = (l16 >> 3) * KG;
+  const int wlane = kMarlin ? tile8 * 256 + 8 * ((kq >> 1) * 16 + (l16 & 4) * 2 + (kq & 1) * 4 + (l16 & 1) * 2 +
+                                                 ((l16 >> 1) & 1))
+                            : l16 * KG * RB + kq * (RB / 4);
+  constexpr int GW = kMarlin ? 256 : RB, GS = kMarlin ? 32 : SB;  // bytes from group to group
+  const uint32_t row_sel = l16 & 1 ? 0x03020706u : 0x05040100u;   // Codes<kCodesMarlin>
   int row0[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) row0[t] = min(unit + t % UPW, a.n_units - 1) * 16 + (kPair && t >= UPW ? a.N : 0);
@@ -170,26 +205,28 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   // request touched 16 cache lines for 4 bytes each, and those requests, not bytes or latency,
   // bound the launch (Q8, 22016 x 4096, 75 rows: 87 us, 59 with constant scales).
   uint32_t sv[NT], sn[NT];
-  u32x4 cv[kQ8 ? 1 : NT], cn[kQ8 ? 1 : NT];
+  u32x4 cv[kRing ? 1 : NT], cn[kRing ? 1 : NT];
   auto load_pair = [&](int p) {
     const int g = min(4 * p + kq, n_grp - 1);  // past the split: its last group again
-    const int so = (l16 * KG + g) * SB, wo = (l16 * KG + g) * RB;
+    const int so = kMarlin ? tile8 * GS + (l16 & 7) * SB + g * GS : (l16 * KG + g) * SB;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int ch = row0[t] * KG + 2 * kbA;
-      if (kBias) sn[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, so, ch * SB, 0);
-      else sn[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, so, ch * SB, 0);
-      if constexpr (!kQ8) cn[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo, ch * RB, 0));
+      const int ch = row0[t] * KG * SB + 2 * kbA * GS;
+      if (kBias) sn[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, so, ch, 0);
+      else sn[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, so, ch, 0);
+      if constexpr (!kRing)
+        cn[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                              rw, (l16 * KG + g) * RB, (row0[t] * KG + 2 * kbA) * RB, 0));
     }
   };
-  // Q8 codes of RING groups: a stage ahead, or (64-row tiles, for their registers) a group ahead.
-  Codes<F> wr[kQ8 ? RING : 1][kQ8 ? NT : 1];
+  // Codes of RING groups: a stage ahead, or (Q8's 64-row tiles, for their registers) a group ahead.
+  Codes<F> wr[kRing ? RING : 1][kRing ? NT : 1];
   auto load_w = [&](int gi, auto bc) {
-    if constexpr (kQ8) {
+    if constexpr (kRing) {
       constexpr int b = decltype(bc)::value;
       const int g = 2 * kbA + min(gi, n_grp - 1);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wr[b][t].load(rw, wlane, (row0[t] * KG + g) * RB);
+      for (int t = 0; t < NT; ++t) wr[b][t].load(rw, wlane, row0[t] * KG * RB + g * GW);
     }
   };
 
@@ -198,13 +235,29 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
   const int xrow = 4 * wave + kq;
   const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  // MARLIN: a row per request, word s of piece (g, quarter, c) from word 32 g + 16 c + 4 s + quarter.
+  int xm[kMarlin ? 4 : 1];
+  if constexpr (kMarlin)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int r = 4 * wave + n, p = (lane >> 2) ^ r;
+      xm[n] = r * a.ldx * 2 + 4 * (32 * (p >> 3) + 16 * (p & 1) + 4 * (lane & 3) + ((p >> 1) & 3));
+    }
   auto load_x = [&](int s, auto bc) {
     constexpr int b = decltype(bc)::value;
     const int so = (kbA + min(s, n_st - 1)) * (kCStage * 2);
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
-                                               so + i * 32 * a.ldx, 0, 0);
+    for (int i = 0; i < MB; ++i) {
+      if constexpr (kMarlin) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave + n) * kCStage]), 4, xm[n],
+                                                   so + i * 32 * a.ldx, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
+                                                 so + i * 32 * a.ldx, 0, 0);
+      }
+    }
   };
 
   f32x4 acc[NT][MB];
@@ -228,7 +281,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       __syncthreads();
     }
     load_x(s + 1, bn);
-    if constexpr (kQ8 && RING == 4) {
+    if constexpr (kRing && RING == 4) {
       load_w(2 * s + 2, std::integral_constant<int, 2 - 2 * b>{});
       load_w(2 * s + 3, std::integral_constant<int, 3 - 2 * b>{});
     }
@@ -237,7 +290,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         sv[t] = sn[t];
-        if constexpr (!kQ8) cv[t] = lane_transpose(cn[t]);
+        if constexpr (!kRing) cv[t] = lane_transpose(cn[t]);
         if (kBias) bb[t] = 2 * s + kq < n_grp ? sv[t] >> 16 : 0u;
       }
       load_pair((s >> 1) + 1);
@@ -281,8 +334,8 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
     auto group = [&](auto gc) {
       constexpr int g = decltype(gc)::value;
       __builtin_amdgcn_sched_barrier(0);
-      constexpr int w = kQ8 ? (2 * b + g) % RING : 0;  // a pair starts at an even stage
-      if constexpr (kQ8 && RING == 2) load_w(2 * s + g + 1, std::integral_constant<int, 1 - g>{});
+      constexpr int w = kRing ? (2 * b + g) % RING : 0;  // a pair starts at an even stage
+      if constexpr (kRing && RING == 2) load_w(2 * s + g + 1, std::integral_constant<int, 1 - g>{});
       f16x8 A[2][MB];
 #pragma unroll
       for (int c = 0; c < 2; ++c)
@@ -293,8 +346,9 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       for (int t = 0; t < NT; ++t) {
         __builtin_amdgcn_sched_barrier(0);
         Codes<F> q;
-        if constexpr (kQ8) q = wr[w][t];
+        if constexpr (kRing) q = wr[w][t];
         else q.w = cv[t][2 * b + g];
+        if constexpr (kMarlin) q.own_rows(row_sel);
         const f16x8 q0 = q.operand(0), q1 = q.operand(1);
         const float sc = h2f(u16_as_h((uint16_t)sc2[t][g]));
         f32x4 d[MB];
@@ -313,7 +367,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
     group(B1{});
     // The next stage's x (requested first in this one) is in LDS; of the loads after it some may
     // still be under way.
-    wait_loads<kQ8 || b == 0 ? NT : 0>();
+    wait_loads<kRing || b == 0 ? NT : 0>();
     __syncthreads();
   };
   // The bias term of the pair of stages that holds stage s (after its barrier).
@@ -619,12 +673,22 @@ void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t
 
 }  // namespace
 
+// Code / scale bytes of a matrix.
+static size_t codes_bytes(int fmt, int rows, int K) {
+  if (fmt == kCodesMarlin) return (size_t)((rows + 7) / 8) * (K / 64) * 256;
+  return (size_t)rows * (fmt == kCodesQ2kGguf ? K / 256 * 84 : fmt == kCodesQ8 ? K : K / 4);
+}
+static size_t scale_bytes(int fmt, int rows, int K) {
+  const size_t r = fmt == kCodesMarlin ? (size_t)(rows + 7) / 8 * 8 : rows;
+  return r * (K / 64) * (fmt == kCodesTernary ? 2 : 4);
+}
+
 bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int rows, int fmt) {
   if (fmt == kCodesQ2kGguf)
     return K > 0 && K % 256 == 0 && K <= 16384 && (size_t)rows * (K / 256) * 84 < (size_t)0x7FFFFFF0 &&
            ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 3) == 0;
-  const size_t code_bytes = (size_t)rows * K / (fmt == kCodesQ8 ? 1 : 4);
-  const uintptr_t wa = fmt == kCodesQ8 ? 15 : 3, sa = fmt == kCodesTernary ? 1 : 3;
+  const size_t code_bytes = codes_bytes(fmt, rows, K);
+  const uintptr_t wa = fmt == kCodesQ8 ? 15 : fmt == kCodesMarlin ? 7 : 3, sa = fmt == kCodesTernary ? 1 : 3;
   return K > 0 && K % 64 == 0 && K <= 32768 && code_bytes < (size_t)0x7FFFFFF0 && ((uintptr_t)x & 15) == 0 &&
          ((uintptr_t)w & wa) == 0 && ((uintptr_t)sb & sa) == 0;
 }
@@ -655,11 +719,11 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
   else if (ws_bytes < p.splits * one) p.splits = (int)(ws_bytes / one);
   a.kb_per_split = axm_ceil_div(a.KB, p.splits);
   p.splits = axm_ceil_div(a.KB, a.kb_per_split);
-  a.w16_bytes = fmt == kCodesQ2kGguf ? (size_t)rows * (a.K / 256) * 84
-                                    : (size_t)rows * a.K / (fmt == kCodesQ8 ? 1 : 4);
-  a.sb16_bytes = (size_t)rows * (a.K / 64) * (fmt == kCodesTernary ? 2 : 4);
+  a.w16_bytes = codes_bytes(fmt, rows, a.K);
+  a.sb16_bytes = scale_bytes(fmt, rows, a.K);
   if (fmt == kCodesQ2kGguf) q2k_launch_shape(a, M, p, s);
   else if (fmt == kCodesQ2) codes_launch_shape<kCodesQ2, Q4_EPI_STORE>(a, M, p, s);
+  else if (fmt == kCodesMarlin) codes_launch_shape<kCodesMarlin, Q4_EPI_STORE>(a, M, p, s);
   else if (fmt == kCodesTernary) codes_launch_shape<kCodesTernary, Q4_EPI_STORE>(a, M, p, s);
   else if (epi == Q4_EPI_STORE) codes_launch_shape<kCodesQ8, Q4_EPI_STORE>(a, M, p, s);
   else if (epi == Q4_EPI_RESID) codes_launch_shape<kCodesQ8, Q4_EPI_RESID>(a, M, p, s);
@@ -689,11 +753,12 @@ static bool lowbit_rows_use_codes(int fmt, int M, int K, int N) {
 
 // Whether M rows of a format go through this kernel (shapes and alignment apart).
 static bool rows_use_codes(int fmt, int M, int K, int N) {
+  if (fmt == kCodesMarlin) return marlin_rows_use_codes(M, K, N);
   return fmt == kCodesQ8 ? M >= kCodesQ8MinRows : M > 4 && lowbit_rows_use_codes(fmt, M, K, N);
 }
 
 extern "C" size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N) {
-  if (format < kCodesQ8 || format > kCodesQ2kGguf || M <= 0 || K <= 0 || N <= 0) return 0;
+  if (format < kCodesQ8 || format > kCodesMarlin || M <= 0 || K <= 0 || N <= 0) return 0;
   return rows_use_codes(format, M, K, N) ? codes_gemm_ws_bytes(M, K, N, Q4_EPI_STORE) : 0;
 }
 
@@ -709,7 +774,7 @@ static int qmm_codes(int fmt, const char* who, const void* x, const void* w, con
   a.y = (f16*)y;
   a.ldy = N;
   a.bias = (const f16*)bias;
-  a.bias_f32 = fmt != kCodesQ8;  // as the formats' GEMVs
+  a.bias_f32 = fmt != kCodesQ8 && fmt != kCodesMarlin;  // as the formats' GEMVs
   const int rc = codes_gemm_launch(fmt, a, M, Q4_EPI_STORE, (float*)ws, ws_bytes, s);
   if (rc) return rc;
   AXM_LAUNCH_CHECK(who);
@@ -722,6 +787,15 @@ extern "C" int axm_qmm_q8_g64(const void* x, const void* w_packed, const void* s
     return axm_qmv_q8_g64(x, w_packed, sb, bias, y, M, K, N, stream);
   AXM_CHECK_ARG(w_packed && sb && x && y && N > 0, -1, "qmm_q8_g64: bad arguments");
   return qmm_codes(kCodesQ8, "qmm_q8_g64", x, w_packed, sb, bias, y, M, K, N, workspace, workspace_bytes,
+                   (hipStream_t)stream);
+}
+
+extern "C" int axm_qmm_q4_marlin(const void* x, const void* w_marlin, const void* sb_marlin, const void* bias, void* y,
+                                 int M, int K, int N, void* workspace, size_t workspace_bytes, void* stream) {
+  if (N <= 0 || !rows_use_codes(kCodesMarlin, M, K, N) || !codes_gemm_takes(x, w_marlin, sb_marlin, K, N, kCodesMarlin))
+    return axm_qmv_q4_marlin(x, w_marlin, sb_marlin, bias, y, M, K, N, stream);
+  AXM_CHECK_ARG(w_marlin && sb_marlin && x && y, -1, "qmm_q4_marlin: bad arguments");
+  return qmm_codes(kCodesMarlin, "qmm_q4_marlin", x, w_marlin, sb_marlin, bias, y, M, K, N, workspace, workspace_bytes,
                    (hipStream_t)stream);
 }
 

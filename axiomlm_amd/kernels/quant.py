@@ -155,9 +155,16 @@ def qmv_q4_marlin(x, w_marlin, sb_marlin, out_features: int | None = None, bias=
     b = None
     if bias is not None:
         b = bias.to(device=x.device, dtype=torch.float16).contiguous()
-    _lib.check(_lib.lib().axm_qmv_q4_marlin(_lib.ptr(xc), _lib.ptr(w_marlin.contiguous()),
+    if M == 1 or (M <= 4 and N * K < 32 << 20):  # the GEMV
+        _lib.check(_lib.lib().axm_qmv_q4_marlin(_lib.ptr(xc), _lib.ptr(w_marlin.contiguous()),
+                                                _lib.ptr(sb_marlin.contiguous()), _lib.ptr(b), _lib.ptr(y), M, K, N,
+                                                _lib.stream_of(x.device)),
+                   "qmv_q4_marlin")
+        return y
+    ws, n = _codes_workspace(4, M, K, N, x.device)
+    _lib.check(_lib.lib().axm_qmm_q4_marlin(_lib.ptr(xc), _lib.ptr(w_marlin.contiguous()),
                                             _lib.ptr(sb_marlin.contiguous()), _lib.ptr(b), _lib.ptr(y), M, K, N,
-                                            _lib.stream_of(x.device)),
+                                            _lib.ptr(ws), n, _lib.stream_of(x.device)),
                "qmv_q4_marlin")
     return y
 
@@ -317,7 +324,7 @@ def dequant_q8_rows(indices, w_packed, scales_biases) -> torch.Tensor:
 
 
 def _codes_workspace(fmt: int, M: int, K: int, N: int, device):
-    """Workspace of the several-row products (0 Q8_G64, 1 affine 2-bit, 2 ternary, 3 GGUF Q2_K)."""
+    """Workspace of the several-row products (0 Q8_G64, 1 affine 2-bit, 2 ternary, 3 GGUF Q2_K, 4 MARLIN)."""
     n = _lib.lib().axm_qmm_codes_workspace_bytes(fmt, M, K, N)
     return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
 

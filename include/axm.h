@@ -127,10 +127,13 @@ int axm_qmv_q2_k(const void* x, const void* w_packed, const void* scales_biases,
 /* The same products for several rows: from a few rows on one matrix-core launch for all of them
  * (exact code products, fp32 sums), with K split across workgroups as far as the workspace
  * (axm_qmm_codes_workspace_bytes for the preferred split; NULL / 0 is allowed) lets it; fewer
- * rows as the qmv entries.  Replaces qmm_q8_g64_mps, qmm_ternary_mps, qmm_q2_k_mps. */
-size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N); /* 0: Q8_G64, 1: affine 2-bit, 2: ternary, 3: GGUF */
+ * rows as the qmv entries.  Replaces qmm_q4_marlin_mps, qmm_q8_g64_mps, qmm_ternary_mps, qmm_q2_k_mps. */
+size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N); /* 0: Q8_G64, 1: affine 2-bit, 2: ternary, 3: GGUF,
+                                                                              4: MARLIN */
 int axm_qmm_q8_g64(const void* x, const void* w_packed, const void* sb, const void* bias, void* y, int M, int K, int N,
                    void* workspace, size_t workspace_bytes, void* stream);
+int axm_qmm_q4_marlin(const void* x, const void* w_marlin, const void* sb_marlin, const void* bias, void* y, int M,
+                      int K, int N, void* workspace, size_t workspace_bytes, void* stream);
 int axm_qmm_ternary(const void* x, const void* w_packed, const void* scales, const void* bias, void* y, int M, int K,
                     int N, void* workspace, size_t workspace_bytes, void* stream);
 int axm_qmm_q2_k(const void* x, const void* w_packed, const void* scales_biases, const void* bias, void* y, int M, int K,

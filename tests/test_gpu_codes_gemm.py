@@ -1,4 +1,5 @@
-"""Several-row GEMM over Q8_G64, ternary and affine 2-bit codes against the float64 product of the decoded codes.
+"""Several-row GEMM over Q8_G64, MARLIN Q4, ternary, affine and GGUF 2-bit codes against the float64 product of the
+decoded codes.
 
 Code products are exact and sums fp32, so the result is the float64 one to the fp16 rounding of the output: 2^-11 of
 each value at most, plus fp32 sums whose error (2^-24 of the sum of magnitudes per add) matters only where a row's
@@ -14,6 +15,13 @@ pytestmark = pytest.mark.gpu
 REL = 1.05 * 2.0 ** -11
 
 
+def _decode_marlin(p, s, K):
+    """float64 rows of the 8-row tiles, padding rows included."""
+    q = fm.unpack_marlin_codes(p).astype(np.float64).reshape(-1, K // 64, 64)
+    sb = s.transpose(0, 2, 1, 3).reshape(-1, K // 64, 2).astype(np.float64)
+    return (q * sb[..., 0:1] + sb[..., 1:2]).reshape(-1, K)
+
+
 def _packed(fmt, rng, N, K):
     """(device arrays, float64 weights)"""
     w = (rng.standard_normal((N, K)) * 0.02).astype(np.float16)
@@ -21,6 +29,9 @@ def _packed(fmt, rng, N, K):
         p, s = fm.pack_linear_q8_g64(w)
         q = p.reshape(N, K // 64, 64).astype(np.float64)
         return (p.view(np.int32).reshape(N, K // 4), s), (q * s[..., 0:1] + s[..., 1:2].astype(np.float64)).reshape(N, K)
+    if fmt == "marlin":
+        p, s = fm.pack_linear_q4_marlin(w, clip_search=False)
+        return (p, s), _decode_marlin(p, s, K)[:N]
     if fmt == "ternary":
         p, s = fm.pack_linear_ternary(w)
         q = fm.ternary_decode_bytes(p).reshape(N, K // 64, 64).astype(np.float64)
@@ -43,10 +54,11 @@ def _run(fmt, x, packs, N, bias=None, ws=True):
 
     L = _lib.lib()
     M, K = x.shape
-    fn = {"q8": L.axm_qmm_q8_g64, "ternary": L.axm_qmm_ternary, "q2": L.axm_qmm_q2_k, "gguf": L.axm_qmm_q2_k_gguf}[fmt]
+    fn = {"q8": L.axm_qmm_q8_g64, "marlin": L.axm_qmm_q4_marlin, "ternary": L.axm_qmm_ternary, "q2": L.axm_qmm_q2_k,
+          "gguf": L.axm_qmm_q2_k_gguf}[fmt]
     weights = [_lib.ptr(p) for p in (packs[:1] if fmt == "gguf" else packs)]
     y = torch.empty((M, N), dtype=torch.float16, device=x.device)
-    n = L.axm_qmm_codes_workspace_bytes({"q8": 0, "q2": 1, "ternary": 2, "gguf": 3}[fmt], M, K, N) if ws else 0
+    n = L.axm_qmm_codes_workspace_bytes({"q8": 0, "q2": 1, "ternary": 2, "gguf": 3, "marlin": 4}[fmt], M, K, N) if ws else 0
     buf = torch.empty(max(n, 1), dtype=torch.uint8, device=x.device)
     _lib.check(fn(_lib.ptr(x), *weights, _lib.ptr(bias), _lib.ptr(y), M, K, N,
                   _lib.ptr(buf) if n else None, n, _lib.stream_of(x.device)), fmt)
@@ -55,15 +67,15 @@ def _run(fmt, x, packs, N, bias=None, ws=True):
 
 # Row tiles of 16 - 64 with remainders, several row blocks, weight tiles past N, one and two stages, odd and even
 # counts, half a stage, split and unsplit K; 2-bit sizes beyond what their GEMV launches take.
-SHAPES = [(5, 16, 64), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96, 8192), (70, 130, 320),
+SHAPES = [(5, 16, 64), (7, 24, 192), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96, 8192), (70, 130, 320),
           (129, 2056, 1024), (17, 40, 192)]
 
 
-@pytest.mark.parametrize("fmt", ["q8", "ternary", "q2", "gguf"])
+@pytest.mark.parametrize("fmt", ["q8", "marlin", "ternary", "q2", "gguf"])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("ws", [True, False])
 def test_codes_gemm_matches_float64(dev, fmt, M, N, K, ws):
-    if fmt != "q8":
+    if fmt not in ("q8", "marlin"):
         M += 64  # four launches of 16 rows and more
     if fmt == "gguf":
         K = (K + 255) // 256 * 256
@@ -110,7 +122,7 @@ def test_codes_gemm_bias_joins_the_fp32_sum(dev, fmt, N, ws):
     assert np.linalg.norm(got - want) <= bound
 
 
-@pytest.mark.parametrize("fmt", ["q8", "q2", "gguf"])
+@pytest.mark.parametrize("fmt", ["q8", "marlin", "q2", "gguf"])
 def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
     """Group sums beyond the fp16 range and activations near its bottom keep 24 bits in the bias term."""
     rng = np.random.default_rng(1)
@@ -133,9 +145,12 @@ def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
             packs[1] = (packs[1].double() * 2.0 ** -6).half()
             s = packs[1].cpu().numpy().astype(np.float64)
             p = packs[0].cpu().numpy()
-            codes = (p.view(np.uint8).reshape(N, K // 64, 64) if fmt == "q8" else
-                     ((p[..., None] >> (2 * np.arange(4))) & 3).reshape(N, K // 64, 64)).astype(np.float64)
-            wn = (codes * s[..., 0:1] + s[..., 1:2]).reshape(N, K)
+            if fmt == "marlin":
+                wn = _decode_marlin(p, s, K)
+            else:
+                codes = (p.view(np.uint8).reshape(N, K // 64, 64) if fmt == "q8" else
+                         ((p[..., None] >> (2 * np.arange(4))) & 3).reshape(N, K // 64, 64)).astype(np.float64)
+                wn = (codes * s[..., 0:1] + s[..., 1:2]).reshape(N, K)
         ref = x.astype(np.float64) @ wn.T
         got = _run(fmt, torch.from_numpy(x).to(dev), packs, N).cpu().numpy().astype(np.float64)
         # fp16 results: half a unit of the last place, which near the bottom of the range is 2^-25
@@ -147,14 +162,16 @@ def test_codes_gemm_bias_term_over_the_fp16_range(dev, fmt):
 
 def test_wrappers_choose_the_same_result_on_both_sides(dev):
     """The Python products just below and above the rows at which the launch changes."""
-    from axiomlm_amd.kernels import qmv_q2_k, qmv_q8_g64, qmv_ternary
+    from axiomlm_amd.kernels import qmv_q2_k, qmv_q4_marlin, qmv_q8_g64, qmv_ternary
 
     rng = np.random.default_rng(5)
     for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("ternary", qmv_ternary, (48, 49), 96, 320),
-                                ("q2", qmv_q2_k, (48, 49), 96, 320), ("ternary", qmv_ternary, (16, 17), 8192, 4096)):
+                                ("q2", qmv_q2_k, (48, 49), 96, 320), ("ternary", qmv_ternary, (8, 9), 8192, 4096),
+                                ("marlin", qmv_q4_marlin, (4, 5), 96, 320),
+                                ("marlin", qmv_q4_marlin, (1, 2, 4), 8192, 4096)):
         packs, w = _packed(fmt, rng, N, K)
         packs = [torch.from_numpy(a).to(dev) for a in packs]
-        x = rng.standard_normal((rows[1], K)).astype(np.float16)
+        x = rng.standard_normal((rows[-1], K)).astype(np.float16)
         ref = x.astype(np.float64) @ w.T
         for M in rows:
             got = fn(torch.from_numpy(x[:M]).to(dev), *packs).cpu().numpy().astype(np.float64)
