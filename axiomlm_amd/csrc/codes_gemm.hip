@@ -19,10 +19,10 @@
 // codes two stages at a time (load_pair).
 //
 // Measured (us, graph of back-to-back calls, against the GEMVs of up to 4 / 16 rows a launch):
-// Q8 12288 x 4096, 16 rows 67 -> 21, 64 rows 244 -> 33.5, 1000 rows -> 177 (569 TFLOP/s); ternary 64
-// rows 91 -> 31, 1000 rows 150 (671); MARLIN, whose GEMV takes 4, 16 rows 98 -> 15.5, 64 rows 373 -> 30.5,
-// 1000 rows 5703 -> 186 (541).  (Scales and codes loaded group by group: 25, 40, 227; 35,
-// 202.)  Large launches are bound by the vector units: per group
+// Q8 12288 x 4096, 16 rows 67 -> 21, 64 rows 244 -> 28, 1000 rows -> 177 (569 TFLOP/s); ternary 64
+// rows 91 -> 25.5, 1000 rows 150 (671); MARLIN, whose GEMV takes 4, 16 rows 98 -> 15.5, 64 rows 373 -> 27.5,
+// 1000 rows 5703 -> 186 (541).  (Scales and codes loaded group by group: Q8 16 rows 25, 1000 rows
+// 227; ternary 1000 rows 202.)  Large launches are bound by the vector units: per group
 // and 16 x 16 tile four multiply-adds (16 cycles) and a share of the code expansion stand beside
 // 32 MFMA cycles.
 #include <type_traits>
@@ -619,22 +619,36 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
 struct CodesPlan {
   int mb, nt, splits;
 };
-// Row tile: the fewest row blocks of up to 64 rows, evenly filled.  Up to 32 rows the launch is
-// bound by the weights' stream: two tiles per wave, K split until three workgroups per CU are in
-// flight (12288 x 4096 Q8, 16 rows: one split 51 us, four 26, eight 24, before the paired loads); more rows take four
-// tiles per wave (each x fragment read from LDS feeds four) and two workgroups per CU (64 rows: one split
-// 94 us, four 38).  Each split keeps two stages.
+// Row tile: the fewest row blocks of up to 64 rows, evenly filled.  Weight tiles per wave (two, or
+// four with 64 rows; 48 rows with four were always slower) and K splits by the time each choice is expected to take: a round of the
+// workgroups that fit a CU (four of up to 32 rows, three with two tiles per wave, two with four)
+// (or part of one past the first) costs kStage[0] us per stage, each workgroup of a CU kStage[1]; partial tiles are written
+// and read back at about 5 TB/s.  Fitted to a sweep of 1-16 splits and both tile counts over 8-1000
+// rows, six matrices (1024-22016 rows) and five formats: the choice is within 1-2 % of the sweep's
+// best on average and 14 % at worst but for one (27 %), four tiles per wave with two workgroups a CU
+// had been 15-35 % off on average (Q8 4096 x 4096, 40 rows: four tiles 20.3 us, two from eight splits
+// 15.1; 12288 x 4096, 75 rows 41.0 / 34.7; 1000 rows: four tiles unsplit 155, two 167).
 CodesPlan codes_plan(int M, int KB, int n_units, int epi) {
-  CodesPlan p;
-  const int nb = axm_ceil_div(M, 64);
-  p.mb = axm_ceil_div(M, 16 * nb);
-  p.nt = p.mb <= 2 ? 2 : 4;
-  const int upw = epi == Q4_EPI_SWIGLU ? p.nt / 2 : p.nt;
-  const int tiles = axm_ceil_div(n_units, kCWaves * upw) * axm_ceil_div(M, 16 * p.mb);
-  int s = (p.mb <= 2 ? 3 : 2) * axm_num_cus() / tiles;
-  s = s > KB / 2 ? KB / 2 : s;
-  p.splits = s < 1 ? 1 : (s > 16 ? 16 : s);
-  return p;
+  static const float kStage[5][2] = {{.18f, .41f}, {.26f, .51f}, {.38f, .51f}, {.53f, .54f},  // 16-64 rows, two tiles
+                                     {1.f, .9f}};                                             // 64, four
+  const int nb = axm_ceil_div(M, 64), mb = axm_ceil_div(M, 16 * nb), cus = axm_num_cus();
+  const float part_us = 1.5e-6f * (float)M * (float)n_units * (epi == Q4_EPI_SWIGLU ? 32.f : 16.f);
+  CodesPlan best{mb, 2, 1};
+  float best_us = 1e30f;
+  for (int nt = 2; nt <= (mb == 4 ? 4 : 2); nt += 2) {
+    const float* st = kStage[nt == 2 ? mb - 1 : 4];
+    const int per_cu = mb <= 2 ? 4 : nt == 2 ? 3 : 2;
+    const int tiles = axm_ceil_div(n_units, kCWaves * (epi == Q4_EPI_SWIGLU ? nt / 2 : nt)) * axm_ceil_div(M, 16 * mb);
+    for (int s = 1; s <= 16 && (s == 1 || s <= KB / 2); ++s) {
+      const int stages = axm_ceil_div(KB, s), splits = axm_ceil_div(KB, stages);
+      const int load = axm_ceil_div(tiles * splits, cus);  // workgroups per CU
+      const float rounds = load > per_cu ? (float)load / (float)per_cu : 1.f;
+      const float us = (float)stages * (st[0] * rounds + st[1] * (float)load) +
+                       (splits == 1 ? 0.f : 1.3f + (float)splits * part_us);
+      if (us < best_us) best_us = us, best = {mb, nt, splits};
+    }
+  }
+  return best;
 }
 
 template <int F, int EPI, int MB, int NT>
@@ -656,8 +670,8 @@ void q2k_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t s
   switch (p.mb) {
     case 1: return q2k_launch<1, 2>(a, M, p.splits, s);
     case 2: return q2k_launch<2, 2>(a, M, p.splits, s);
-    case 3: return q2k_launch<3, 4>(a, M, p.splits, s);
-    default: return q2k_launch<4, 4>(a, M, p.splits, s);
+    case 3: return q2k_launch<3, 2>(a, M, p.splits, s);
+    default: return p.nt == 2 ? q2k_launch<4, 2>(a, M, p.splits, s) : q2k_launch<4, 4>(a, M, p.splits, s);
   }
 }
 
@@ -666,8 +680,8 @@ void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t
   switch (p.mb) {
     case 1: return codes_launch<F, EPI, 1, 2>(a, M, p.splits, s);
     case 2: return codes_launch<F, EPI, 2, 2>(a, M, p.splits, s);
-    case 3: return codes_launch<F, EPI, 3, 4>(a, M, p.splits, s);
-    default: return codes_launch<F, EPI, 4, 4>(a, M, p.splits, s);
+    case 3: return codes_launch<F, EPI, 3, 2>(a, M, p.splits, s);
+    default: return p.nt == 2 ? codes_launch<F, EPI, 4, 2>(a, M, p.splits, s) : codes_launch<F, EPI, 4, 4>(a, M, p.splits, s);
   }
 }
 
@@ -738,15 +752,16 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
 // fill LDS); this kernel takes over where they need four, and for a large matrix (32 Mi weights)
 // where they need two, or one of ternary or affine codes with more than eight rows and a K that
 // splits well (us, ternary, 12288 x 4096: eight rows in one launch 13.3, ten 20.6 against 15.8 here,
-// sixteen 23.2 / 16.8, 17 in two 28.7 / 17.7, 64 in four 90.7 / 30.6; 32000 x 2048 affine: ten 17.8 / 18.7;
-// 4096 x 4096: 32 in two 13.6 / 15.2, 48 in three 20.2 / 18.9, 64 in four 26.4 / 22.5;
-// 4096 x 11008: six in one 11.5 / 14.6, eight in two 20.2 / 14.8; GGUF 4096 x 11008: eight in two
-// 16.2 / 16.8, twelve 17.8 / 17.2, sixteen in three 25.5 / 17.7, 64 in ten 87.5 / 31.9).
+// sixteen 23.2 / 16.4, 17 in two 28.7 / 17.7, 64 in four 90.7 / 25.7; 32000 x 2048 affine: ten 17.8 / 18.7;
+// 4096 x 4096: 32 in two 13.6 / 14, 40 in three 19.1 / 13.2, 64 in four 26.4 / 16.2;
+// 4096 x 11008: six in one 11.5 / 14.4, eight in two 20.2 / 14.9; GGUF 4096 x 11008: eight in two
+// 16.2 / 16.5, twelve 17.8 / 16.9, sixteen in three 25.5 / 17, 64 in ten 87.5 / 30; 4096 x 4096: 48 in
+// three 19.3 / 16.4).
 static bool lowbit_rows_use_codes(int fmt, int M, int K, int N) {
   const bool gguf = fmt == kCodesQ2kGguf;
   const int per = gguf ? q2k_gguf_mfma_rows(K) : lowbit_mfma_rows(N, K);
   const int launches = per > 0 ? axm_ceil_div(M, per) : M;
-  if (launches >= 4) return true;
+  if (launches >= 3) return true;
   if ((size_t)N * K < (size_t)32 << 20) return false;
   return gguf ? launches >= 2 && M >= 12 : launches >= 2 || (M > 8 && K >= 4096);
 }

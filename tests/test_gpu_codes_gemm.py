@@ -65,10 +65,11 @@ def _run(fmt, x, packs, N, bias=None, ws=True):
     return y
 
 
-# Row tiles of 16 - 64 with remainders, several row blocks, weight tiles past N, one and two stages, odd and even
+# Row tiles of 16 - 64 with remainders, two and four weight tiles per wave (the last: four), several row blocks, weight tiles past N, one and two stages, odd and even
 # counts, half a stage, split and unsplit K; 2-bit sizes beyond what their GEMV launches take.
 SHAPES = [(5, 16, 64), (7, 24, 192), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96, 8192), (70, 130, 320),
-          (129, 2056, 1024), (17, 40, 192)]
+          (129, 2056, 1024), (17, 40, 192),
+          (930, 12280, 128)]
 
 
 @pytest.mark.parametrize("fmt", ["q8", "marlin", "ternary", "q2", "gguf"])
@@ -165,8 +166,8 @@ def test_wrappers_choose_the_same_result_on_both_sides(dev):
     from axiomlm_amd.kernels import qmv_q2_k, qmv_q4_marlin, qmv_q8_g64, qmv_ternary
 
     rng = np.random.default_rng(5)
-    for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("ternary", qmv_ternary, (48, 49), 96, 320),
-                                ("q2", qmv_q2_k, (48, 49), 96, 320), ("ternary", qmv_ternary, (8, 9), 8192, 4096),
+    for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("ternary", qmv_ternary, (32, 33), 96, 320),
+                                ("q2", qmv_q2_k, (32, 33), 96, 320), ("ternary", qmv_ternary, (8, 9), 8192, 4096),
                                 ("marlin", qmv_q4_marlin, (4, 5), 96, 320),
                                 ("marlin", qmv_q4_marlin, (1, 2, 4), 8192, 4096)):
         packs, w = _packed(fmt, rng, N, K)
