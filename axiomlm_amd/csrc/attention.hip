@@ -1072,7 +1072,7 @@ int attn_flash_splits(int B, int Hq, int Hkv, int hd, int kv_dtype, int active_l
 }
 
 // A decode step of one sequence.  Grouped-query heads take the matrix-core kernel at every
-// length, with splits of about 128 keys up to one workgroup per CU: the vector kernel with eight
+// length, from 32 keys on with splits of about 128 keys up to one workgroup per CU: the vector kernel with eight
 // splits per head set fills 64 CUs at 8 KV heads and multiplies every key once per query head (us per
 // layer of a 7B-shape step with 32 / 8 heads and an FP8 cache, vector kernel / four / eight / 32
 // splits here: 100 keys 46.1 / 43.5 / 43.6 / 44.6, 1000 keys 48.9 / 44.9 / 44.1 / 44.8, 4000 keys
@@ -1084,8 +1084,8 @@ int attn_step_splits(int Hq, int Hkv, int active_len) {
   const int n_rep = Hq / Hkv;
   const int fill = axm_ceil_div(axm_num_cus(), Hkv);  // one workgroup per CU
   if (n_rep >= 2 && n_rep <= 16) {
-    int splits = 4;
-    while (splits < fill && splits < 64 && 128 * splits < active_len) splits <<= 1;
+    int splits = active_len < 32 ? 1 : 4;  // (7 keys, FP16 cache, four layers: one 164 us, four 175)
+    while (splits > 1 && splits < fill && splits < 64 && 128 * splits < active_len) splits <<= 1;
     return splits;
   }
   return kAttnMaxParts * Hkv <= axm_num_cus() / 2 && active_len >= 1000 * kAttnMaxParts ? (fill < 32 ? fill : 32) : 0;
