@@ -1,5 +1,6 @@
 // Several-row GEMM over code matrices with a scale (and bias) per 64 columns -- row-major Q8_G64,
-// ternary and affine 2-bit, and the MARLIN Q4 tiles -- on v_mfma_f32_16x16x32_f16, with exact code products:
+// ternary and affine 2-bit, and the MARLIN Q4 tiles -- on v_mfma_f32_16x16x32_f16, with exact code
+// products (and over plain fp16 rows, without the scales):
 //
 //   y[m][n] = sum_g s_ng (sum_k q_nk x_mk) + b_ng (sum_k x_mk)       (g: 64 columns)
 //
@@ -111,6 +112,18 @@ struct Codes<kCodesMarlin> {
     return __builtin_bit_cast(f16x8, u) - m;
   }
 };
+// Plain fp16 weights: a group's MFMAs add to the accumulator directly.
+template <>
+struct Codes<kCodesF16> {
+  static constexpr int kRowBytes64 = 128;
+  u32x4 w[2];
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      w[c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * c, soff, 0));
+  }
+  __device__ __forceinline__ f16x8 operand(int c) const { return __builtin_bit_cast(f16x8, w[c]); }
+};
 // Sixteen 2-bit fields, element i at bits 2 i.
 struct Codes2 {
   static constexpr int kRowBytes64 = 16;
@@ -150,12 +163,13 @@ __device__ __forceinline__ void wait_loads() {
 template <int F, int EPI, int MB, int NT>
 __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
   constexpr bool kPair = EPI == Q4_EPI_SWIGLU;
-  constexpr bool kBias = F != kCodesTernary;
+  constexpr bool kPlain = F == kCodesF16;
+  constexpr bool kBias = F != kCodesTernary && !kPlain;
   constexpr int TOK = 16 * MB;
   constexpr int UPW = kPair ? NT / 2 : NT;  // units per wave
   constexpr bool kMarlin = F == kCodesMarlin;
-  constexpr bool kRing = F == kCodesQ8 || kMarlin;  // codes requested by the group
-  constexpr int RING = F == kCodesQ8 && MB > 3 ? 2 : 4;
+  constexpr bool kRing = F == kCodesQ8 || kMarlin || kPlain;  // codes requested by the group
+  constexpr int RING = (F == kCodesQ8 && MB > 3) || (kPlain && NT > 2) ? 2 : 4;
   __shared__ __align__(16) f16 xs[2][TOK * kCStage];
   // Group sums of four groups (a pair of stages) as bf16 parts (s0, s1, s2, s0, s1, s2, 0, 0).
   __shared__ __align__(16) u32x4 sx[kBias ? 2 : 1][kBias ? TOK * 4 : 1];
@@ -207,6 +221,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   uint32_t sv[NT], sn[NT];
   u32x4 cv[kRing ? 1 : NT], cn[kRing ? 1 : NT];
   auto load_pair = [&](int p) {
+    if constexpr (kPlain) return;
     const int g = min(4 * p + kq, n_grp - 1);  // past the split: its last group again
     const int so = kMarlin ? tile8 * GS + (l16 & 7) * SB + g * GS : (l16 * KG + g) * SB;
 #pragma unroll
@@ -285,7 +300,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       load_w(2 * s + 2, std::integral_constant<int, 2 - 2 * b>{});
       load_w(2 * s + 3, std::integral_constant<int, 3 - 2 * b>{});
     }
-    if constexpr (b == 0) {
+    if constexpr (b == 0 && !kPlain) {
       // A pair of stages begins: its scales and codes are there, the next pair's are requested.
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
@@ -297,7 +312,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
     }
     u32x2 sc2[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) sc2[t] = lane_rows<b>(sv[t]);
+    for (int t = 0; t < NT; ++t) sc2[t] = kPlain ? u32x2{0, 0} : lane_rows<b>(sv[t]);
     if (kBias) {
       // Sums of the stage's two groups per row, TPP threads each.
       constexpr int TPP = MB == 1 ? 8 : (MB == 2 ? 4 : 2);
@@ -350,6 +365,15 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
         else q.w = cv[t][2 * b + g];
         if constexpr (kMarlin) q.own_rows(row_sel);
         const f16x8 q0 = q.operand(0), q1 = q.operand(1);
+        if constexpr (kPlain) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[0][mb], q0, acc[t][mb], 0, 0, 0);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[1][mb], q1, acc[t][mb], 0, 0, 0);
+          continue;
+        }
         const float sc = h2f(u16_as_h((uint16_t)sc2[t][g]));
         f32x4 d[MB];
 #pragma unroll
@@ -364,10 +388,10 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       }
     };
     group(B0{});
-    group(B1{});
+    if (!kPlain || s != s_tail) group(B1{});  // (plain weights may be infinite: not even times zero)
     // The next stage's x (requested first in this one) is in LDS; of the loads after it some may
     // still be under way.
-    wait_loads<kRing || b == 0 ? NT : 0>();
+    wait_loads<kPlain ? 2 * NT : kRing || b == 0 ? NT : 0>();
     __syncthreads();
   };
   // The bias term of the pair of stages that holds stage s (after its barrier).
@@ -685,12 +709,19 @@ void codes_launch_shape(const T16Args& a, int M, const CodesPlan& p, hipStream_t
   }
 }
 
+template <int F>
+void codes_launch_epi(const T16Args& a, int M, int epi, const CodesPlan& p, hipStream_t s) {
+  if (epi == Q4_EPI_STORE) codes_launch_shape<F, Q4_EPI_STORE>(a, M, p, s);
+  else if (epi == Q4_EPI_RESID) codes_launch_shape<F, Q4_EPI_RESID>(a, M, p, s);
+  else codes_launch_shape<F, Q4_EPI_SWIGLU>(a, M, p, s);
+}
+
 }  // namespace
 
 // Code / scale bytes of a matrix.
 static size_t codes_bytes(int fmt, int rows, int K) {
   if (fmt == kCodesMarlin) return (size_t)((rows + 7) / 8) * (K / 64) * 256;
-  return (size_t)rows * (fmt == kCodesQ2kGguf ? K / 256 * 84 : fmt == kCodesQ8 ? K : K / 4);
+  return (size_t)rows * (fmt == kCodesF16 ? 2 * K : fmt == kCodesQ2kGguf ? K / 256 * 84 : fmt == kCodesQ8 ? K : K / 4);
 }
 static size_t scale_bytes(int fmt, int rows, int K) {
   const size_t r = fmt == kCodesMarlin ? (size_t)(rows + 7) / 8 * 8 : rows;
@@ -702,7 +733,7 @@ bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int r
     return K > 0 && K % 256 == 0 && K <= 16384 && (size_t)rows * (K / 256) * 84 < (size_t)0x7FFFFFF0 &&
            ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 3) == 0;
   const size_t code_bytes = codes_bytes(fmt, rows, K);
-  const uintptr_t wa = fmt == kCodesQ8 ? 15 : fmt == kCodesMarlin ? 7 : 3, sa = fmt == kCodesTernary ? 1 : 3;
+  const uintptr_t wa = fmt == kCodesQ8 || fmt == kCodesF16 ? 15 : fmt == kCodesMarlin ? 7 : 3, sa = fmt == kCodesTernary ? 1 : 3;
   return K > 0 && K % 64 == 0 && K <= 32768 && code_bytes < (size_t)0x7FFFFFF0 && ((uintptr_t)x & 15) == 0 &&
          ((uintptr_t)w & wa) == 0 && ((uintptr_t)sb & sa) == 0;
 }
@@ -716,7 +747,7 @@ size_t codes_gemm_ws_bytes(int M, int K, int N, int epi) {
 int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s) {
   const int rows = epi == Q4_EPI_SWIGLU ? 2 * a.N : a.N;
   if (M < 1 || !codes_gemm_takes(a.x, a.w16, a.sb16, a.K, rows, fmt) || a.ldx % 8 != 0 || a.ln_w != nullptr ||
-      (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) || (fmt != kCodesQ8 && epi != Q4_EPI_STORE) ||
+      (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) || (fmt != kCodesQ8 && fmt != kCodesF16 && epi != Q4_EPI_STORE) ||
       (a.post_ln_w != nullptr && (epi != Q4_EPI_RESID || a.post_norm_out == nullptr || a.ldr != a.N))) {
     axm_set_error("codes gemm: format %d, M=%d, epi=%d, K=%d unsupported", fmt, M, epi, a.K);
     return -2;
@@ -739,9 +770,8 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
   else if (fmt == kCodesQ2) codes_launch_shape<kCodesQ2, Q4_EPI_STORE>(a, M, p, s);
   else if (fmt == kCodesMarlin) codes_launch_shape<kCodesMarlin, Q4_EPI_STORE>(a, M, p, s);
   else if (fmt == kCodesTernary) codes_launch_shape<kCodesTernary, Q4_EPI_STORE>(a, M, p, s);
-  else if (epi == Q4_EPI_STORE) codes_launch_shape<kCodesQ8, Q4_EPI_STORE>(a, M, p, s);
-  else if (epi == Q4_EPI_RESID) codes_launch_shape<kCodesQ8, Q4_EPI_RESID>(a, M, p, s);
-  else codes_launch_shape<kCodesQ8, Q4_EPI_SWIGLU>(a, M, p, s);
+  else if (fmt == kCodesF16) codes_launch_epi<kCodesF16>(a, M, epi, p, s);
+  else codes_launch_epi<kCodesQ8>(a, M, epi, p, s);
   return t16_gemm_finish(a, M, epi, p.splits, M, s);
 }
 

@@ -653,16 +653,20 @@ struct axm_runner {
   // Q8_G64 (format 1) or fp16 (format 2) lm_head over T rows into logits: with ln_w the
   // GEMV applies the final RMSNorm itself and writes the normalized rows to xn_out (one
   // launch where a separate norm took two); without, the rows are normalized already.
+  // The several-row GEMM's format and fewest rows for a Q8_G64 (fmt 1) or fp16 (fmt 2) matrix.
+  static int dense_codes(int fmt) { return fmt == 1 ? kCodesQ8 : kCodesF16; }
+  static int dense_min_rows(int fmt) { return fmt == 1 ? kCodesQ8MinRows : kCodesF16MinRows; }
+
   int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s, f16* out = nullptr,
                     const RowBufs* b = nullptr) {
     if (out == nullptr) out = logits;
-    if (b != nullptr && ln_w == nullptr && d.lm_head_format == 1 && T >= kCodesQ8MinRows) {
+    if (b != nullptr && ln_w == nullptr && T >= dense_min_rows(d.lm_head_format)) {
       Mat m;
       m.w = d.lm_head_w;
       m.sb = d.lm_head_sb;
       m.N = d.vocab_size;
       m.K = d.d_model;
-      m.fmt = 1;
+      m.fmt = d.lm_head_format;
       GemvCall c{};
       c.x = x;
       c.ldx = d.d_model;
@@ -780,10 +784,10 @@ struct axm_runner {
       }
       return 0;
     }
-    if (m.fmt == 1 && T >= kCodesQ8MinRows && c.argmax_keys == nullptr && c.q_dim == 0 &&
+    if (m.fmt != 0 && T >= dense_min_rows(m.fmt) && c.argmax_keys == nullptr && c.q_dim == 0 &&
         (epi == Q4_EPI_STORE || epi == Q4_EPI_RESID || epi == Q4_EPI_SWIGLU) &&
-        codes_gemm_takes(c.x, m.w, m.sb, m.K, m.N, kCodesQ8)) {
-      // Q8_G64: all rows in one launch over the codes as stored.
+        codes_gemm_takes(c.x, m.w, m.sb, m.K, m.N, dense_codes(m.fmt))) {
+      // Q8_G64 or fp16: all rows in one launch over the weights as stored.
       T16Args a{};
       a.x = c.x;
       if (c.ln_w != nullptr) {
@@ -805,7 +809,7 @@ struct axm_runner {
       a.post_norm_out = c.post_norm_out;
       a.eps = c.eps;
       a.split_info = c.split_info;
-      return codes_gemm_launch(kCodesQ8, a, T, epi, b.ws, b.ws_bytes, s);
+      return codes_gemm_launch(dense_codes(m.fmt), a, T, epi, b.ws, b.ws_bytes, s);
     }
     for (int t0 = 0; t0 < T; t0 += 4) {
       const int mc = (T - t0) < 4 ? (T - t0) : 4;
@@ -973,8 +977,8 @@ struct axm_runner {
     size_t w = tree_workspace_bytes(T, d.n_head, d.head_dim,
                                     tree_choose_splits(T, d.n_head, d.n_kv_head, d.max_seq_len));
     auto gemm = [&](const Mat& m, int rows, int epi) {
-      if (m.w16 == nullptr && m.fmt != 1) return;
-      const size_t g = m.fmt == 1 ? codes_gemm_ws_bytes(T, m.K, rows, epi)
+      if (m.w16 == nullptr && m.fmt == 0) return;
+      const size_t g = m.fmt != 0 ? codes_gemm_ws_bytes(T, m.K, rows, epi)
                        : T > kTile16GemmMaxTokens ? t16_rows_gemm_ws_bytes(T, m.K, (rows + 15) / 16, epi)
                                                 : t16_gemm_ws_bytes(m.K, (rows + 15) / 16, epi == Q4_EPI_SWIGLU ? 2 : 1);
       w = g > w ? g : w;
@@ -983,10 +987,10 @@ struct axm_runner {
     gemm(m_o[0], d.d_model, Q4_EPI_RESID);
     gemm(m_gu[0], d.hidden_dim, Q4_EPI_SWIGLU);
     gemm(m_dn[0], d.d_model, Q4_EPI_RESID);
-    if (d.lm_head_format == 1) {
+    if (d.lm_head_format != 0) {
       Mat head;
       head.K = d.d_model;
-      head.fmt = 1;
+      head.fmt = d.lm_head_format;
       gemm(head, d.vocab_size, Q4_EPI_STORE);
     } else {
       gemm(m_lmh, d.vocab_size, Q4_EPI_STORE);
@@ -1150,12 +1154,12 @@ extern "C" int axm_runner_create(const axm_runner_desc* desc, axm_runner_t* out)
     for (size_t b : g) r->ws_bytes = b > r->ws_bytes ? b : r->ws_bytes;
   }
   for (int t = kCodesQ8MinRows; t <= T; ++t) {
-    // Partial tiles of the Q8_G64 several-row GEMM.
-    const size_t g[] = {d.qkv_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, r->qkv_dim, Q4_EPI_STORE) : 0,
-                        d.o_format == 1 ? codes_gemm_ws_bytes(t, r->q_dim, d.d_model, Q4_EPI_RESID) : 0,
-                        d.gu_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, d.hidden_dim, Q4_EPI_SWIGLU) : 0,
-                        d.down_format == 1 ? codes_gemm_ws_bytes(t, d.hidden_dim, d.d_model, Q4_EPI_RESID) : 0,
-                        d.lm_head_format == 1 ? codes_gemm_ws_bytes(t, d.d_model, d.vocab_size, Q4_EPI_STORE) : 0};
+    // Partial tiles of the Q8_G64 and fp16 several-row GEMM.
+    const size_t g[] = {d.qkv_format != 0 ? codes_gemm_ws_bytes(t, d.d_model, r->qkv_dim, Q4_EPI_STORE) : 0,
+                        d.o_format != 0 ? codes_gemm_ws_bytes(t, r->q_dim, d.d_model, Q4_EPI_RESID) : 0,
+                        d.gu_format != 0 ? codes_gemm_ws_bytes(t, d.d_model, d.hidden_dim, Q4_EPI_SWIGLU) : 0,
+                        d.down_format != 0 ? codes_gemm_ws_bytes(t, d.hidden_dim, d.d_model, Q4_EPI_RESID) : 0,
+                        d.lm_head_format != 0 ? codes_gemm_ws_bytes(t, d.d_model, d.vocab_size, Q4_EPI_STORE) : 0};
     for (size_t b : g) r->ws_bytes = b > r->ws_bytes ? b : r->ws_bytes;
   }
   struct {

@@ -113,3 +113,56 @@ def test_forward_prompt_equals_verify_chunks(dev, ring, S, T, every):
     assert (na.float() - nb.float()).abs().max().item() <= 2e-2
     used = min(T, S)
     assert (ca.cache[..., :used, :].float() - cb.cache[..., :used, :].float()).abs().max().item() <= 2e-2
+
+
+# Rows per GEMM: 5 the smallest, 16-64-row tiles with remainders, several row blocks; K = 704 ends inside a stage.
+@pytest.mark.parametrize("T", [5, 17, 40, 64, 131])
+def test_fp16_weights_prompt_matches_oracle(dev, T):
+    print(f"[fp16_prompt] T={T}", flush=True)
+    cfg = om.OracleConfig(n_layer=2, n_head=4, n_kv_head=2, d_model=256, hidden=704, vocab=1000, eps=1e-5,
+                          block_size=256)
+    ow = om.fp16_model(cfg, om.make_float_weights(cfg, seed=7))
+    rng = np.random.default_rng(T)
+    ow.c_attn_b = [(rng.standard_normal((cfg.n_head + 2 * cfg.n_kv_head) * cfg.head_dim) * 0.1).astype(np.float16)
+                   for _ in range(cfg.n_layer)]
+    cos, sin = om.rope_tables(cfg.head_dim, cfg.block_size)
+    runner, cache = _fp16_runner(cfg, ow, cos, sin, dev, 192)
+    toks = rng.integers(0, cfg.vocab, T).tolist()
+    got = runner.prompt_step(torch.tensor([toks], device=dev), 0, 0, "all", 1)[0].float().cpu().numpy()
+    model = om.OracleModel(cfg, ow, cos, sin)
+    ref = model.forward(toks, om.OracleKVCache(192, cfg.n_layer, cfg.n_kv_head, cfg.head_dim, "fp16"),
+                        return_all_logits=True)
+    for t in range(T):
+        _check_logits(got[t], ref[t], f"fp16 prompt token {t} of {T}")
+
+
+def test_fp16_weights_long_prompt_matches_four_token_steps(dev):
+    """Four weight tiles per wave (64-row tiles of a large launch) against the GEMVs, four tokens at a time."""
+    cfg = om.OracleConfig(n_layer=1, n_head=8, n_kv_head=4, d_model=512, hidden=5632, vocab=1000, eps=1e-5,
+                          block_size=1024)
+    ow = om.fp16_model(cfg, om.make_float_weights(cfg, seed=3))
+    cos, sin = om.rope_tables(cfg.head_dim, cfg.block_size)
+    T = 932
+    idx = torch.from_numpy(np.random.default_rng(4).integers(0, cfg.vocab, (1, T))).to(dev)
+    runner, cache = _fp16_runner(cfg, ow, cos, sin, dev, 1024)
+    got = runner.prompt_step(idx, 0, 0, "all", 1)[0].float().cpu().numpy()
+    runner, cache = _fp16_runner(cfg, ow, cos, sin, dev, 1024)
+    for t0 in range(0, T, 4):
+        ref = runner.prompt_step(idx[:, t0:t0 + 4], t0, t0, "all", 1)[0].float().cpu().numpy()
+        for t in range(4):
+            _check_logits(got[t0 + t], ref[t], f"fp16 prompt token {t0 + t}")
+
+
+def _fp16_runner(cfg, ow, cos, sin, dev, S):
+    from axiomlm_amd.cache import StaticKVCache
+    from axiomlm_amd.runner import DecodeRunner
+
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    cache = StaticKVCache(1, S, cfg.n_layer, cfg.n_kv_head, cfg.head_dim, device=dev, cache_dtype="fp16")
+    runner = DecodeRunner(t(ow.wte_p), t(np.stack([cos, sin], axis=-1).astype(np.float32)), [t(x) for x in ow.ln1],
+                          [t(x) for x in ow.c_attn_p], [t(x) for x in ow.c_proj_p], [t(x) for x in ow.ln2],
+                          [t(x) for x in ow.gu_p], [t(x) for x in ow.wd_p], t(ow.lnf), cache.k_caches, cache.v_caches,
+                          cfg.n_head, cfg.n_kv_head, cfg.head_dim, cfg.eps, lm_head_w=t(ow.lmh_p),
+                          c_attn_bs=[t(b) for b in (ow.c_attn_b or [])], k_scales=cache.k_scales,
+                          v_scales=cache.v_scales, kv_dtype="fp16")
+    return runner, cache
