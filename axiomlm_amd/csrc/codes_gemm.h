@@ -1,4 +1,4 @@
-// Several-row GEMM over row-major code matrices with 64-column groups (codes_gemm.hip).
+// Several-row GEMM over code matrices with 64-column groups and over fp16 rows (codes_gemm.hip).
 #pragma once
 #include "q4_tile16.h"
 

@@ -217,7 +217,7 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   // Scales (and biases), and 2-bit codes, are requested for two stages at a time, lane quarter kq
   // taking group kq of the four: 16 (64) contiguous bytes per row and request.  Group by group each
   // request touched 16 cache lines for 4 bytes each, and those requests, not bytes or latency,
-  // bound the launch (Q8, 22016 x 4096, 75 rows: 87 us, 59 with constant scales).
+  // bound the launch (Q8, 22016 x 4096, 75 rows: 87 us, 59 with constant scales, 68.5 this way).
   uint32_t sv[NT], sn[NT];
   u32x4 cv[kRing ? 1 : NT], cn[kRing ? 1 : NT];
   auto load_pair = [&](int p) {
@@ -459,6 +459,9 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
 // columns in order.  sc q (at most 45) comes from a four-entry byte table of multiples of sc by one byte
 // permute and enters the MFMA as an exact half; the min term is one bf16 MFMA per half block
 // whose A holds the sixteen-column sums in three parts and whose B the integers m.
+// Against the GEMV's launches of 4-16 rows (us): 4096 x 11008, 16 rows 25.5 -> 17, 40 rows 53 -> 25.5, 64
+// rows 87.5 -> 30; 12288 x 4096, 64 rows 90.5 -> 30, 1000 rows 204 here.  Few rows are bound by the
+// latency of the few stages of a split, many by the vector units, as above.
 template <int MB, int NT>
 __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
   constexpr int TOK = 16 * MB;
@@ -644,14 +647,15 @@ struct CodesPlan {
   int mb, nt, splits;
 };
 // Row tile: the fewest row blocks of up to 64 rows, evenly filled.  Weight tiles per wave (two, or
-// four with 64 rows; 48 rows with four were always slower) and K splits by the time each choice is expected to take: a round of the
-// workgroups that fit a CU (four of up to 32 rows, three with two tiles per wave, two with four)
-// (or part of one past the first) costs kStage[0] us per stage, each workgroup of a CU kStage[1]; partial tiles are written
-// and read back at about 5 TB/s.  Fitted to a sweep of 1-16 splits and both tile counts over 8-1000
-// rows, six matrices (1024-22016 rows) and five formats: the choice is within 1-2 % of the sweep's
-// best on average and 14 % at worst but for one (27 %), four tiles per wave with two workgroups a CU
-// had been 15-35 % off on average (Q8 4096 x 4096, 40 rows: four tiles 20.3 us, two from eight splits
-// 15.1; 12288 x 4096, 75 rows 41.0 / 34.7; 1000 rows: four tiles unsplit 155, two 167).
+// four with 64 rows; 48 rows with four were always slower) and K splits by the time each choice is
+// expected to take: a round of the workgroups that fit a CU (four of up to 32 rows, three with two
+// tiles per wave, two with four) (or part of one past the first) costs kStage[0] us per stage,
+// each workgroup of a CU kStage[1]; partial tiles are written and read back at about 5 TB/s.
+// Fitted to a sweep of 1-16 splits and both tile counts over 8-1000 rows, six matrices (1024-22016
+// rows) and five formats: the choice is within 1-2 % of the sweep's best on average and 14 % at
+// worst but for one (27 %), four tiles per wave with two workgroups a CU had been 15-35 % off on
+// average (Q8 4096 x 4096, 40 rows: four tiles 20.3 us, two from eight splits 15.1; 12288 x 4096,
+// 75 rows 41.0 / 34.7; 1000 rows: four tiles unsplit 155, two 167).
 CodesPlan codes_plan(int M, int KB, int n_units, int epi) {
   static const float kStage[5][2] = {{.18f, .41f}, {.26f, .51f}, {.38f, .51f}, {.53f, .54f},  // 16-64 rows, two tiles
                                      {1.f, .9f}};                                             // 64, four
