@@ -30,6 +30,7 @@
 
 #include "axm.h"
 #include "codes_gemm.h"
+#include "gemm_offsets.h"
 #include "kernels.h"
 #include "t16_device.h"
 
@@ -37,7 +38,7 @@ namespace {
 
 constexpr int kCThreads = 256;
 constexpr int kCWaves = kCThreads / 64;
-constexpr int kCStage = 128;
+constexpr int kCStage = go::kStage;
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -197,18 +198,15 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       __builtin_amdgcn_make_buffer_rsrc((void*)a.sb16, (short)0, (int)a.sb16_bytes, 0x00020000);
 
   // This lane's codes of tile 0, and the (wave-uniform) first row of tile t: an up tile starts
-  // a.N rows after its gate tile.  Tiles past the matrix read the last one, the last one's rows
-  // past it zeros; neither is stored.
-  // (MARLIN: 256 code and 32 scale bytes per eight rows and group.)
-  const int tile8 = (l16 >> 3) * KG;
-  const int wlane = kMarlin ? tile8 * 256 + 8 * ((kq >> 1) * 16 + (l16 & 4) * 2 + (kq & 1) * 4 + (l16 & 1) * 2 +
-                                                 ((l16 >> 1) & 1))
-                            : l16 * KG * RB + kq * (RB / 4);
-  constexpr int GW = kMarlin ? 256 : RB, GS = kMarlin ? 32 : SB;  // bytes from group to group
+  // a.N rows after its gate tile.  Tiles past the matrix read the last one and are not stored.
+  const int w_rows = kMarlin ? (a.N + 7) & ~7 : a.N;
+  const int lrow = go::w_lane_row(l16, w_rows);
+  const int wlane = go::w_lane(kMarlin, lrow, kq, KG, RB);
   const uint32_t row_sel = l16 & 1 ? 0x03020706u : 0x05040100u;   // Codes<kCodesMarlin>
   int row0[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) row0[t] = min(unit + t % UPW, a.n_units - 1) * 16 + (kPair && t >= UPW ? a.N : 0);
+  for (int t = 0; t < NT; ++t)
+    row0[t] = go::w_row0(unit + t % UPW, a.n_units, w_rows) + (kPair && t >= UPW ? a.N : 0);
   // The row's last stage has one group only if K % 128 == 64: its second one reads that group
   // again, and zeros of x.
   const int s_tail = a.K % kCStage != 0 && kbA + n_st == a.KB ? n_st - 1 : -1;
@@ -223,15 +221,15 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   auto load_pair = [&](int p) {
     if constexpr (kPlain) return;
     const int g = min(4 * p + kq, n_grp - 1);  // past the split: its last group again
-    const int so = kMarlin ? tile8 * GS + (l16 & 7) * SB + g * GS : (l16 * KG + g) * SB;
+    const int so = go::s_lane(kMarlin, lrow, g, KG, SB);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int ch = row0[t] * KG * SB + 2 * kbA * GS;
+      const int ch = go::s_soff(kMarlin, row0[t], kbA, KG, SB);
       if (kBias) sn[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, so, ch, 0);
       else sn[t] = __builtin_amdgcn_raw_buffer_load_b16(rs, so, ch, 0);
       if constexpr (!kRing)
         cn[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                              rw, (l16 * KG + g) * RB, (row0[t] * KG + 2 * kbA) * RB, 0));
+                                              rw, (lrow * KG + g) * RB, (row0[t] * KG + 2 * kbA) * RB, 0));
     }
   };
   // Codes of RING groups: a stage ahead, or (Q8's 64-row tiles, for their registers) a group ahead.
@@ -241,36 +239,40 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       constexpr int b = decltype(bc)::value;
       const int g = 2 * kbA + min(gi, n_grp - 1);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wr[b][t].load(rw, wlane, row0[t] * KG * RB + g * GW);
+      for (int t = 0; t < NT; ++t) wr[b][t].load(rw, wlane, go::w_soff(kMarlin, row0[t], g, KG, RB));
     }
   };
 
   // Activations to LDS as in rows_gemm.hip: row r's 16-byte piece p at position p ^ (r % 16).
+  const int x_rows = min(a.M_tokens - m0, TOK), x_last = go::x_last(x_rows);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
+      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, x_rows * a.ldx * (int)sizeof(f16), 0x00020000);
   const int xrow = 4 * wave + kq;
-  const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  const int xoff = go::x_lane(xrow, l16, a.ldx);
   // MARLIN: a row per request, word s of piece (g, quarter, c) from word 32 g + 16 c + 4 s + quarter.
   int xm[kMarlin ? 4 : 1];
   if constexpr (kMarlin)
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int r = 4 * wave + n, p = (lane >> 2) ^ r;
-      xm[n] = r * a.ldx * 2 + 4 * (32 * (p >> 3) + 16 * (p & 1) + 4 * (lane & 3) + ((p >> 1) & 3));
-    }
+    for (int n = 0; n < 4; ++n) xm[n] = go::x_marlin_lane(4 * wave + n, lane, a.ldx);
   auto load_x = [&](int s, auto bc) {
     constexpr int b = decltype(bc)::value;
-    const int so = (kbA + min(s, n_st - 1)) * (kCStage * 2);
+    const int st = kbA + min(s, n_st - 1);
+    const bool half = go::x_half_stage(st, a.K);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
+      const int so = go::x_soff(st, i, x_last, a.ldx);
       if constexpr (kMarlin) {
 #pragma unroll
-        for (int n = 0; n < 4; ++n)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave + n) * kCStage]), 4, xm[n],
-                                                   so + i * 32 * a.ldx, 0, 0);
+        for (int n = 0; n < 4; ++n) {
+          const int r = 4 * wave + n;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              rx, (lds_void*)(&xs[b][(16 * i + r) * kCStage]), 4,
+              go::x_voff(xm[n], i, x_last, 16 * x_last + r < x_rows, half && go::x_marlin_hi(r, lane)), so, 0, 0);
+        }
       } else {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
-                                                 so + i * 32 * a.ldx, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16,
+            go::x_voff(xoff, i, x_last, 16 * x_last + xrow < x_rows, half && go::x_lane_hi(xrow, l16)), so, 0, 0);
       }
     }
   };
@@ -435,8 +437,8 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
   // Lane: weight row l16 of each tile, tokens 4 kq .. + 3 of each 16.
 #pragma unroll
   for (int t = 0; t < (n_split == 1 ? UPW : NT); ++t) {
-    const int u = unit + t % UPW, row = u * 16 + l16;
-    if (u >= a.n_units || (n_split == 1 && row >= a.N)) continue;
+    const int u = unit + t % UPW, row = go::w_row0(u, a.n_units, w_rows) + l16;
+    if (u >= a.n_units || row < u * 16 || row >= a.N) continue;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -465,7 +467,6 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
 template <int MB, int NT>
 __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n_mblk, int n_split, int n_tile) {
   constexpr int TOK = 16 * MB;
-  constexpr int kBlock = 84;
   __shared__ __align__(16) f16 xs[2][TOK * kCStage];
   __shared__ __align__(16) u32x2 sx[2][TOK * 8];  // bf16 parts (s0, s1, s2, 0) of each sub-block's sum
 
@@ -486,7 +487,7 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
   const int NB = a.K / 256;
   const __amdgpu_buffer_rsrc_t rw =
       __builtin_amdgcn_make_buffer_rsrc((void*)a.w16, (short)0, (int)a.w16_bytes, 0x00020000);
-  const int wlane = l16 * NB * kBlock;
+  const int wlane = go::q2k_lane(go::w_lane_row(l16, a.N), NB);
 
   u32x2 cw[2][NT], sw[2][NT];
   uint32_t dw[2][NT];
@@ -496,24 +497,25 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
     const int h = hb & 1;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      // Wave-uniform; tiles past the matrix read the last one, the last one's rows past it zeros.
-      const int base = (min(unit + t, a.n_units - 1) * 16 * NB + (hb >> 1)) * kBlock;
+      const int base = go::q2k_soff(go::w_row0(unit + t, a.n_units, a.N), hb, NB);  // wave-uniform
       cw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane + 8 * kq, base + 16 + 32 * h, 0));
       sw[b][t] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, wlane, base + 8 * h, 0));
       dw[b][t] = __builtin_amdgcn_raw_buffer_load_b32(rw, wlane, base + 80, 0);
     }
   };
+  const int x_rows = min(a.M_tokens - m0, TOK), x_last = go::x_last(x_rows);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
+      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, x_rows * a.ldx * (int)sizeof(f16), 0x00020000);
   const int xrow = 4 * wave + kq;
-  const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  const int xoff = go::x_lane(xrow, l16, a.ldx);
   auto load_x = [&](int s, auto bc) {
     constexpr int b = decltype(bc)::value;
-    const int so = (kbA + min(s, n_st - 1)) * (kCStage * 2);
+    const int st = kbA + min(s, n_st - 1);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16, xoff,
-                                               so + i * 32 * a.ldx, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kCStage]), 16,
+                                               go::x_voff(xoff, i, x_last, 16 * x_last + xrow < x_rows, false),
+                                               go::x_soff(st, i, x_last, a.ldx), 0, 0);
   };
 
   f32x4 acc[NT][MB];
@@ -629,8 +631,8 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
 
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    const int row = (unit + t) * 16 + l16;
-    if (unit + t >= a.n_units || (n_split == 1 && row >= a.N)) continue;
+    const int row = go::w_row0(unit + t, a.n_units, a.N) + l16;
+    if (unit + t >= a.n_units || row < (unit + t) * 16 || row >= a.N) continue;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

@@ -22,6 +22,7 @@
 // rows QKV 177 (1164).  A large fp16 library product reaches 1340-1410 TFLOP/s on this card.
 #include <type_traits>
 
+#include "gemm_offsets.h"
 #include "kernels.h"
 #include "q4_tile16.h"
 #include "t16_device.h"
@@ -30,8 +31,7 @@ namespace {
 
 constexpr int kRThreads = 256;
 constexpr int kRWaves = kRThreads / 64;
-constexpr int kRStage = 128;  // columns per stage (one tile16 chunk)
-constexpr int kROOB = 0x7FFFFFF0;
+constexpr int kRStage = go::kStage;  // columns per stage (one tile16 chunk)
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -94,19 +94,23 @@ __global__ void __launch_bounds__(kRThreads, 2) rows_gemm_kernel(T16Args a, int 
 
   // Activations of stage s into buffer b: load i of wave w covers rows 16 i + 4 w .. + 3,
   // lane l the piece (l % 16) ^ (row % 16) of row l / 16 of them, which lands at LDS
-  // position l % 16 of that row.  Rows past M are out of the descriptor's range; whatever
-  // their LDS rows hold, their results are never stored.
+  // position l % 16 of that row.  Rows past M, and columns past K, are requested out of the
+  // descriptor's range; whatever the LDS rows of the former hold, their results are never stored.
+  const int x_rows = min(a.M_tokens - m0, TOK), x_last = go::x_last(x_rows);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, min(a.M_tokens - m0, TOK) * a.ldx * (int)sizeof(f16), 0x00020000);
+      (void*)(a.x + (size_t)m0 * a.ldx), (short)0, x_rows * a.ldx * (int)sizeof(f16), 0x00020000);
   const int xrow = 4 * wave + kq;
-  const int xoff = xrow * a.ldx * 2 + ((l16 ^ xrow) * 16);
+  const int xoff = go::x_lane(xrow, l16, a.ldx);
   auto load_x = [&](int s, auto bc) {
     constexpr int b = decltype(bc)::value;
-    const int so = (kbA + min(s, n_st - 1)) * (kRStage * 2);
+    const int st = kbA + min(s, n_st - 1);
+    const bool half = go::x_half_stage(st, a.K);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kRStage]), 16, xoff,
-                                               so + i * 32 * a.ldx, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rx, (lds_void*)(&xs[b][(16 * i + 4 * wave) * kRStage]), 16,
+          go::x_voff(xoff, i, x_last, 16 * x_last + xrow < x_rows, half && go::x_lane_hi(xrow, l16)),
+          go::x_soff(st, i, x_last, a.ldx), 0, 0);
   };
 
   f32x4 acc[NT][MB];
