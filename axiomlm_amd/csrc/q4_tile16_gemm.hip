@@ -509,8 +509,12 @@ extern "C" size_t axm_qmm_q4_tile16_workspace_bytes(int K, int N, int swiglu) {
 
 extern "C" size_t axm_qmm_q4_tile16_rows_workspace_bytes(int M, int K, int N, int swiglu) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
-  return M <= kTile16GemmMaxTokens ? axm_qmm_q4_tile16_workspace_bytes(K, N, swiglu)
-                                   : t16_rows_gemm_ws_bytes(M, K, (N + 15) / 16, swiglu ? Q4_EPI_SWIGLU : Q4_EPI_STORE);
+  // Enough for either path of qmm_tile16_rows: rows that the many-row GEMM cannot load go through
+  // the 64-row passes, which need theirs.
+  const size_t pass = axm_qmm_q4_tile16_workspace_bytes(K, N, swiglu);
+  if (M <= kTile16GemmMaxTokens) return pass;
+  const size_t rows = t16_rows_gemm_ws_bytes(M, K, (N + 15) / 16, swiglu ? Q4_EPI_SWIGLU : Q4_EPI_STORE);
+  return rows > pass ? rows : pass;
 }
 
 static int qmm_tile16_rows(const void* x, const void* w16, const void* sb16, const void* bias, void* y, int M, int K,

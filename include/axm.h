@@ -76,7 +76,9 @@ int axm_qmv_q4_tile16_swiglu(const void* x, const void* ln_w, float eps, const v
  * (axm_qmm_q4_tile16_workspace_bytes: enough for any M, 0 when no split is used). */
 size_t axm_qmm_q4_tile16_workspace_bytes(int K, int N, int swiglu);
 /* The workspace that M rows use best: from 65 rows on one launch of the many-row GEMM, which
- * splits K where M and N leave CUs idle, as far as the workspace given allows. */
+ * splits K where M and N leave CUs idle, as far as the workspace given allows.  Never less than
+ * axm_qmm_q4_tile16_workspace_bytes, which more than 64 rows need where x is not 16-byte aligned
+ * (they then run in passes of 64). */
 size_t axm_qmm_q4_tile16_rows_workspace_bytes(int M, int K, int N, int swiglu);
 int axm_qmm_q4_tile16(const void* x, const void* w16, const void* sb16, const void* bias, void* y, int M, int K,
                       int N, int group_size, void* workspace, size_t workspace_bytes, void* stream);

@@ -97,3 +97,34 @@ def test_rows_gemm_workspace_is_optional(dev):
                                                 N, 64, ws.data_ptr() if size else None, size, _lib.stream_of(dev)),
                    "qmm_q4_tile16")
         assert np.linalg.norm(y.cpu().numpy().astype(np.float64) - ref) <= REL * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("skip", [4, 1])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_rows_of_a_misaligned_view(dev, skip, swiglu):
+    """Rows that start 8 or 2 bytes past a 16-byte boundary (contiguous: nothing copies them) run in passes of 64, also
+    where the many-row GEMM would want no workspace (unsplit) and the passes split K."""
+    import torch
+
+    from axiomlm_amd import _lib
+    from axiomlm_amd.kernels import qmv_q4_tile16, qmv_q4_tile16_swiglu
+
+    M, N, K = 130, 4096, 1024
+    L = _lib.lib()
+    assert L.axm_qmm_q4_tile16_rows_workspace_bytes(M, K, N, 0) >= L.axm_qmm_q4_tile16_workspace_bytes(K, N, 0) > 0
+    rng = np.random.default_rng(skip)
+    p, s, w = _pack(rng, N, K, 64)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    buf = torch.empty(skip + M * K, dtype=torch.float16, device=dev)
+    buf[skip:] = torch.from_numpy(x.reshape(-1)).to(dev)
+    xd = buf[skip:].view(M, K)
+    assert xd.data_ptr() % 16 == 2 * skip
+    y = x.astype(np.float64) @ w.T
+    if swiglu:
+        got = qmv_q4_tile16_swiglu(xd, None, 1e-5, *_tile16(dev, p, s, N, K), N // 2)
+        g, u = np.split(y, 2, axis=1)
+        y = g / (1 + np.exp(-g)) * u
+    else:
+        got = qmv_q4_tile16(xd, *_tile16(dev, p, s, N, K), N)
+    # bounds as for the aligned rows
+    assert np.linalg.norm(got.cpu().numpy().astype(np.float64) - y) <= (4 if swiglu else 1) * REL * np.linalg.norm(y)

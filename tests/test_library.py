@@ -52,3 +52,16 @@ def test_error_path_without_gpu_compute():
                                       ctypes.c_void_p(16), 1, 100, 8, None)
     assert rc != 0
     assert b"multiple of 64" in _lib.lib().axm_last_error()
+
+
+def test_many_row_workspace_covers_the_64_row_passes():
+    # Rows of x that the many-row GEMM cannot load (not 16-byte aligned) run in passes of 64,
+    # which refuse a workspace smaller than their own: the size for M rows is enough for both.
+    from axiomlm_amd import _lib
+
+    L = _lib.lib()
+    for M, N, K in [(1000, 12288, 4096), (128, 12288, 4096), (100, 4096, 11008), (130, 4096, 1024), (2048, 4096, 4096)]:
+        for swiglu in (0, 1):
+            one = L.axm_qmm_q4_tile16_workspace_bytes(K, N, swiglu)
+            assert L.axm_qmm_q4_tile16_rows_workspace_bytes(M, K, N, swiglu) >= one
+            assert L.axm_qmm_q4_tile16_rows_workspace_bytes(64, K, N, swiglu) == one
