@@ -44,9 +44,11 @@ GO_HD int x_marlin_lane(int row, int lane, int ldx) {
 GO_HD bool x_marlin_hi(int row, int lane) { return x_marlin_piece(row, lane) >= 8; }
 
 // Lane offset of piece i: `off` where the row exists and its columns lie inside K (the last stage
-// of K % 128 == 64 ends after 64).  row_in_last: the lane's row exists in piece x_last.
+// of K % 128 == 64 ends after 64).  row_in_last: the lane's row exists in piece x_last, which
+// pieces past it read again (one select fewer; nothing uses them).
 GO_HD int x_voff(int off, int i, int last, bool row_in_last, bool past_k) {
-  return i > last || (i == last && !row_in_last) || past_k ? kOOB : off;
+  const int full = past_k ? kOOB : off, ragged = row_in_last ? full : kOOB;
+  return i < last ? full : ragged;
 }
 GO_HD int x_soff(int stage, int i, int last, int ldx) { return stage * (kStage * 2) + min_i(i, last) * 32 * ldx; }
 GO_HD bool x_half_stage(int stage, int K) { return stage * kStage + 64 >= K; }
