@@ -307,6 +307,8 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       __syncthreads();
     }
     load_x(s + 1, bn);
+    // The wait at the stage's end counts the loads requested after these: none may move before them.
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (kRing && RING == 4) {
       load_w(2 * s + 2, std::integral_constant<int, 2 - 2 * b>{});
       load_w(2 * s + 3, std::integral_constant<int, 3 - 2 * b>{});
