@@ -255,12 +255,15 @@ class Transformer:
                        for b in bias],
             k_scales=cache0.k_scales, v_scales=cache0.v_scales, kv_dtype=cache0.cache_dtype, max_tokens=64)
 
-    @staticmethod
-    def _prompt_rows(cache0: StaticKVCache, n: int) -> int:
+    def _prompt_rows(self, cache0: StaticKVCache, n: int) -> int:
         """Tokens of the n left that the next pass takes as one prompt step, or 0: a verify chunk takes the
-        rest, a whole number of chunks goes before what does not fit the cache's tail (where the ring wraps)."""
+        rest.  Only a whole number of chunks goes before what does not fit the cache's tail (where the ring
+        wraps), and before a last token, or two or three of a model with Q4 matrices, alone past a chunk: one
+        token's attention keeps fp32 weights, and up to three rows are multiplied with the exact Q4 codes, where
+        more rows round each weight to fp16."""
         rows = min(n, PROMPT_ROWS, cache0.max_seq_len - cache0.total_seen_tokens[0])
-        if rows < n:
+        few = 1 if self._quant_mode in ("q8", None) else 3
+        if rows < n or 1 <= n % VERIFY_CHUNK <= few:
             rows -= rows % VERIFY_CHUNK
         return rows if rows > VERIFY_CHUNK else 0
 

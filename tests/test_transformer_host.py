@@ -76,3 +76,58 @@ def test_quantize_modes_and_tied_head():
     m.quantize("q4_rtn")
     with pytest.raises(RuntimeError):
         Transformer(c, sd, device="cpu").forward(torch.zeros(1, 1, dtype=torch.long), kv_caches=None)
+
+
+@pytest.mark.parametrize("mode,few", [("q4", 3), ("q4_rtn", 3), ("q4_k_m", 3), ("q8", 1), (None, 1)])
+def test_prompt_passes(mode, few):
+    """How a prompt is cut: one pass of all rows, but for up to `few` tokens past the last whole chunk of 32, which
+    run as they do alone (one token's attention, and up to three rows' Q4 products, are the more precise forms)."""
+    class Runner:
+        def __init__(self):
+            self.calls = []
+
+        def step(self, idx, *a):
+            self.calls.append(("step", idx.shape[1]))
+            return torch.zeros(1, 1, 8)
+
+        def verify_step(self, idx, *a):
+            self.calls.append(("verify", idx.shape[1]))
+            return torch.zeros(1, idx.shape[1], 8)
+
+        def prompt_step(self, idx, rope, write, logits, norm_rows):
+            self.calls.append(("prompt", idx.shape[1]))
+            return None if logits == "none" else torch.zeros(1, 1 if logits == "last" else idx.shape[1], 8)
+
+    class Cache:
+        n_layer, ring_buffer = 1, True
+
+        def __init__(self, S, seen):
+            self.max_seq_len, self.total_seen_tokens, self.layer_seq_lens = S, [seen], [min(seen, S)]
+
+    c = ModelConfig(n_layer=1, n_embd=64, n_head=1, vocab_size=8, intermediate_size=64, block_size=8192)
+    sd = {"transformer.wte.weight": torch.zeros(8, 64, dtype=torch.float16)}
+    m = Transformer(c, sd, device="cpu").quantize(mode)
+
+    def passes(T, S=8192, seen=0, every=False):
+        r = Runner()
+        m.get_decode_runner = lambda cache: r
+        cache = Cache(S, seen)
+        out = m.forward(torch.zeros(1, T, dtype=torch.long), kv_caches=cache, return_all_logits=every)[0]
+        assert out.shape == (1, T if every else 1, 8) and cache.total_seen_tokens == [seen + T]
+        return r.calls
+
+    one = [("step", 1)]
+    for every in (False, True):
+        assert passes(1, every=every) == one
+        assert passes(32, every=every) == [("verify", 32)]
+        assert passes(33, every=every) == [("verify", 32)] + one
+        assert passes(64, every=every) == [("prompt", 64)]
+        assert passes(65, every=every) == [("prompt", 64)] + one
+        for n in (2, 3):
+            tail = [("verify", n)]
+            assert passes(96 + n, every=every) == ([("prompt", 96)] + tail if n <= few else [("prompt", 96 + n)])
+            assert passes(2048 + n, every=every) == [("prompt", 2048)] + tail
+        assert passes(100, every=every) == [("prompt", 100)]
+        assert passes(2048 + 65, every=every) == [("prompt", 2048), ("prompt", 64)] + one
+        assert passes(150, S=128, every=every) == [("prompt", 128), ("verify", 22)]  # the ring wraps
+        assert passes(70, S=128, seen=100, every=every) == [("verify", 32), ("verify", 32), ("verify", 6)]
