@@ -1071,20 +1071,20 @@ int attn_flash_splits(int B, int Hq, int Hkv, int hd, int kv_dtype, int active_l
   return splits;
 }
 
-// A decode step of one sequence.  Grouped-query heads take the matrix-core kernel at every
-// length, from 32 keys on with splits of about 128 keys up to one workgroup per CU: the vector kernel with eight
-// splits per head set fills 64 CUs at 8 KV heads and multiplies every key once per query head (us per
-// layer of a 7B-shape step with 32 / 8 heads and an FP8 cache, vector kernel / four / eight / 32
-// splits here: 100 keys 46.1 / 43.5 / 43.6 / 44.6, 1000 keys 48.9 / 44.9 / 44.1 / 44.8, 4000 keys
-// 61.0 / 50.5 / 47.0 / 45.6, 16000 keys 113 / 73 / 59 / 51).  One query head per KV head: splits
-// merged by a reduce launch only where eight leave over half of the CUs idle for long (4 heads
-// of 64, FP8: 4000 keys eight merged by the O projection 31.9, 32 splits 33.0; 8000 keys 36.4 / 34.1;
-// 16000 keys 43.1 / 35.7; 32 heads: never faster).
+// A decode step of one sequence.  Two to sixteen query heads per KV head take the matrix-core kernel at
+// every length, from 32 keys on with splits of about 128 keys up to one workgroup per CU: the vector
+// kernel with eight splits per head set fills 64 CUs at 8 KV heads and multiplies every key once per
+// query head (us per layer of a 7B-shape step with 32 / 8 heads and an FP8 cache, vector kernel /
+// four / eight / 32 splits here: 100 keys 46.3 / 44.8 / 45.0 / 45.9, 1000 keys 49.5 / 48.2 / 46.0 /
+// 46.5, 4000 keys 61.6 / 60.4 / 52.4 / 47.3, 16000 keys 113 / 110 / 78 / 57).  Other groupings (one query
+// head per KV head, or more than sixteen): splits merged by a reduce launch only where eight leave over
+// half of the CUs idle for long (4 heads of 64, FP8: 4000 keys eight merged by the O projection 31.9, 32
+// splits 33.0; 8000 keys 36.4 / 34.1; 16000 keys 43.1 / 35.7; 32 heads: never faster).
 int attn_step_splits(int Hq, int Hkv, int active_len) {
   const int n_rep = Hq / Hkv;
   const int fill = axm_ceil_div(axm_num_cus(), Hkv);  // one workgroup per CU
   if (n_rep >= 2 && n_rep <= 16) {
-    int splits = active_len < 32 ? 1 : 4;  // (7 keys, FP16 cache, four layers: one 164 us, four 175)
+    int splits = active_len < 32 ? 1 : 4;  // (7 keys, FP16 cache, per layer: one 38.7 us, four 42.7)
     while (splits > 1 && splits < fill && splits < 64 && 128 * splits < active_len) splits <<= 1;
     return splits;
   }
@@ -1205,6 +1205,11 @@ constexpr int kTreeKeys = 32;    // keys per block (the k extent of one P V MFMA
 __device__ __forceinline__ int pt_index(int row, int key) {
   return row * kTreeKeys + (((key >> 3) ^ ((row >> 2) & 3)) << 3) + (key & 7);
 }
+// The same of fp32 weights: a row's 4-key groups are swizzled by its low bits (rows are a multiple of
+// all banks apart; eight rows then read one group from different banks).
+__device__ __forceinline__ int pt32_index(int row, int key) {
+  return row * kTreeKeys + (((key >> 2) ^ (row & 7)) << 2) + (key & 3);
+}
 
 // B operand of O += P V from V rows stored key-major (row stride vrow halves;
 // seg = row 0 of a 16-dim tile): lane (l16, lq) needs dim column l16 of keys
@@ -1243,12 +1248,13 @@ constexpr int kTreeRows = 64;    // query rows per workgroup (four waves of 16)
 // exp2(s - m) stay below 2^kMaxSlack with no row reduction, and only the
 // rescaling path takes the row maxima.  The caller sums l over each row's 16
 // lanes once after the last block.  The quotient o / l does not depend on m; the
-// fp16 weights P keep their relative precision up to 2^kMaxSlack.
-// With pt_lo the rest of each weight (what its fp16 rounding left out) goes to a second tile.
+// fp16 weights P keep their relative precision up to 2^kMaxSlack.  PT float: the weights stay fp32.
 constexpr float kMaxSlack = 8.f;
-template <int DT>
+__device__ __forceinline__ void put_weight(f16* pt, int row, int key, float p) { pt[pt_index(row, key)] = f2h(p); }
+__device__ __forceinline__ void put_weight(float* pt, int row, int key, float p) { pt[pt32_index(row, key)] = p; }
+template <int DT, typename PT>
 __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows, float (&m)[4], float (&l)[4],
-                                              f32x4 (&o)[DT], f16* pt, int lq, int l16, f16* pt_lo = nullptr) {
+                                              f32x4 (&o)[DT], PT* pt, int lq, int l16) {
   if (__builtin_amdgcn_ballot_w64(grows)) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1267,11 +1273,7 @@ __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows
     for (int h = 0; h < 2; ++h) pr[h] = s[v][h] == kNegBig ? 0.f : fast_exp2(s[v][h] - m[v]);
     l[v] += pr[0] + pr[1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const f16 hi = f2h(pr[h]);
-      pt[pt_index(4 * lq + v, 16 * h + l16)] = hi;
-      if (pt_lo != nullptr) pt_lo[pt_index(4 * lq + v, 16 * h + l16)] = f2h(pr[h] - h2f(hi));
-    }
+    for (int h = 0; h < 2; ++h) put_weight(pt, 4 * lq + v, 16 * h + l16, pr[h]);
   }
 }
 
@@ -1498,18 +1500,22 @@ int launch_tree_mfma(const AttnParams& p, dim3 grid, hipStream_t s) {
 // (wave-private transposed V and P tiles, no barrier in the loop) and merge
 // their (m, l, o) through LDS at the end.
 // ---------------------------------------------------------------------------
-// P32: the weights enter P V as two fp16 parts (22 bits, as the vector kernel's fp32 weights),
-// one more MFMA per tile.
+// P32: the weights stay fp32 as in the vector kernel, and P V runs on the fp32 matrix instruction
+// (16x16x4): lane (l16, lq) holds keys 8 lq .. + 7 of its row of P and of its column of V, so
+// step s takes key 8 lq + s of each quarter, and V goes in as the fp16 operand reads it, widened.
+// (Weights as two fp16 parts, one more fp16 MFMA per tile, took 1.9 us less per layer at 6000 FP8
+// keys of 8 KV heads and 5 at 16000, but weights below 2^-14 of the largest lost bits to fp16's
+// range, those below 2^-25 all of them, and an infinite value times a zero part was NaN.)
 template <int KVT, int HD, bool P32>
-__global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
+__global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParams p) {
   constexpr int KSTEPS = HD / 32;
   constexpr int DT = HD / 16;
   constexpr int kVPL = kTreeKeys * HD / 8 / 64;  // 8-element V vectors per lane and block
   // V rows as stored (key-major, padded rows) for the transposing LDS reads.
   constexpr int VROW = HD + 16;
   __shared__ __align__(16) f16 vr[4][kTreeKeys * VROW];
-  __shared__ __align__(16) f16 pt[4][16 * kTreeKeys];
-  __shared__ __align__(16) f16 pt_lo[P32 ? 4 : 1][P32 ? 16 * kTreeKeys : 8];
+  using PT = typename std::conditional<P32, float, f16>::type;
+  __shared__ __align__(16) PT pt[4][16 * kTreeKeys];
   __shared__ float mrg[4][16][2 + HD];
   auto pt_at = pt_index;
   const int lane = threadIdx.x & 63;
@@ -1620,17 +1626,27 @@ __global__ void __launch_bounds__(256) decode_mfma_kernel(AttnParams p) {
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16, P32 ? pt_lo[wave] : nullptr);
+    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16);
     // The wave reads back its own LDS writes: DS operations of one wave complete
     // in order, and the reads below wait for them.
-    const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
-    f16x8 pb;
-    if constexpr (P32) pb = *reinterpret_cast<const f16x8*>(&pt_lo[wave][pt_at(l16, 8 * lq)]);
+    if constexpr (P32) {
+      f32x4 pa[2];
 #pragma unroll
-    for (int d = 0; d < DT; ++d) {
-      const f16x8 vb = v_operand(&vr[wave][16 * d], VROW, l16, lq);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[d], 0, 0, 0);
-      if constexpr (P32) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pb, vb, o[d], 0, 0, 0);
+      for (int i = 0; i < 2; ++i) pa[i] = *reinterpret_cast<const f32x4*>(&pt[wave][pt32_index(l16, 8 * lq + 4 * i)]);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        const f16x8 vb = v_operand(&vr[wave][16 * d], VROW, l16, lq);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[k >> 2][k & 3], h2f(vb[k]), o[d], 0, 0, 0);
+      }
+    } else {
+      const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        const f16x8 vb = v_operand(&vr[wave][16 * d], VROW, l16, lq);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[d], 0, 0, 0);
+      }
     }
   };
   // With two buffers both blocks of an iteration run unconditionally and an odd

@@ -50,3 +50,54 @@ def test_step_attention_matches_oracle(dev, heads, lengths, kv):
         got = runner.step(torch.tensor([[tok]], device=dev), n, n, n + 1)[0, 0].float().cpu().numpy()
         _sync_frozen(ocache, cache, n, S)
         _check_logits(got, model.forward([tok], ocache)[-1], f"{heads} {kv} {n + 1} keys")
+
+
+@pytest.mark.parametrize("heads", [(4, 2, 64), (4, 1, 128)])
+def test_step_attention_keeps_small_weights(dev, heads):
+    """Grouped-query softmax weights stay fp32: keys 2^-22 below the largest, whose values fill dims in which the
+    large keys have none, keep the full precision of the result (weights as fp16 parts keep two bits of them).
+
+    An fp16 model that shows the attention output: the token's normalized row is n0 in coordinate 0, q = n0 / 2 in dim 0
+    of every head, the O projection and the head are the identity, the MLP and the new key are zero, and RoPE does not
+    rotate.  The output, its sum with the residual, the norm's two products and the head round to fp16: 5 x 2^-11."""
+    from axiomlm_amd.cache import StaticKVCache
+    from axiomlm_amd.runner import DecodeRunner
+
+    H, Hkv, hd = heads
+    d, n, S = H * hd, 600, 640
+    z = lambda *s: torch.zeros(*s, dtype=torch.float16, device=dev)  # noqa: E731
+    wte = z(8, d)
+    wte[:, 0] = 1
+    qkv = z(d + 2 * Hkv * hd, d)
+    qkv[0:d:hd, 0] = 0.5
+    qkv[d + Hkv * hd, 0] = 1  # the new value's dim 0: n0 itself, read back from the cache
+    one = torch.ones(d, dtype=torch.float16, device=dev)
+    eye = torch.eye(d, dtype=torch.float16, device=dev)
+    freqs = torch.stack([torch.ones(S, hd // 2), torch.zeros(S, hd // 2)], -1).to(dev)
+    cache = StaticKVCache(1, S, 1, Hkv, hd, device=dev)
+    cache.cache.zero_()
+    g = torch.Generator(device=dev)
+    g.manual_seed(4)
+    low = torch.arange(n, device=dev) % 8 != 0
+    # scores q0 k0 / sqrt(hd) with q0 = sqrt(d) / 2: 0 to 0.5 of the low keys, 15.25 of the others
+    k0 = torch.where(low, torch.rand(n, generator=g, device=dev) * 0.5, 15.25) * 2 / H ** 0.5
+    cache.cache[0, 0, 0, :, :n, 0] = k0.half()
+    v = (torch.rand(Hkv, n, hd, generator=g, device=dev) * 20000 + 10000).half()
+    # each dim from three keys only, so that no two dims share a weight's error
+    pick = torch.rand(Hkv, n, hd, generator=g, device=dev).masked_fill(~low[None, :, None], -1).topk(3, dim=1).indices
+    v = v * z(Hkv, n, hd).scatter_(1, pick, 1)
+    v[:, :, 0] = 0
+    cache.cache[0, 1, 0, :, :n] = v
+    runner = DecodeRunner(wte, freqs, [one], [qkv], [eye], [one], [z(512, d)], [z(d, 256)], one, cache.k_caches,
+                          cache.v_caches, H, Hkv, hd, 1e-5, lm_head_w=eye, kv_dtype="fp16")
+    got = runner.step(torch.zeros(1, 1, dtype=torch.int64, device=dev), n, n, n + 1)[0, 0].double()
+    n0 = cache.cache[0, 1, 0, 0, n, 0].double()
+    kk, vv = cache.cache[0, 0, 0, :, : n + 1, 0].double(), cache.cache[0, 1, 0, :, : n + 1].double()
+    p = torch.softmax(n0 / 2 * kk / hd ** 0.5, -1)
+    o = torch.matmul(p[:, None, :], vv)[:, 0].repeat_interleave(H // Hkv, 0).reshape(-1)
+    x = wte[0].double() + o
+    want = x / (x.square().mean() + 1e-5).sqrt()
+    on = (o > 0) & (want.abs() > 2.0 ** -14)  # (below, fp16 itself has fewer bits)
+    on[::hd] = False
+    assert on.sum() > 0.9 * (d - H)
+    assert ((got - want).abs() <= 5 * 2.0 ** -11 * want.abs())[on].all()
