@@ -1249,10 +1249,19 @@ constexpr int kTreeRows = 64;    // query rows per workgroup (four waves of 16)
 // rescaling path takes the row maxima.  The caller sums l over each row's 16
 // lanes once after the last block.  The quotient o / l does not depend on m; the
 // fp16 weights P keep their relative precision up to 2^kMaxSlack.  PT float: the weights stay fp32.
+// SUM_STORED (prompts): l sums the weights as rounded to fp16, so that the quotient is a mean of values
+// and a dominant key's rounding cancels.  (Prompts in chunks of 32 have more key splits, each with an
+// exact weight at its own maximum: error of a second layer's keys after 300 tokens, 7B shape, 2.244e-3
+// by chunks, 2.247e-3 in one pass with l of the unrounded weights, 2.243e-3 so; same time.)
 constexpr float kMaxSlack = 8.f;
-__device__ __forceinline__ void put_weight(f16* pt, int row, int key, float p) { pt[pt_index(row, key)] = f2h(p); }
-__device__ __forceinline__ void put_weight(float* pt, int row, int key, float p) { pt[pt32_index(row, key)] = p; }
-template <int DT, typename PT>
+// Each stores a weight and returns what it stored.
+__device__ __forceinline__ float put_weight(f16* pt, int row, int key, float p) {
+  return h2f(pt[pt_index(row, key)] = f2h(p));
+}
+__device__ __forceinline__ float put_weight(float* pt, int row, int key, float p) {
+  return pt[pt32_index(row, key)] = p;
+}
+template <bool SUM_STORED, int DT, typename PT>
 __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows, float (&m)[4], float (&l)[4],
                                               f32x4 (&o)[DT], PT* pt, int lq, int l16) {
   if (__builtin_amdgcn_ballot_w64(grows)) {
@@ -1271,9 +1280,12 @@ __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows
     float pr[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) pr[h] = s[v][h] == kNegBig ? 0.f : fast_exp2(s[v][h] - m[v]);
-    l[v] += pr[0] + pr[1];
+    if (!SUM_STORED) l[v] += pr[0] + pr[1];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) put_weight(pt, 4 * lq + v, 16 * h + l16, pr[h]);
+    for (int h = 0; h < 2; ++h) {
+      const float w = put_weight(pt, 4 * lq + v, 16 * h + l16, pr[h]);
+      if (SUM_STORED) l[v] += w;
+    }
   }
 }
 
@@ -1429,7 +1441,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16);
+    softmax_block<CAUSAL>(s2, grows, m, l, o, pt[wave], lq, l16);
     __syncthreads();  // V staged by every wave; P tiles written
     // O += P V: A = P[row l16][keys 8 lq ..], B = V^T[dim 16 d + l16][keys 8 lq ..].
     const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
@@ -1626,7 +1638,7 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block(s2, grows, m, l, o, pt[wave], lq, l16);
+    softmax_block<false>(s2, grows, m, l, o, pt[wave], lq, l16);
     // The wave reads back its own LDS writes: DS operations of one wave complete
     // in order, and the reads below wait for them.
     if constexpr (P32) {

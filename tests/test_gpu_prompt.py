@@ -166,3 +166,42 @@ def _fp16_runner(cfg, ow, cos, sin, dev, S):
                           c_attn_bs=[t(b) for b in (ow.c_attn_b or [])], k_scales=cache.k_scales,
                           v_scales=cache.v_scales, kv_dtype="fp16")
     return runner, cache
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(32, 32, 64), (32, 8, 128)])
+def test_prompt_attention_is_a_mean_of_values(dev, H, Hkv, hd):
+    """Equal values under unequal scores come out as they went in, whatever fp16 makes of the weights: the weights are
+    summed as they are multiplied (2^-22 of the value at most, far below its own rounding).  The first 40 tokens set a
+    maximum that later keys exceed by five to seven powers of two, another amount for each head.
+
+    An fp16 model that shows the attention output in dims 8 and up: embeddings have a one in coordinate 0 (query and
+    value) and in coordinate 1 or 2 (the key's score), the O projection and the head are the identity, the MLP is zero and
+    RoPE does not rotate.  The first token sees its own value only."""
+    from axiomlm_amd.cache import StaticKVCache
+    from axiomlm_amd.runner import DecodeRunner
+
+    d, T, S = H * hd, 600, 640
+    z = lambda *s: torch.zeros(*s, dtype=torch.float16, device=dev)  # noqa: E731
+    wte = z(2, d)
+    wte[:, 0] = 1
+    wte[0, 1] = wte[1, 2] = 1
+    n0 = (d / 2) ** 0.5  # a normalized one
+    qkv = z(d + 2 * Hkv * hd, d)
+    qkv[0:d:hd, 0] = 1 / n0
+    kv = d + Hkv * hd
+    qkv[d:kv:hd, 2] = (torch.linspace(5, 7, Hkv, device=dev) * np.log(2) * hd ** 0.5 / n0).half()
+    qkv[kv:, 0] = 1.97 / n0
+    for h in range(Hkv):
+        qkv[kv + h * hd:kv + h * hd + 8, 0] = 0
+    one = torch.ones(d, dtype=torch.float16, device=dev)
+    eye = torch.eye(d, dtype=torch.float16, device=dev)
+    freqs = torch.stack([torch.ones(S, hd // 2), torch.zeros(S, hd // 2)], -1).to(dev)
+    cache = StaticKVCache(1, S, 1, Hkv, hd, device=dev)
+    runner = DecodeRunner(wte, freqs, [one], [qkv], [eye], [one], [z(512, d)], [z(d, 256)], one, cache.k_caches,
+                          cache.v_caches, H, Hkv, hd, 1e-5, lm_head_w=eye, kv_dtype="fp16")
+    idx = (torch.arange(T, device=dev) >= 40).long()[None]
+    got = runner.prompt_step(idx, 0, 0, "all", 1)[0].view(T, H, hd)[:, :, 8:]
+    v = cache.cache[0, 1, 0, :, :T, 8:]
+    assert (v == v[:, :1]).all() and v.min() > 1.9 and (cache.cache[0, 0, 0, :, 40, 0] > 0).all()
+    assert (got[0] != 0).all()
+    assert (got == got[0]).all(), (got != got[0]).float().mean().item()
