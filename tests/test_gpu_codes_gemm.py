@@ -192,3 +192,25 @@ def test_codes_gemm_few_rows_of_a_large_matrix(dev, fmt):
         for ws in (True, False):
             got = _run(fmt, torch.from_numpy(x[:M]).to(dev), packs, N, None, ws).cpu().numpy()
             assert np.linalg.norm(got.astype(np.float32) - ref[:M]) <= REL * np.linalg.norm(ref[:M]), (M, ws)
+
+
+def test_affine_2bit_infinite_activations(dev):
+    """An infinite activation gives what the few-row kernel gives: infinity where its code is not zero and the group's
+    bias has the code term's sign, else NaN (a zero code, or two infinities of opposite sign)."""
+    rng = np.random.default_rng(8)
+    N, K = 96, 256
+    w = (np.abs(rng.standard_normal((N, K))) * 0.02 + 0.01).astype(np.float16)
+    w[N // 2:] -= np.float16(0.03)  # biases below zero
+    packs = [torch.from_numpy(a).to(dev) for a in fm.pack_linear_q2_k(w)]
+    x = rng.standard_normal((80, K)).astype(np.float16)
+    x[3, 70], x[5, 200], x[64, 1], x[79, 255] = np.inf, -np.inf, np.inf, np.inf
+    xd = torch.from_numpy(x).to(dev)
+    got = _run("q2", xd, packs, N).cpu().numpy()
+    few = np.concatenate([_run("q2", xd[m:m + 16], packs, N).cpu().numpy() for m in range(0, 80, 16)])
+    bad = np.array([3, 5, 64, 79])
+    assert np.isinf(few[bad, :N // 2]).any() and np.isnan(few[bad]).any()
+    assert np.array_equal(np.isnan(got), np.isnan(few))
+    inf = np.isinf(few)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], few[inf])
+    keep = np.setdiff1d(np.arange(80), bad)
+    assert np.isfinite(got[keep]).all()
