@@ -314,12 +314,14 @@ __global__ void __launch_bounds__(kCThreads, 2) codes_gemm_kernel(T16Args a, int
       load_w(2 * s + 3, std::integral_constant<int, 3 - 2 * b>{});
     }
     if constexpr (b == 0 && !kPlain) {
-      // A pair of stages begins: its scales and codes are there, the next pair's are requested.
+      // A pair of stages begins: its scales and codes are there, the next pair's are requested.  Past
+      // K the scale is zero, not the last group's again, which may be infinite.
+      const uint32_t in_k = 2 * s + kq < n_grp ? ~0u : 0u;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        sv[t] = sn[t];
+        sv[t] = sn[t] & in_k;
         if constexpr (!kRing) cv[t] = lane_transpose(cn[t]);
-        if (kBias) bb[t] = 2 * s + kq < n_grp ? sv[t] >> 16 : 0u;
+        if (kBias) bb[t] = sv[t] >> 16;
       }
       load_pair((s >> 1) + 1);
     }

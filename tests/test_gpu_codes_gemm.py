@@ -214,3 +214,18 @@ def test_affine_2bit_infinite_activations(dev):
     assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], few[inf])
     keep = np.setdiff1d(np.arange(80), bad)
     assert np.isfinite(got[keep]).all()
+
+
+def test_infinite_scale_of_a_last_half_stage(dev):
+    """K % 128 == 64: the half stage past K adds nothing, also to rows whose last scale is infinite."""
+    rng = np.random.default_rng(9)
+    N, K = 40, 320
+    packs = list(_packed("ternary", rng, N, K)[0])
+    packs[1] = packs[1].copy()
+    packs[1].reshape(N, K // 64)[7, -1] = np.inf
+    packs = [torch.from_numpy(a).to(dev) for a in packs]
+    xd = torch.from_numpy(rng.standard_normal((80, K)).astype(np.float16)).to(dev)
+    got = _run("ternary", xd, packs, N).cpu().numpy()
+    few = np.concatenate([_run("ternary", xd[m:m + 16], packs, N).cpu().numpy() for m in range(0, 80, 16)])
+    assert np.isinf(few[:, 7]).all() and np.array_equal(got[:, 7], few[:, 7])
+    assert np.isfinite(np.delete(got, 7, 1)).all()
