@@ -23,6 +23,7 @@
 #include "axm.h"
 #include "codes_gemm.h"
 #include "kernels.h"
+#include "step_attn.h"
 #include "step_kernel.h"
 #include "q4_tile16.h"
 
@@ -470,15 +471,7 @@ struct axm_runner {
     return v;
   }
 
-  // How a one-token step over active_len keys runs its attention: key splits (bucketed, so
-  // that one graph covers a range of lengths), splits of at most 64 keys on a smaller launch
-  // shape, and whether the split partials stay for the O projection to merge while staging its
-  // activations (parts) or a reduce launch merges them.
-  struct StepAttn {
-    int splits;
-    bool short_splits, parts;
-    int key() const { return 4 * splits + (parts ? 2 : 0) + (short_splits ? 1 : 0); }
-  };
+  // How a one-token step over active_len keys runs its attention.
   StepAttn step_attn(int active_len) const {
     int want = attn_step_splits(d.n_head, d.n_kv_head, active_len);
     bool parts = false;
@@ -487,10 +480,7 @@ struct axm_runner {
                       : attn_choose_splits(1, d.n_kv_head, active_len);
       parts = parts_ok && want > 1;
     }
-    int bucket = 1;
-    while (bucket < want) bucket <<= 1;
-    if (bucket > max_splits) bucket = max_splits;
-    return {bucket, active_len <= 64 * bucket, parts};
+    return step_attn_of(want, parts, max_splits, active_len);
   }
 
   // Enqueue the whole single-token step on stream s (no host synchronization).
@@ -1269,7 +1259,7 @@ extern "C" int axm_runner_step(axm_runner_t r, const void* idx_dev, int64_t tok_
   const EmbedArgs emb{d.wte, (const f16*)d.wte_sb, d.wte_format, d.d_model, d.vocab_size, r->x};
   hipLaunchKernelGGL(set_params_kernel, dim3(1), dim3(256), 0, s, r->params, (const int64_t*)idx_dev, tok_host,
                      rope_pos, write_pos, active_len, r->argmax_keys, (d.vocab_size + 7) / 8, emb);
-  const axm_runner::StepAttn at = r->step_attn(active_len);
+  const StepAttn at = r->step_attn(active_len);
   const int key = at.key();
   if (r->mode == AXM_RUNNER_MODE_EAGER) {
     int rc = r->enqueue_step(at, s);
@@ -1324,7 +1314,7 @@ extern "C" int axm_runner_time_kernels(axm_runner_t r, int position, int active_
   const EmbedArgs emb{d.wte, (const f16*)d.wte_sb, d.wte_format, d.d_model, d.vocab_size, r->x};
   hipLaunchKernelGGL(set_params_kernel, dim3(1), dim3(256), 0, s, r->params, (const int64_t*)nullptr, (int64_t)0,
                      position % d.rope_len, position, active_len, r->argmax_keys, (d.vocab_size + 7) / 8, emb);
-  const axm_runner::StepAttn at = r->step_attn(active_len);
+  const StepAttn at = r->step_attn(active_len);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
     if (e0) (void)hipEventDestroy(e0);

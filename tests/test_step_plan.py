@@ -27,3 +27,13 @@ def test_step_plan_offsets_in_bounds_under_asan(tmp_path):
     res = subprocess.run([exe], capture_output=True, text=True, timeout=600)
     assert res.returncode == 0, res.stdout + res.stderr
     assert res.stdout.count("ok ") == 7, res.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_step_graph_keys_differ_only_with_the_launches(tmp_path):
+    """A graph is captured inside the first step that needs it: lengths that enqueue the same launches share one."""
+    exe = str(tmp_path / "step_attn_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", f"-I{INC}", os.path.join(ROOT, "tests", "cpu", "step_attn_check.cpp"),
+                    "-o", exe], check=True)
+    res = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert res.returncode == 0, res.stdout + res.stderr
