@@ -155,7 +155,7 @@ def qmv_q4_marlin(x, w_marlin, sb_marlin, out_features: int | None = None, bias=
     b = None
     if bias is not None:
         b = bias.to(device=x.device, dtype=torch.float16).contiguous()
-    if M == 1 or (M <= 4 and N * K < 32 << 20):  # the GEMV
+    if M == 1 or (M <= 4 and N * K < 32 << 20):  # the GEMV (the rule of marlin_rows_use_codes, checked by a test)
         _lib.check(_lib.lib().axm_qmv_q4_marlin(_lib.ptr(xc), _lib.ptr(w_marlin.contiguous()),
                                                 _lib.ptr(sb_marlin.contiguous()), _lib.ptr(b), _lib.ptr(y), M, K, N,
                                                 _lib.stream_of(x.device)),

@@ -168,6 +168,59 @@ def _fp16_runner(cfg, ow, cos, sin, dev, S):
     return runner, cache
 
 
+# 33: 48-row tiles; 64: one block of 64; 75 and 150: several blocks with a ragged last one; with heads of 128 the QKV
+# splits are summed by the RoPE launch; SwiGLU and residual epilogues (fused with the norm) of split and unsplit K.
+@pytest.mark.parametrize("mode,kv,hd", [("q8", "fp16", 64), ("q8", "fp16", 128), ("q8", "fp8", 128),
+                                        ("q4_k_m", "fp16", 128)])
+@pytest.mark.parametrize("T,past", [(33, 0), (64, 20), (75, 7), (150, 0)])
+def test_q8_prompt_matches_oracle(dev, mode, kv, hd, T, past):
+    print(f"[q8_prompt] {mode} kv={kv} hd={hd} T={T} past={past}", flush=True)
+    cfg = om.OracleConfig(n_layer=2, n_head=512 // hd, n_kv_head=256 // hd, d_model=512, hidden=1408, vocab=1000,
+                          eps=1e-5, block_size=256)
+    ow = om.pack_model(cfg, om.make_float_weights(cfg, seed=6), mode)
+    cos, sin = om.rope_tables(cfg.head_dim, cfg.block_size)
+    model = om.OracleModel(cfg, ow, cos, sin)
+    S = 192
+    runner, cache = build_runner(cfg, ow, cos, sin, dev, S, kv)
+    ocache = om.OracleKVCache(S, cfg.n_layer, cfg.n_kv_head, cfg.head_dim, kv)
+    ocache.frozen = kv != "fp16"
+    rng = np.random.default_rng(T + past)
+    prefix = rng.integers(0, cfg.vocab, past).tolist()
+    if ocache.frozen:
+        run_steps(runner, cache, prefix, dev)
+    else:
+        _prefill(runner, cache, ocache, model, prefix, dev)
+    toks = rng.integers(0, cfg.vocab, T).tolist()
+    got = runner.prompt_step(torch.tensor([toks], device=dev), past, past, "all", 1)[0].float().cpu().numpy()
+    if ocache.frozen:
+        _sync_frozen(ocache, cache, past, S)
+    ref = model.forward(toks, ocache, return_all_logits=True)
+    for t in range(T):
+        _check_logits(got[t], ref[t], f"{mode} prompt token {t} of {T}")
+    if ocache.frozen:
+        _check_codes(kv, _code_diffs(kv, ocache), f"{mode} prompt T={T}")
+
+
+@pytest.mark.parametrize("mode", ["q4_rtn", "q8"])
+def test_long_prompt_equals_verify_chunks(dev, mode):
+    """700 tokens: many row blocks of the GEMMs, split K with the residual and norm reduced together, causal attention
+    of many row blocks; against verify chunks of 32 tokens, both within the oracle bar of the same values."""
+    cfg = om.OracleConfig(n_layer=2, n_head=8, n_kv_head=2, d_model=1024, hidden=2816, vocab=1000, eps=1e-5,
+                          block_size=1024)
+    ow = om.pack_model(cfg, om.make_float_weights(cfg, seed=8), mode)
+    cos, sin = om.rope_tables(cfg.head_dim, cfg.block_size)
+    T = 700
+    idx = torch.from_numpy(np.random.default_rng(3).integers(0, cfg.vocab, (1, T))).to(dev)
+    runner, cache = build_runner(cfg, ow, cos, sin, dev, 768)
+    got = runner.prompt_step(idx, 0, 0, "all", 1)[0].float()
+    runner2, cache2 = build_runner(cfg, ow, cos, sin, dev, 768)
+    for t0 in range(0, T, 32):
+        n = min(32, T - t0)
+        ref = runner2.verify_step(idx[:, t0:t0 + n], t0, t0, t0 + n)[0].float()
+        assert (got[t0:t0 + n] - ref).abs().max().item() <= 2 * TOL, f"tokens {t0}.."
+    assert (cache.cache[..., :T, :].float() - cache2.cache[..., :T, :].float()).abs().max().item() <= 2e-2
+
+
 @pytest.mark.parametrize("H,Hkv,hd", [(32, 32, 64), (32, 8, 128)])
 def test_prompt_attention_is_a_mean_of_values(dev, H, Hkv, hd):
     """Equal values under unequal scores come out as they went in, whatever fp16 makes of the weights: the weights are

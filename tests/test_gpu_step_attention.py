@@ -23,7 +23,9 @@ GQA = [0, 1, 3, 31, 32, 127, 512, 513, 1025, 2100]
 
 
 @pytest.mark.parametrize("heads,lengths", [((4, 2, 64), GQA), ((8, 2, 128), GQA), ((16, 1, 64), GQA),
-                                           ((4, 4, 64), [7998, 7999, 8100])])
+                                           ((4, 4, 64), [7998, 7999, 8100]),
+                                           # more than sixteen query heads per KV head: the vector kernel
+                                           ((32, 1, 64), [0, 40, 600, 8010])])
 @pytest.mark.parametrize("kv", ["fp16", "fp8", "int4"])
 def test_step_attention_matches_oracle(dev, heads, lengths, kv):
     cfg, ow, cos, sin = _model(*heads)

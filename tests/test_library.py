@@ -65,3 +65,22 @@ def test_many_row_workspace_covers_the_64_row_passes():
             one = L.axm_qmm_q4_tile16_workspace_bytes(K, N, swiglu)
             assert L.axm_qmm_q4_tile16_rows_workspace_bytes(M, K, N, swiglu) >= one
             assert L.axm_qmm_q4_tile16_rows_workspace_bytes(64, K, N, swiglu) == one
+
+
+def test_wrappers_skip_the_several_row_entry_only_where_it_would_run_the_gemv():
+    # The Python products call the GEMV entry without a workspace query up to these rows; the rows from
+    # which the library takes the several-row kernel are its own (a workspace is asked for only then, and these
+    # shapes split K there).
+    from axiomlm_amd import _lib
+
+    L = _lib.lib()
+    q8, affine, ternary, gguf, marlin = range(5)
+    for N, K in [(512, 4096), (1024, 11008), (4096, 4096)]:
+        for fmt in (q8, marlin):
+            assert L.axm_qmm_codes_workspace_bytes(fmt, 5, K, N) > 0
+        for fmt in (q8, affine, ternary, gguf, marlin):
+            for M in range(1, 5):
+                assert L.axm_qmm_codes_workspace_bytes(fmt, M, K, N) == 0
+    for M in range(1, 5):  # MARLIN from 32 Mi weights on: two rows
+        assert (L.axm_qmm_codes_workspace_bytes(marlin, M, 32768, 1024) > 0) == (M > 1)
+        assert L.axm_qmm_codes_workspace_bytes(marlin, M, 32768, 1016) == 0
