@@ -565,7 +565,9 @@ __global__ void __launch_bounds__(kCThreads, 2) q2k_gemm_kernel(T16Args a, int n
           for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_fdot2(as_h2(x[e]), one, v, false);
         }
         const uint32_t s0 = __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u;
-        const float r1 = v - __builtin_bit_cast(float, s0);
+        // (At most 2^13; an infinite sum's rest, a NaN, becomes any number: the sum's products with the
+        // mins are infinite, as in the few-row kernel.  A branch as in codes_gemm_kernel cost 2 %.)
+        const float r1 = __builtin_fminf(v - __builtin_bit_cast(float, s0), 0x1p20f);
         const uint32_t s1 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
         const uint32_t s2 = __builtin_bit_cast(uint32_t, r1 - __builtin_bit_cast(float, s1));
         sx[b][p] = u32x2{(s0 >> 16) | s1, s2 >> 16};

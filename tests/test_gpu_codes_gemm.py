@@ -229,3 +229,23 @@ def test_infinite_scale_of_a_last_half_stage(dev):
     few = np.concatenate([_run("ternary", xd[m:m + 16], packs, N).cpu().numpy() for m in range(0, 80, 16)])
     assert np.isinf(few[:, 7]).all() and np.array_equal(got[:, 7], few[:, 7])
     assert np.isfinite(np.delete(got, 7, 1)).all()
+
+
+def test_gguf_infinite_activations(dev):
+    """The same of GGUF blocks, whose two terms have one sign only where d and dmin have opposite ones."""
+    rng = np.random.default_rng(10)
+    N, K = 96, 512
+    blocks = fm.pack_q2_k_gguf((rng.standard_normal((N, K)) * 0.02).astype(np.float16))
+    blocks[N // 2:, :, 83] ^= 0x80  # dmin < 0
+    packs = [torch.from_numpy(blocks).to(dev)]
+    x = rng.standard_normal((80, K)).astype(np.float16)
+    x[3, 70], x[5, 200], x[64, 300], x[79, 511] = np.inf, -np.inf, np.inf, np.inf
+    xd = torch.from_numpy(x).to(dev)
+    got = _run("gguf", xd, packs, N).cpu().numpy()
+    few = np.concatenate([_run("gguf", xd[m:m + 16], packs, N).cpu().numpy() for m in range(0, 80, 16)])
+    bad = np.array([3, 5, 64, 79])
+    assert np.isinf(few[bad, N // 2:]).any() and np.isnan(few[bad]).any()
+    assert np.array_equal(np.isnan(got), np.isnan(few))
+    inf = np.isinf(few)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], few[inf])
+    assert np.isfinite(np.delete(got, bad, 0)).all()
