@@ -1371,6 +1371,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
   // D-tile rows of this lane: row0 + 4 lq + v.
   uint64_t mask[4];
   int key_end[4];  // CAUSAL: keys the row sees
+  // CAUSAL: keys that some row of the wave sees.  Values past them are left out of P V, where a zero
+  // weight would not keep a value that is not finite from the tokens before its own 16 rows.
+  const int wave_end = __builtin_amdgcn_readfirstlane(CAUSAL ? prefix + min(row0 + 15, R - 1) / p.n_rep + 1 : 0);
   bool row_ok[4];
   float m[4], l[4];
   f32x4 o[DT];
@@ -1445,11 +1448,23 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
     __syncthreads();  // V staged by every wave; P tiles written
     // O += P V: A = P[row l16][keys 8 lq ..], B = V^T[dim 16 d + l16][keys 8 lq ..].
     const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
+    auto add_pv = [&](auto masked) {
+      u32x4 keep;
+      if constexpr (decltype(masked)::value) {
+        const int n = wave_end - kb0 - 8 * lq;
 #pragma unroll
-    for (int d = 0; d < DT; ++d) {
-      const f16x8 vb = v_operand(&vr[16 * d], VROW, l16, lq);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[d], 0, 0, 0);
-    }
+        for (int i = 0; i < 4; ++i) keep[i] = (n > 2 * i ? 0xFFFFu : 0u) | (n > 2 * i + 1 ? 0xFFFF0000u : 0u);
+      }
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        f16x8 vb = v_operand(&vr[16 * d], VROW, l16, lq);
+        if constexpr (decltype(masked)::value)
+          vb = __builtin_bit_cast(f16x8, __builtin_bit_cast(u32x4, vb) & keep);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, vb, o[d], 0, 0, 0);
+      }
+    };
+    if (!CAUSAL || kb0 + kTreeKeys <= wave_end) add_pv(std::false_type{});
+    else if (kb0 < wave_end) add_pv(std::true_type{});
     __syncthreads();  // before the next block overwrites vt / pt
   };
   // Both blocks of an iteration run unconditionally and an odd last block is peeled

@@ -258,3 +258,28 @@ def test_prompt_attention_is_a_mean_of_values(dev, H, Hkv, hd):
     assert (v == v[:, :1]).all() and v.min() > 1.9 and (cache.cache[0, 0, 0, :, 40, 0] > 0).all()
     assert (got[0] != 0).all()
     assert (got == got[0]).all(), (got != got[0]).float().mean().item()
+
+
+# Row blocks of 64 tokens, whose second half starts at token 32; keys aligned to the blocks of 32 and not.
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("past", [0, 7])
+@pytest.mark.parametrize("at", [32, 47, 75])
+def test_token_that_is_not_finite_leaves_earlier_tokens_alone(dev, heads, past, at):
+    """A token whose keys and values are NaN reaches no token before its own 16, in any layer."""
+    cfg = om.OracleConfig(n_layer=2, n_head=heads, n_kv_head=heads, d_model=256, hidden=704, vocab=1000, eps=1e-5,
+                          block_size=256)
+    ow = om.fp16_model(cfg, om.make_float_weights(cfg, seed=7))
+    ow.wte_p = ow.wte_p.copy()
+    ow.wte_p[999] = np.inf
+    cos, sin = om.rope_tables(cfg.head_dim, cfg.block_size)
+    toks = torch.from_numpy(np.random.default_rng(at).integers(0, 999, (1, past + 150))).to(dev)
+    out = []
+    for tok in (999, 998):
+        runner, _ = _fp16_runner(cfg, ow, cos, sin, dev, 192)
+        toks[0, past + at] = tok
+        if past:
+            runner.prompt_step(toks[:, :past], 0, 0)
+        out.append(runner.prompt_step(toks[:, past:], past, past, "all", 1)[0].clone())
+    before = at // 16 * 16
+    assert torch.isnan(out[0][at]).all() and torch.isfinite(out[1]).all()
+    assert torch.equal(out[0][:before], out[1][:before])
