@@ -586,7 +586,15 @@ struct AttnParams {
   int write_pos;          // slot of tree node 0
   const uint64_t* masks;  // [T] ancestor bitmasks (tree mode)
   float scale_log2;       // log2(e) / sqrt(hd)
+  int keep_nan;           // decode partials: see split_ml
 };
+
+// The (running max, sum) that a split stores.  The reduce kernels give zeros for a sum that is NaN (a key or
+// query that is not finite), the O projection that merges partials itself gives NaN: keep_nan
+// stores a finite pair instead, beside outputs that are NaN in every dim then.
+__device__ __forceinline__ f32x2 split_ml(const AttnParams& p, float m, float l) {
+  return p.keep_nan && l != l ? f32x2{kNegBig, 1.f} : f32x2{m, l};
+}
 
 // Rows of one workgroup: decode -> (b, kv head, replica r) with r < n_rep;
 // tree -> (node u, kv head, replica) flattened, QR rows per workgroup.
@@ -838,8 +846,9 @@ __global__ void __launch_bounds__(NW * 64) attn_split_kernel(AttnParams p) {
                              : (((row_base + r) / p.n_rep) * p.Hq + kvh * p.n_rep + (row_base + r) % p.n_rep);
       float* dst = p.ws + ((size_t)gr * p.n_splits + split) * (2 + hd);
       if (e == 0) {
-        dst[0] = mm;
-        dst[1] = ll;
+        const f32x2 ml = split_ml(p, mm, ll);
+        dst[0] = ml.x;
+        dst[1] = ml.y;
       }
       dst[2 + e] = oo;
     }
@@ -1133,7 +1142,7 @@ int launch_flash_decode_parts(const f16* q, const KvView& kv, int Hq, int active
 int launch_decode_mfma(const AttnParams& p, dim3 grid, bool p32, hipStream_t s);
 
 int launch_flash_decode(const f16* q, const KvView& kv, f16* out, int Hq, int active_len, const int* active_len_dev,
-                        int n_splits, float* ws, hipStream_t s, bool p32) {
+                        int n_splits, float* ws, hipStream_t s, bool p32, bool keep_nan) {
   AttnParams p{};
   p.q = q;
   p.kv = kv;
@@ -1146,6 +1155,7 @@ int launch_flash_decode(const f16* q, const KvView& kv, f16* out, int Hq, int ac
   p.prefix_dev = active_len_dev;
   p.T = 0;
   p.scale_log2 = kLog2e / sqrtf((float)kv.hd);
+  p.keep_nan = keep_nan;
   int rc;
   if (p.n_rep >= 2 && p.n_rep <= 16 && (kv.hd == 64 || kv.hd == 128)) {
     rc = launch_decode_mfma(p, dim3(kv.B * kv.Hkv, n_splits), p32, s);
@@ -1724,8 +1734,9 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
     } else {
       float* dst = p.ws + (gr * p.n_splits + split) * (2 + HD);
       if (e == 0) {
-        dst[0] = mm;
-        dst[1] = ll;
+        const f32x2 ml = split_ml(p, mm, ll);
+        dst[0] = ml.x;
+        dst[1] = ml.y;
       }
       dst[2 + e] = oo;
     }

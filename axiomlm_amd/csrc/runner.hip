@@ -571,7 +571,8 @@ struct axm_runner {
       return launch_flash_decode_parts(q, kv, d.n_head, 0, params + P_ACTIVE, at.splits, parts_o, parts_ml,
                                        at.short_splits, s);
     // One split (a few keys): fp16 weights, as in the batched decode attention.
-    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, at.splits, ws, s, at.splits > 1);
+    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, at.splits, ws, s, at.splits > 1,
+                               parts_ok);
   }
 
   // 3. O projection, residual add into x.

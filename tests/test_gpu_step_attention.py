@@ -103,3 +103,16 @@ def test_step_attention_keeps_small_weights(dev, heads):
     on[::hd] = False
     assert on.sum() > 0.9 * (d - H)
     assert ((got - want).abs() <= 5 * 2.0 ** -11 * want.abs())[on].all()
+
+
+@pytest.mark.parametrize("heads,n", [((4, 2, 64), 40), ((4, 2, 64), 2100), ((8, 2, 128), 600), ((4, 4, 64), 600),
+                                     ((4, 4, 64), 8010)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_step_over_a_key_that_is_not_finite(dev, heads, n, value):
+    """A cached key of NaN (or of infinite score) makes the step's logits NaN, whichever launch merges the splits."""
+    cfg, ow, cos, sin = _model(*heads)
+    runner, cache = build_runner(cfg, ow, cos, sin, dev, n + 1)
+    cache.cache.normal_()
+    cache.cache[0, 0, 0, :, n // 2] = value
+    got = runner.step(torch.tensor([[3]], device=dev), n, n, n + 1)
+    assert torch.isnan(got).all()
