@@ -9,7 +9,8 @@ enum { kCodesQ8 = 0, kCodesQ2 = 1, kCodesTernary = 2, kCodesQ2kGguf = 3, kCodesM
 // bias) [rows][K / 64][2], ternary [rows][K / 64]), or the MARLIN tiles' (q4_marlin.hip);
 // kCodesF16: plain fp16 weights [rows][K].  SwiGLU and residual epilogues: Q8 and fp16.
 // a.x 16-byte aligned with ldx % 8 == 0; K % 64 == 0; a.N output rows (SwiGLU: gate rows [0, N),
-// up rows [N, 2 N)).  Epilogues, residual norm and split_info as t16_gemm_launch.  K is split as far as ws_bytes allows.
+// up rows [N, 2 N)).  Epilogues, residual norm and split_info as t16_gemm_launch.  K is split as far as
+// ws_bytes allows.
 bool codes_gemm_takes(const void* x, const void* w, const void* sb, int K, int rows, int fmt);
 size_t codes_gemm_ws_bytes(int M, int K, int N, int epi);
 int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s);

@@ -15,9 +15,12 @@
 // Workgroup: four waves, 16 MB rows of x, NT weight tiles of 16 rows per wave.  Lane (row r of a
 // tile, quarter q) holds columns 16 q .. + 15 of a group, so its codes of a group are 16 (Q8) or
 // 4 contiguous bytes; the MFMA's k order is that order of columns, also for the x fragments.
-// Activations go to LDS one 128-column stage ahead as in the many-row tile16 GEMM
+// Activations are requested to LDS one 128-column stage ahead as in the many-row tile16 GEMM
 // (rows_gemm.hip), Q8 codes to registers a stage ahead (64-row tiles: a group), scales and 2-bit
-// codes two stages at a time (load_pair).
+// codes two stages at a time (load_pair).  Only ternary and fp16 weights multiply while those
+// activations are under way: in the forms with a bias term the group sums are a second LDS array (sx), and
+// the compiler, which cannot tell the two apart, waits for the requests before the stage's first
+// LDS read (vmcnt(6) after three LDS and six register loads, 48 rows).
 //
 // Measured (us, graph of back-to-back calls, against the GEMVs of up to 4 / 16 rows a launch):
 // Q8 12288 x 4096, 16 rows 67 -> 21, 64 rows 244 -> 28, 1000 rows -> 177 (569 TFLOP/s); ternary 64
@@ -776,7 +779,8 @@ size_t codes_gemm_ws_bytes(int M, int K, int N, int epi) {
 int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s) {
   const int rows = epi == Q4_EPI_SWIGLU ? 2 * a.N : a.N;
   if (M < 1 || !codes_gemm_takes(a.x, a.w16, a.sb16, a.K, rows, fmt) || a.ldx % 8 != 0 || a.ln_w != nullptr ||
-      (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) || (fmt != kCodesQ8 && fmt != kCodesF16 && epi != Q4_EPI_STORE) ||
+      (epi != Q4_EPI_STORE && epi != Q4_EPI_RESID && epi != Q4_EPI_SWIGLU) ||
+      (fmt != kCodesQ8 && fmt != kCodesF16 && epi != Q4_EPI_STORE) ||
       (a.post_ln_w != nullptr && (epi != Q4_EPI_RESID || a.post_norm_out == nullptr || a.ldr != a.N))) {
     axm_set_error("codes gemm: format %d, M=%d, epi=%d, K=%d unsupported", fmt, M, epi, a.K);
     return -2;

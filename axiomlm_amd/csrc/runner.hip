@@ -641,13 +641,14 @@ struct axm_runner {
   };
   RowBufs own_bufs() const { return {x, norm, q, attn_y, hbuf, qkvbuf, kvst, tree_pos, ws, ws_bytes}; }
 
-  // Q8_G64 (format 1) or fp16 (format 2) lm_head over T rows into logits: with ln_w the
-  // GEMV applies the final RMSNorm itself and writes the normalized rows to xn_out (one
-  // launch where a separate norm took two); without, the rows are normalized already.
   // The several-row GEMM's format and fewest rows for a Q8_G64 (fmt 1) or fp16 (fmt 2) matrix.
   static int dense_codes(int fmt) { return fmt == 1 ? kCodesQ8 : kCodesF16; }
   static int dense_min_rows(int fmt) { return fmt == 1 ? kCodesQ8MinRows : kCodesF16MinRows; }
 
+  // Q8_G64 (format 1) or fp16 (format 2) lm_head over T rows into out (null: logits): with ln_w the
+  // GEMV applies the final RMSNorm itself and writes the normalized rows to xn_out (one
+  // launch where a separate norm took two); without, the rows are normalized already, and enough
+  // of them go through the several-row GEMM, whose split-K workspace is b's.
   int lm_head_dense(const f16* x, int T, const f16* ln_w, f16* xn_out, hipStream_t s, f16* out = nullptr,
                     const RowBufs* b = nullptr) {
     if (out == nullptr) out = logits;
@@ -730,13 +731,14 @@ struct axm_runner {
     return m.fmt != 0 ? run_dense(m, epi, out_rows, c, M, s) : run_gemv(m, epi, out_rows, c, M, s);
   }
 
-  // GEMV over T token rows in launches of at most 4 rows, or the multi-token GEMM
-  // from kGemmMinTokens rows on.
+  // A product over T token rows.  tile16 matrices: the multi-token GEMM from kGemmMinTokens rows on, the
+  // many-row GEMM from 65.  Q8_G64 and fp16 ones: the several-row GEMM from dense_min_rows on.  Else
+  // the GEMV in launches of at most 4 rows.
   int gemv_rows(const RowBufs& b, const Mat& m, int epi, int out_rows, GemvCall c, int T, hipStream_t s) {
     if (m.w16 != nullptr && T >= kGemmMinTokens && c.argmax_keys == nullptr && c.q_dim == 0 &&
         (epi == Q4_EPI_STORE || epi == Q4_EPI_RESID || epi == Q4_EPI_SWIGLU)) {
-      // Multi-token GEMM: up to 64 tokens per weight pass, activations normalized first
-      // (into x_norm_out when the caller wants them, else into the norm scratch).
+      // All tokens in one pass over the weights, activations normalized first (into x_norm_out
+      // when the caller wants them, else into the norm scratch).
       const f16* xall = c.x;
       if (c.ln_w != nullptr) {
         f16* nrm = c.x_norm_out ? c.x_norm_out : b.norm;
@@ -963,15 +965,15 @@ struct axm_runner {
     r.qkvbuf = (f16*)take((size_t)T * qkv_dim * h);
     r.kvst = (f16*)take(d.head_dim == 128 ? 0 : (size_t)T * 2 * kv_dim * h);
     r.pos = (int*)take((size_t)T * sizeof(int));
-    // Attention partials and GEMM partial tiles share one region.  The split count falls
-    // with the number of keys, so the longest prefix bounds it.
+    // Attention partials and GEMM partial tiles share one region.  The split count grows
+    // with the number of keys, so a full cache bounds it.
     size_t w = tree_workspace_bytes(T, d.n_head, d.head_dim,
                                     tree_choose_splits(T, d.n_head, d.n_kv_head, d.max_seq_len));
     auto gemm = [&](const Mat& m, int rows, int epi) {
       if (m.w16 == nullptr && m.fmt == 0) return;
       const size_t g = m.fmt != 0 ? codes_gemm_ws_bytes(T, m.K, rows, epi)
                        : T > kTile16GemmMaxTokens ? t16_rows_gemm_ws_bytes(T, m.K, (rows + 15) / 16, epi)
-                                                : t16_gemm_ws_bytes(m.K, (rows + 15) / 16, epi == Q4_EPI_SWIGLU ? 2 : 1);
+                                                  : t16_gemm_ws_bytes(m.K, (rows + 15) / 16, epi == Q4_EPI_SWIGLU ? 2 : 1);
       w = g > w ? g : w;
     };
     gemm(m_qkv[0], qkv_dim, Q4_EPI_STORE);

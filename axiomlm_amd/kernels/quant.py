@@ -215,8 +215,8 @@ TILE16_GEMM_MIN_ROWS = 4
 
 def qmv_q4_tile16(x, w16, sb16, out_features: int, bias=None) -> torch.Tensor:
     """y = x @ W^T (+ bias) on a tile16 copy made by :func:`repack_q4_marlin_tile16`: the
-    decode GEMV for up to three rows, the multi-token GEMM (up to 64 rows per weight pass)
-    from four."""
+    decode GEMV for up to three rows, the multi-token GEMM from four, one launch of the
+    many-row GEMM from 65."""
     _lib.require_gpu(x, "qmv_q4_tile16")
     K = x.size(-1)
     M = x.numel() // K

@@ -65,8 +65,9 @@ def _run(fmt, x, packs, N, bias=None, ws=True):
     return y
 
 
-# Row tiles of 16 - 64 with remainders, two and four weight tiles per wave (the last: four), several row blocks, weight tiles past N, one and two stages, odd and even
-# counts, half a stage, split and unsplit K; 2-bit sizes beyond what their GEMV launches take.
+# Row tiles of 16 - 64 with remainders, two and four weight tiles per wave (the last: four), several row blocks, weight
+# tiles past N, one and two stages, odd and even counts, half a stage, split and unsplit K; 2-bit sizes beyond what their
+# GEMV launches take.
 SHAPES = [(5, 16, 64), (7, 24, 192), (16, 1000, 704), (33, 72, 128), (48, 264, 4096), (64, 96, 8192), (70, 130, 320),
           (129, 2056, 1024), (17, 40, 192),
           (930, 12280, 128)]
