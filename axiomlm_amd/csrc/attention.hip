@@ -1271,9 +1271,10 @@ __device__ __forceinline__ float put_weight(f16* pt, int row, int key, float p) 
 __device__ __forceinline__ float put_weight(float* pt, int row, int key, float p) {
   return pt[pt32_index(row, key)] = p;
 }
-template <bool SUM_STORED, int DT, typename PT>
+// rescale(v, alpha) multiplies the outputs of row 4 lq + v (alpha: the same in the row's 16 lanes).
+template <bool SUM_STORED, typename PT, typename F>
 __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows, float (&m)[4], float (&l)[4],
-                                              f32x4 (&o)[DT], PT* pt, int lq, int l16) {
+                                              const F& rescale, PT* pt, int lq, int l16) {
   if (__builtin_amdgcn_ballot_w64(grows)) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1281,8 +1282,7 @@ __device__ __forceinline__ void softmax_block(const float (&s)[4][2], bool grows
       const float alpha = fast_exp2(m[v] - m_new);
       m[v] = m_new;
       l[v] *= alpha;
-#pragma unroll
-      for (int d = 0; d < DT; ++d) o[d][v] *= alpha;
+      rescale(v, alpha);
     }
   }
 #pragma unroll
@@ -1454,7 +1454,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) t
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block<CAUSAL>(s2, grows, m, l, o, pt[wave], lq, l16);
+    softmax_block<CAUSAL>(s2, grows, m, l, [&](int v, float alpha) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d][v] *= alpha;
+    }, pt[wave], lq, l16);
     __syncthreads();  // V staged by every wave; P tiles written
     // O += P V: A = P[row l16][keys 8 lq ..], B = V^T[dim 16 d + l16][keys 8 lq ..].
     const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
@@ -1537,20 +1540,31 @@ int launch_tree_mfma(const AttnParams& p, dim3 grid, hipStream_t s) {
 // (wave-private transposed V and P tiles, no barrier in the loop) and merge
 // their (m, l, o) through LDS at the end.
 // ---------------------------------------------------------------------------
-// P32: the weights stay fp32 as in the vector kernel, and P V runs on the fp32 matrix instruction
-// (16x16x4): lane (l16, lq) holds keys 8 lq .. + 7 of its row of P and of its column of V, so
-// step s takes key 8 lq + s of each quarter, and V goes in as the fp16 operand reads it, widened.
-// (Weights as two fp16 parts, one more fp16 MFMA per tile, took 1.9 us less per layer at 6000 FP8
-// keys of 8 KV heads and 5 at 16000, but weights below 2^-14 of the largest lost bits to fp16's
-// range, those below 2^-25 all of them, and an infinite value times a zero part was NaN.)
-template <int KVT, int HD, bool P32>
-__global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParams p) {
+// RG > 0: the weights stay fp32 as in the vector kernel, and P V runs on the fp32 matrix instruction that
+// multiplies 4 rows by 64 columns and one k (4x4x1, 16 blocks; one key of 128 dims takes two), RG of them
+// for up to 4 RG query rows.  A lane holds two neighbouring dims of V (heads of 64: of every other key, by
+// wave half) and, of P, row lane % 4 of key lane / 4: the broadcast modifier hands key k's
+// rows to all blocks.  With the 16-row form (16x16x4, three quarters of it idle at four rows) a block
+// of 32 keys took four times the matrix cycles (us per layer at 8 KV heads of 128, 4 rows each, 16x16x4 /
+// this: fp16 6000 keys 50.3 / 49.4, 12000 keys 53.9 / 52.8; FP8 52.5 / 51.4, 55.7 / 54.4); weights as two fp16
+// parts (50.4, 52.8 of FP8) lose bits below 2^-14 of the largest to fp16's range, those below 2^-25 all of
+// them, and an infinite value times a zero part is NaN.
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(const F& f) {
+  if constexpr (N > 0) {
+    unrolled<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+template <int KVT, int HD, int RG>
+__global__ void __launch_bounds__(256, RG ? 2 : 1) decode_mfma_kernel(AttnParams p) {
   constexpr int KSTEPS = HD / 32;
   constexpr int DT = HD / 16;
   constexpr int kVPL = kTreeKeys * HD / 8 / 64;  // 8-element V vectors per lane and block
   // V rows as stored (key-major, padded rows) for the transposing LDS reads.
   constexpr int VROW = HD + 16;
   __shared__ __align__(16) f16 vr[4][kTreeKeys * VROW];
+  constexpr bool P32 = RG > 0;
   using PT = typename std::conditional<P32, float, f16>::type;
   __shared__ __align__(16) PT pt[4][16 * kTreeKeys];
   __shared__ float mrg[4][16][2 + HD];
@@ -1620,6 +1634,15 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
   }
 #pragma unroll
   for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // P32: rows 4 g .. + 3 of the lane's two dims, in NP alternating sums.
+  constexpr int NP = RG == 1 ? 2 : 1;
+  f32x4 ow[P32 ? RG : 1][2][NP];
+#pragma unroll
+  for (int g = 0; g < RG; ++g)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int i = 0; i < NP; ++i) ow[g][c][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   // The first key blocks are requested after the query rows: loads complete in
   // order, so the loop's waits for a key block also cover the query loads
   // (requested last, they made every iteration wait for all loads in flight).
@@ -1663,19 +1686,45 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
         s2[v][h] = vis ? sc[h][v] * p.scale_log2 : kNegBig;
         grows |= s2[v][h] > m[v] + kMaxSlack;
       }
-    softmax_block<false>(s2, grows, m, l, o, pt[wave], lq, l16);
+    softmax_block<false>(s2, grows, m, l, [&](int v, float alpha) {
+      if constexpr (P32) {
+#pragma unroll
+        for (int g = 0; g < RG; ++g) {
+          const float ag =
+              __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, alpha), 16 * g));
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int i = 0; i < NP; ++i) ow[g][c][i][v] *= ag;
+        }
+      } else {
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[d][v] *= alpha;
+      }
+    }, pt[wave], lq, l16);
     // The wave reads back its own LDS writes: DS operations of one wave complete
     // in order, and the reads below wait for them.
     if constexpr (P32) {
-      f32x4 pa[2];
+      // Half t of the block's keys: matrix step k takes key 16 t + k (heads of 64: 16 t + 2 k in the wave's
+      // first half, the key after it in the second).
+      constexpr int kSteps = HD == 128 ? 16 : 8;
+      const int pkey = HD == 128 ? lane >> 2 : 2 * ((lane >> 2) & 7) + (lane >> 5);
+      const f16* vl = &vr[wave][HD == 128 ? 2 * lane : (lane >> 5) * VROW + 2 * (lane & 31)];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) pa[i] = *reinterpret_cast<const f32x4*>(&pt[wave][pt32_index(l16, 8 * lq + 4 * i)]);
+      for (int t = 0; t < 2; ++t) {
+        float pa[RG];
 #pragma unroll
-      for (int d = 0; d < DT; ++d) {
-        const f16x8 vb = v_operand(&vr[wave][16 * d], VROW, l16, lq);
+        for (int g = 0; g < RG; ++g) pa[g] = pt[wave][pt32_index(4 * g + (lane & 3), 16 * t + pkey)];
+        unrolled<kSteps>([&](auto kc) {
+          constexpr int k = decltype(kc)::value;
+          const f16x2 vb = *reinterpret_cast<const f16x2*>(vl + (16 * t + 16 / kSteps * k) * VROW);
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[k >> 2][k & 3], h2f(vb[k]), o[d], 0, 0, 0);
+          for (int g = 0; g < RG; ++g)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+              ow[g][c][k % NP] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa[g], h2f(vb[c]), ow[g][c][k % NP],
+                                                                    HD == 128 ? 4 : 3, k, 0);
+        });
       }
     } else {
       const f16x8 pa = *reinterpret_cast<const f16x8*>(&pt[wave][pt_at(l16, 8 * lq)]);
@@ -1712,8 +1761,25 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
       mrg[wave][row][1] = l[v];
     }
     // Output column l16 of tile d is dim 16 d + kv_col_dim<KVT>(l16).
+    if constexpr (!P32) {
 #pragma unroll
-    for (int d = 0; d < DT; ++d) mrg[wave][row][2 + 16 * d + kv_col_dim<KVT>(l16)] = o[d][v];
+      for (int d = 0; d < DT; ++d) mrg[wave][row][2 + 16 * d + kv_col_dim<KVT>(l16)] = o[d][v];
+    }
+  }
+  if constexpr (P32) {
+#pragma unroll
+    for (int g = 0; g < RG; ++g)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int pos = 2 * (HD == 128 ? lane : lane & 31) + c;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float x = ow[g][c][0][v];
+          if constexpr (NP == 2) x += ow[g][c][1][v];
+          if constexpr (HD == 64) x += __shfl_xor(x, 32, 64);
+          mrg[wave][4 * g + v][2 + (pos & ~15) + kv_col_dim<KVT>(pos & 15)] = x;
+        }
+      }
   }
   __syncthreads();
   for (int t = threadIdx.x; t < R * HD; t += 256) {
@@ -1745,8 +1811,10 @@ __global__ void __launch_bounds__(256, P32 ? 2 : 1) decode_mfma_kernel(AttnParam
 
 template <int KVT, int HD>
 void launch_decode_mfma_p(const AttnParams& p, dim3 grid, bool p32, hipStream_t s) {
-  if (p32) hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, true>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, false>), grid, dim3(256), 0, s, p);
+  if (!p32) hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, 0>), grid, dim3(256), 0, s, p);
+  else if (p.n_rep <= 4) hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, 1>), grid, dim3(256), 0, s, p);
+  else if (p.n_rep <= 8) hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, 2>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((decode_mfma_kernel<KVT, HD, 4>), grid, dim3(256), 0, s, p);
 }
 
 int launch_decode_mfma(const AttnParams& p, dim3 grid, bool p32, hipStream_t s) {
