@@ -586,12 +586,12 @@ struct AttnParams {
   int write_pos;          // slot of tree node 0
   const uint64_t* masks;  // [T] ancestor bitmasks (tree mode)
   float scale_log2;       // log2(e) / sqrt(hd)
-  int keep_nan;           // decode partials: see split_ml
+  int keep_nan;           // decode: see split_ml
 };
 
-// The (running max, sum) that a split stores.  The reduce kernels give zeros for a sum that is NaN (a key or
-// query that is not finite), the O projection that merges partials itself gives NaN: keep_nan
-// stores a finite pair instead, beside outputs that are NaN in every dim then.
+// The (running max, sum) that a split stores.  The reduce kernels, and a single split, give zeros for a sum that
+// is NaN (a key or query that is not finite), the O projection that merges partials itself gives NaN:
+// keep_nan stores a finite pair instead, beside outputs that are NaN in every dim then.
 __device__ __forceinline__ f32x2 split_ml(const AttnParams& p, float m, float l) {
   return p.keep_nan && l != l ? f32x2{kNegBig, 1.f} : f32x2{m, l};
 }
@@ -1081,19 +1081,21 @@ int attn_flash_splits(int B, int Hq, int Hkv, int hd, int kv_dtype, int active_l
 }
 
 // A decode step of one sequence.  Two to sixteen query heads per KV head take the matrix-core kernel at
-// every length, from 32 keys on with splits of about 128 keys up to one workgroup per CU: the vector
-// kernel with eight splits per head set fills 64 CUs at 8 KV heads and multiplies every key once per
-// query head (us per layer of a 7B-shape step with 32 / 8 heads and an FP8 cache, vector kernel /
-// four / eight / 32 splits here: 100 keys 46.3 / 44.8 / 45.0 / 45.9, 1000 keys 49.5 / 48.2 / 46.0 /
-// 46.5, 4000 keys 61.6 / 60.4 / 52.4 / 47.3, 16000 keys 113 / 110 / 78 / 57).  Other groupings (one query
-// head per KV head, or more than sixteen): splits merged by a reduce launch only where eight leave over
-// half of the CUs idle for long (4 heads of 64, FP8: 4000 keys eight merged by the O projection 31.9, 32
-// splits 33.0; 8000 keys 36.4 / 34.1; 16000 keys 43.1 / 35.7; 32 heads: never faster).
+// every length: one split, without a reduce launch, for the two rounds of 32 keys that its four waves make of 256,
+// then splits of about 128 keys up to one workgroup per CU (the vector kernel with eight splits per head set
+// fills 64 CUs at 8 KV heads and multiplies every key once per query head).  us per layer of a
+// 7B-shape step, 32 / 8 heads, FP8 cache, vector kernel / one / four / eight / 32 splits here: 100 keys 49.6 /
+// 45.2 / 47.4 / 48.3 / 48.8, 200 keys - / 47.1 / 48.0 / 47.9 / 48.3, 300 keys - / 48.5 / 47.6 / 48.2 / 48.7,
+// 800 keys - / 54.9 / 49.4 / 48.7 / 48.9, 6000 keys 71.8 / - / 66.3 / 57.0 / 51.3.  Other groupings (one query head per
+// KV head, or more than sixteen): splits merged by a reduce launch only where eight leave over half of the
+// CUs idle for long (4 heads of 64, FP8: 4000 keys eight merged by the O projection 31.9, 32 splits 33.0;
+// 8000 keys 36.4 / 34.1; 16000 keys 43.1 / 35.7; 32 heads: never faster).
+constexpr int kStepOneSplitKeys = 256;
 int attn_step_splits(int Hq, int Hkv, int active_len) {
   const int n_rep = Hq / Hkv;
   const int fill = axm_ceil_div(axm_num_cus(), Hkv);  // one workgroup per CU
   if (n_rep >= 2 && n_rep <= 16) {
-    int splits = active_len < 32 ? 1 : 4;  // (7 keys, FP16 cache, per layer: one 38.7 us, four 42.7)
+    int splits = active_len <= kStepOneSplitKeys ? 1 : 4;
     while (splits > 1 && splits < fill && splits < 64 && 128 * splits < active_len) splits <<= 1;
     return splits;
   }
@@ -1796,7 +1798,7 @@ __global__ void __launch_bounds__(256, RG ? 2 : 1) decode_mfma_kernel(AttnParams
     }
     const size_t gr = qrow0 + row;
     if (p.n_splits == 1) {
-      p.out[gr * HD + e] = f2h(ll > 0.f ? oo / ll : 0.f);
+      p.out[gr * HD + e] = f2h(ll > 0.f || (P32 && p.keep_nan && ll != ll) ? oo / ll : 0.f);
     } else {
       float* dst = p.ws + (gr * p.n_splits + split) * (2 + HD);
       if (e == 0) {

@@ -102,10 +102,10 @@ int attn_choose_splits(int B, int Hkv, int active_len);
 // form for 2-16 query heads per KV head and head size 64 / 128).
 int attn_flash_splits(int B, int Hq, int Hkv, int hd, int kv_dtype, int active_len);
 // p32: grouped-query heads on the matrix cores keep the softmax weights in fp32 for P V.  keep_nan: with
-// several splits, keys that are not finite give NaN and not zeros, as launch_flash_decode_parts.
+// p32 or several splits, keys that are not finite give NaN and not zeros, as launch_flash_decode_parts.
 int launch_flash_decode(const f16* q, const KvView& kv, f16* out, int Hq, int active_len, const int* active_len_dev,
                         int n_splits, float* ws, hipStream_t s, bool p32 = false, bool keep_nan = false);
-// Splits of a decode step's attention that a reduce launch merges, or 0 where partials merged by
+// Splits of a decode step's attention (several: merged by a reduce launch), or 0 where partials merged by
 // the O projection (launch_flash_decode_parts) are faster.  Head size 64 / 128.
 int attn_step_splits(int Hq, int Hkv, int active_len);
 

@@ -480,7 +480,8 @@ struct axm_runner {
                       : attn_choose_splits(1, d.n_kv_head, active_len);
       parts = parts_ok && want > 1;
     }
-    return step_attn_of(want, parts, max_splits, active_len);
+    const int n_rep = d.n_head / d.n_kv_head;
+    return step_attn_of(want, parts, n_rep >= 2 && n_rep <= 16, max_splits, active_len);
   }
 
   // Enqueue the whole single-token step on stream s (no host synchronization).
@@ -570,9 +571,8 @@ struct axm_runner {
     if (at.parts)
       return launch_flash_decode_parts(q, kv, d.n_head, 0, params + P_ACTIVE, at.splits, parts_o, parts_ml,
                                        at.short_splits, s);
-    // One split (a few keys): fp16 weights, as in the batched decode attention.
-    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, at.splits, ws, s, at.splits > 1,
-                               parts_ok);
+    return launch_flash_decode(q, kv, attn_y, d.n_head, 0, params + P_ACTIVE, at.splits, ws, s, at.p32,
+                               parts_ok && (at.p32 || at.splits > 1));
   }
 
   // 3. O projection, residual add into x.

@@ -19,10 +19,12 @@ def _model(n_head, n_kv_head, hd):
 
 
 # The smallest caches (fewer keys than splits), block edges, each doubling of the split count and its last length.
-GQA = [0, 1, 3, 31, 32, 127, 512, 513, 1025, 2100]
+GQA = [0, 1, 3, 30, 31, 32, 127, 255, 256, 512, 513, 1025, 2100]
 
 
 @pytest.mark.parametrize("heads,lengths", [((4, 2, 64), GQA), ((8, 2, 128), GQA), ((16, 1, 64), GQA),
+                                           # two and four groups of four rows for both head sizes, a ragged group
+                                           ((6, 1, 64), [40, 300]), ((8, 1, 128), [40, 300]), ((12, 1, 128), [40, 300]),
                                            ((4, 4, 64), [7998, 7999, 8100]),
                                            # more than sixteen query heads per KV head: the vector kernel
                                            ((32, 1, 64), [0, 40, 600, 8010])])
@@ -54,8 +56,9 @@ def test_step_attention_matches_oracle(dev, heads, lengths, kv):
         _check_logits(got, model.forward([tok], ocache)[-1], f"{heads} {kv} {n + 1} keys")
 
 
-@pytest.mark.parametrize("heads", [(4, 2, 64), (4, 1, 128)])
-def test_step_attention_keeps_small_weights(dev, heads):
+@pytest.mark.parametrize("heads", [(4, 2, 64), (4, 1, 128), (8, 1, 128), (16, 1, 64)])
+@pytest.mark.parametrize("n", [200, 600])
+def test_step_attention_keeps_small_weights(dev, heads, n):
     """Grouped-query softmax weights stay fp32: keys 2^-22 below the largest, whose values fill dims in which the
     large keys have none, keep the full precision of the result (weights as fp16 parts keep two bits of them).
 
@@ -66,7 +69,7 @@ def test_step_attention_keeps_small_weights(dev, heads):
     from axiomlm_amd.runner import DecodeRunner
 
     H, Hkv, hd = heads
-    d, n, S = H * hd, 600, 640
+    d, S = H * hd, 640
     z = lambda *s: torch.zeros(*s, dtype=torch.float16, device=dev)  # noqa: E731
     wte = z(8, d)
     wte[:, 0] = 1
@@ -105,7 +108,7 @@ def test_step_attention_keeps_small_weights(dev, heads):
     assert ((got - want).abs() <= 5 * 2.0 ** -11 * want.abs())[on].all()
 
 
-@pytest.mark.parametrize("heads,n", [((4, 2, 64), 40), ((4, 2, 64), 2100), ((8, 2, 128), 600), ((4, 4, 64), 600),
+@pytest.mark.parametrize("heads,n", [((4, 2, 64), 40), ((4, 2, 64), 300), ((4, 2, 64), 2100), ((8, 2, 128), 600), ((4, 4, 64), 600),
                                      ((4, 4, 64), 8010)])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 def test_step_over_a_key_that_is_not_finite(dev, heads, n, value):
