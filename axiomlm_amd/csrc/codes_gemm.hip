@@ -805,7 +805,7 @@ int codes_gemm_launch(int fmt, T16Args a, int M, int epi, float* ws, size_t ws_b
   else if (fmt == kCodesTernary) codes_launch_shape<kCodesTernary, Q4_EPI_STORE>(a, M, p, s);
   else if (fmt == kCodesF16) codes_launch_epi<kCodesF16>(a, M, epi, p, s);
   else codes_launch_epi<kCodesQ8>(a, M, epi, p, s);
-  return t16_gemm_finish(a, M, epi, p.splits, M, s);
+  return t16_gemm_finish(a, M, epi, p.splits, M, true, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -88,7 +88,7 @@ constexpr int kTile16GemmMaxTokens = 64;
 constexpr int kTile16GemmMaxSplits = 16;
 size_t t16_gemm_ws_bytes(int K, int n_units, int NT);
 int t16_gemm_launch(T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipStream_t s);
-int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, hipStream_t s);
+int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, bool vec, hipStream_t s);
 // Many-row GEMM over the same weights, any M in one launch (rows_gemm.hip; meant for M > 64):
 // a.x 16-byte aligned with ldx % 8 == 0, other arguments as t16_gemm_launch.  K is split
 // where M and N leave CUs idle, as far as ws_bytes allows (t16_rows_gemm_ws_bytes for the

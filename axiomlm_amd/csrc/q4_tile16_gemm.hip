@@ -276,9 +276,10 @@ __global__ void t16g_reduce_kernel(T16Args a, int n_splits, int up_col, int tok_
   t16g_store<EPI>(a, tok, row, v0, v1);
 }
 
-// The same with a thread per four rows of a token: 16-byte partial loads (N % 4 == 0).  A
-// thread per row read 4 bytes at a time (the 1000 x 12288 x 4096 many-row GEMM from two
-// splits, 128-row tiles: 132 -> 119 us).
+// The same with a thread per four rows of a token: 16-byte partial loads (N % 4 == 0), for the many-row
+// and code GEMMs (1000 x 12288 x 4096 from two splits, 128-row tiles: 132 -> 119 us; Q8 64 x 12288 x
+// 4096 25.0 -> 24.1).  After it the next 64-row launch is slower (six products of 12288 x 4096
+// in turn, 64 rows: 110 -> 136 us, 48 rows 105 -> 125; of 4096 x 4096 67 -> 88), so those keep a thread per row.
 template <int EPI>
 __global__ void __launch_bounds__(256) t16g_reduce4_kernel(T16Args a, int n_splits, int up_col, int tok_stride) {
   const int nv = a.N / 4;
@@ -296,8 +297,8 @@ __global__ void __launch_bounds__(256) t16g_reduce4_kernel(T16Args a, int n_spli
 }
 
 template <int EPI>
-void t16g_reduce(const T16Args& a, int M, int splits, int up_col, int ts, hipStream_t s) {
-  if (a.N % 4 == 0) {
+void t16g_reduce(const T16Args& a, int M, int splits, int up_col, int ts, bool vec, hipStream_t s) {
+  if (vec && a.N % 4 == 0) {
     const long n = (long)M * (a.N / 4);
     hipLaunchKernelGGL(t16g_reduce4_kernel<EPI>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, splits, up_col,
                        ts);
@@ -424,8 +425,9 @@ size_t t16_gemm_ws_bytes(int K, int n_units, int NT) {
 }
 
 // After a GEMM of `splits` K splits: the epilogue over the summed partials (ts token rows per
-// split), and the RMSNorm of the updated residual rows where it is asked for.
-int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, hipStream_t s) {
+// split; vec: by the four-row reduction), and the RMSNorm of the updated residual rows where it is
+// asked for.
+int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, bool vec, hipStream_t s) {
   if (a.split_info != nullptr) {
     a.split_info[0] = a.split_info[1] = a.split_info[2] = 0;
     if (splits > 1 && epi == Q4_EPI_STORE && a.post_ln_w == nullptr) {
@@ -442,14 +444,14 @@ int t16_gemm_finish(const T16Args& a, int M, int epi, int splits, int ts, hipStr
       hipLaunchKernelGGL(t16g_reduce_resid_norm_kernel, dim3(M), dim3(kRnThreads), 0, s, a, splits, ts);
       return 0;
     }
-    if (splits > 1) t16g_reduce<Q4_EPI_RESID>(a, M, splits, 0, ts, s);
+    if (splits > 1) t16g_reduce<Q4_EPI_RESID>(a, M, splits, 0, ts, vec, s);
     return launch_rmsnorm(a.resid, a.post_ln_w, a.post_norm_out, M, a.N, a.eps, s);
   }
   if (splits > 1) {
     const int up_col = a.pair_offset * 16;
-    if (epi == Q4_EPI_STORE) t16g_reduce<Q4_EPI_STORE>(a, M, splits, up_col, ts, s);
-    else if (epi == Q4_EPI_RESID) t16g_reduce<Q4_EPI_RESID>(a, M, splits, up_col, ts, s);
-    else t16g_reduce<Q4_EPI_SWIGLU>(a, M, splits, up_col, ts, s);
+    if (epi == Q4_EPI_STORE) t16g_reduce<Q4_EPI_STORE>(a, M, splits, up_col, ts, vec, s);
+    else if (epi == Q4_EPI_RESID) t16g_reduce<Q4_EPI_RESID>(a, M, splits, up_col, ts, vec, s);
+    else t16g_reduce<Q4_EPI_SWIGLU>(a, M, splits, up_col, ts, vec, s);
   }
   return 0;
 }
@@ -496,7 +498,7 @@ int t16_gemm_launch(T16Args a, int M, int epi, float* ws, size_t ws_bytes, hipSt
       t16g_launch_epi<Q4_EPI_SWIGLU>(a, cfg, grid, s);
       break;
   }
-  return t16_gemm_finish(a, M, epi, splits, 16 * cfg.mb, s);
+  return t16_gemm_finish(a, M, epi, splits, 16 * cfg.mb, false, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -284,5 +284,5 @@ int t16_rows_gemm_launch(T16Args a, int M, int epi, float* ws, size_t ws_bytes, 
   a.unpack[3] = 0x54005400u;
   if (plan.mb == 4) rows_launch_epi<4>(a, M, epi, splits, s);
   else rows_launch_epi<8>(a, M, epi, splits, s);
-  return t16_gemm_finish(a, M, epi, splits, M, s);
+  return t16_gemm_finish(a, M, epi, splits, M, true, s);
 }
