@@ -829,10 +829,14 @@ static bool lowbit_rows_use_codes(int fmt, int M, int K, int N) {
   return gguf ? launches >= 2 && M >= 12 : launches >= 2 || (M > 8 && K >= 4096);
 }
 
-// Whether M rows of a format go through this kernel (shapes and alignment apart).
+// Whether M rows of a format go through this kernel (shapes and alignment apart).  Q8 products of five or six
+// rows and few weight rows stay with the GEMV's two launches where K is too short to pay for split K and
+// its reduction (us, GEMV / here, 1000 weight rows: K = 256 five rows 6.3 / 4.9; 512 6.2 / 6.4; 1024 five 6.4 / 7.0,
+// six 6.7 / 7.1, seven 7.0 / 7.0; 2048 five 7.0 / 7.4, six 7.5 / 7.4; 4096 five 9.0 / 8.2; 2048 weight rows: never).
 static bool rows_use_codes(int fmt, int M, int K, int N) {
   if (fmt == kCodesMarlin) return marlin_rows_use_codes(M, K, N);
-  return fmt == kCodesQ8 ? M >= kCodesQ8MinRows : M > 4 && lowbit_rows_use_codes(fmt, M, K, N);
+  if (fmt == kCodesQ8) return M >= 7 || (M >= kCodesQ8MinRows && (N > 1024 || K < 512 || K > 2048));
+  return M > 4 && lowbit_rows_use_codes(fmt, M, K, N);
 }
 
 extern "C" size_t axm_qmm_codes_workspace_bytes(int format, int M, int K, int N) {

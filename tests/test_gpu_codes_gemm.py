@@ -167,7 +167,8 @@ def test_wrappers_choose_the_same_result_on_both_sides(dev):
     from axiomlm_amd.kernels import qmv_q2_k, qmv_q4_marlin, qmv_q8_g64, qmv_ternary
 
     rng = np.random.default_rng(5)
-    for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("ternary", qmv_ternary, (32, 33), 96, 320),
+    for fmt, fn, rows, N, K in (("q8", qmv_q8_g64, (4, 5), 96, 320), ("q8", qmv_q8_g64, (5, 6, 7), 96, 1024),
+                                ("ternary", qmv_ternary, (32, 33), 96, 320),
                                 ("q2", qmv_q2_k, (32, 33), 96, 320), ("ternary", qmv_ternary, (8, 9), 8192, 4096),
                                 ("marlin", qmv_q4_marlin, (4, 5), 96, 320),
                                 ("marlin", qmv_q4_marlin, (1, 2, 4), 8192, 4096)):
